@@ -133,6 +133,7 @@ struct Launch {
   uint32_t ev_thresh;    /* min #lanes needing the EVENT branch */
   uint32_t seg_thresh;   /* min #lanes needing the SEG step while others can collide */
   uint32_t max_steps;    /* micro-step budget of one query */
+  uint32_t lanes;        /* lanes of each wavefront that take work (64: all) */
   unsigned int* counters; /* [kXcds] next chunk of each XCD range */
   htgx_mc_accum* partials; /* [ntiles*nsub*64] */
   unsigned long long* stats; /* event counters */
@@ -163,6 +164,33 @@ struct KArgs {
   DevMap M;
   Launch P;
 };
+
+/* Kernel features: without kFeatRare, the features that few maps use (cloud
+ * and ground repetition, spectral BRDFs and interfaces, orthographic and
+ * thin-lens cameras, CIE XYZ wavelength sampling, Planck wavelength sampling
+ * over a continuous range) are compiled out; without kFeatMesh, the mesh
+ * ground (its BVH casts, its deferred casts). Their tests below are constants
+ * then, so that their code and registers do not weigh on the kernels of the
+ * maps that do without them. */
+enum { kFeatRare = 1, kFeatMesh = 2 };
+
+template<int FEAT>
+__device__ __forceinline__ bool is_mesh(const SceneF& S)
+{
+  return (FEAT & kFeatMesh) && S.ground_type == HTGX_GROUND_MESH;
+}
+
+template<int FEAT>
+__device__ __forceinline__ bool is_repeated(const SceneF& S)
+{
+  return (FEAT & kFeatRare) && S.repeat;
+}
+
+template<int FEAT>
+__device__ __forceinline__ bool has_gmat(const SceneF& S)
+{
+  return (FEAT & kFeatRare) && S.gmat;
+}
 
 enum { LS_SEG = 0, LS_COLL = 1, LS_EVENT = 2, LS_DONE = 3 };
 enum { MODE_TR = 0, MODE_SC = 1, MODE_LW = 2 };
@@ -368,17 +396,19 @@ struct GroundF {
 
 /* World position of a point of the lane's frame (-r moves the frame with
  * the copies of the cloud grid); only a mesh ground needs it */
+template<int FEAT>
 __device__ __forceinline__ void world_posf(const SceneF& S, const float p[3], float w[3])
 {
   w[0] = p[0];
   w[1] = p[1];
   w[2] = p[2];
-  if(S.repeat && S.ground_type == HTGX_GROUND_MESH) {
+  if(is_repeated<FEAT>(S) && is_mesh<FEAT>(S)) {
     w[0] += LCA(shift, 0);
     w[1] += LCA(shift, 1);
   }
 }
 
+template<int FEAT>
 __device__ __forceinline__ GroundF ground_tracef(const SceneF& S, const float o[3], const float d[3],
                                                  float r1, int32_t prev_prim, bool prev_edge,
                                                  bool any)
@@ -394,10 +424,12 @@ __device__ __forceinline__ GroundF ground_tracef(const SceneF& S, const float o[
       const float tt = (S.plane_z - o[2]) / d[2];
       if(tt > 0.f && tt < r1) { g.hit = true; g.t = tt; g.prim = 0; g.mtl = S.plane_mtl; }
     }
-  } else if(S.ground_type == HTGX_GROUND_MESH && !(o[2] > S.ghi[2] && d[2] >= 0.f)) {
+  } else if(is_mesh<FEAT>(S) && !(o[2] > S.ghi[2] && d[2] >= 0.f)) {
     /* (a ray from above the mesh's top going up or level meets none of it) */
-    const MeshHit m = mesh_trace_copies<float>(S.bvh, S.nbvh, S.tris, S.ground_repeat != 0, S.glo,
-                                               S.ghi, o, d, 0.f, r1, prev_prim, prev_edge, any);
+    const bool copies = (FEAT & kFeatRare) && S.ground_repeat;
+    const float glo[3] = {S.glo[0], S.glo[1], S.glo[2]}, ghi[3] = {S.ghi[0], S.ghi[1], S.ghi[2]};
+    const MeshHit m = mesh_trace_copies<float>(S.bvh, S.nbvh, S.tris, copies, glo, ghi, o, d, 0.f, r1,
+                                               prev_prim, prev_edge, any);
     g.nodes = m.nodes;
     g.ntris = m.ntris;
     if(m.tri >= 0) {
@@ -413,9 +445,10 @@ __device__ __forceinline__ GroundF ground_tracef(const SceneF& S, const float o[
 
 /* Unit geometric normal of a ground primitive: +z for the plane,
  * (v1 - v0) x (v2 - v0) for a mesh triangle; its side is the sky side */
+template<int FEAT>
 __device__ __forceinline__ void ground_normalf(const SceneF& S, int32_t prim, float N[3])
 {
-  if(S.ground_type == HTGX_GROUND_MESH) {
+  if(is_mesh<FEAT>(S)) {
     const BvhTri& T = S.tris[prim];
     N[0] = T.e1[1] * T.e2[2] - T.e1[2] * T.e2[1];
     N[1] = T.e1[2] * T.e2[0] - T.e1[0] * T.e2[2];
@@ -536,6 +569,7 @@ __device__ __forceinline__ void load_leaf(const SceneF& S, const TrackRegs& G, L
  * the current leaf, other axes clamped into its block range); false when the
  * step leaves the grid. One code path for both, so that a wavefront pays for
  * a single leaf load per pass whatever mix of states its lanes are in. */
+template<int FEAT>
 __device__ __forceinline__ bool next_cell(const SceneF& S, Lane& L, uint32_t c[3])
 {
   const bool step = L.cstate == 4;
@@ -559,7 +593,7 @@ __device__ __forceinline__ bool next_cell(const SceneF& S, Lane& L, uint32_t c[3
   if(out) {
     /* -r: into the next copy of the grid along X or Y; the lane's frame
      * moves with it (a bounded number of copies per query) */
-    if(oa == 2 || !S.repeat || ++LC(ntiles) > kMaxTilesF) return false;
+    if(oa == 2 || !is_repeated<FEAT>(S) || ++LC(ntiles) > kMaxTilesF) return false;
 #pragma unroll
     for(int a = 0; a < 2; ++a) {
       if(a == oa) {
@@ -576,6 +610,7 @@ __device__ __forceinline__ bool next_cell(const SceneF& S, Lane& L, uint32_t c[3
 
 /* Start the iterator of the query over [0, qr] along (pos, dir); no memory
  * access here */
+template<int FEAT>
 __device__ __forceinline__ void iter_init(const SceneF& S, Lane& L)
 {
   const float r1 = L.qr;
@@ -584,7 +619,7 @@ __device__ __forceinline__ void iter_init(const SceneF& S, Lane& L)
   L.adv = false;
   L.cstate = 2;
   L.nsteps = 0;
-  if(S.repeat) LC(ntiles) = 0;
+  if(is_repeated<FEAT>(S)) LC(ntiles) = 0;
 #pragma unroll
   for(int a = 0; a < 3; ++a) L.inv_dir[a] = 1.f / L.dir[a];
   if(S.has_clouds) {
@@ -592,7 +627,7 @@ __device__ __forceinline__ void iter_init(const SceneF& S, Lane& L)
     bool miss = false;
 #pragma unroll
     for(int a = 0; a < 3; ++a) {
-      if(S.repeat && a < 2) continue; /* -r: an infinite layer along X, Y */
+      if(is_repeated<FEAT>(S) && a < 2) continue; /* -r: an infinite layer along X, Y */
       const float plo = planef(S, a, 0), phi = planef(S, a, S.dims0[a]);
       if(L.dir[a] != 0.f) {
         const float ta = (plo - L.pos[a]) * L.inv_dir[a];
@@ -604,7 +639,7 @@ __device__ __forceinline__ void iter_init(const SceneF& S, Lane& L)
       }
     }
     if(!miss && fmaxf(tn, 0.f) < fminf(tf, r1)) {
-      if(S.repeat) {
+      if(is_repeated<FEAT>(S)) {
         /* the frame of the copy of the grid holding the entry point */
         const float te = fmaxf(tn, 0.f);
 #pragma unroll
@@ -675,7 +710,7 @@ __device__ __forceinline__ float gas_depth(const SceneF& S, const Lane& L, int p
  * The iterator only moves past an emitted segment at the next call, so that
  * the leaf range used to clamp the cells of its collisions stays the one of
  * the segment. Each pass of the loop loads at most one leaf, at one site. */
-template<bool COUNT>
+template<bool COUNT, int FEAT>
 __device__ __forceinline__ bool iter_next(const SceneF& S, const TrackRegs& G, Lane& L, int prop,
                                           float* t0, bool runs = false)
 {
@@ -688,7 +723,7 @@ __device__ __forceinline__ bool iter_next(const SceneF& S, const TrackRegs& G, L
     if(L.itdone || !(L.tit < tmax)) return false;
     if(L.cstate >= 3) {
       uint32_t c[3];
-      if(next_cell(S, L, c)) { load_leaf<COUNT>(S, G, L, c[0], c[1], c[2]); L.cstate = 1; }
+      if(next_cell<FEAT>(S, L, c)) { load_leaf<COUNT>(S, G, L, c[0], c[1], c[2]); L.cstate = 1; }
       else L.cstate = 2;
     }
     const float t = L.tit;
@@ -818,7 +853,7 @@ __device__ __forceinline__ void count_ground(Lane& L, const GroundF& g)
   if(COUNT) { L.c_bvh += g.nodes; L.c_tri += g.ntris; }
 }
 
-template<bool COUNT>
+template<bool COUNT, int FEAT>
 __device__ __forceinline__ void sw_begin(const SceneF& S, Lane& L, int mask, const float p[3],
                                          const float d[3])
 {
@@ -832,8 +867,8 @@ __device__ __forceinline__ void sw_begin(const SceneF& S, Lane& L, int mask, con
   L.prev_edge = false;
   if((mask & HTGX_RADIANCE_DIRECT) && dot3f(L.dir, S.sun_dir) >= S.sun_cos_half) {
     float wp[3];
-    world_posf(S, L.pos, wp);
-    const GroundF g = ground_tracef(S, wp, L.dir, FLT_MAX, -1, false, true);
+    world_posf<FEAT>(S, L.pos, wp);
+    const GroundF g = ground_tracef<FEAT>(S, wp, L.dir, FLT_MAX, -1, false, true);
     count_ground<COUNT>(L, g);
     if(!g.hit) {
       LC(stage) = ST_DIRECT;
@@ -863,7 +898,7 @@ __device__ __forceinline__ float query_tr(const Lane& L)
 }
 
 /* Consume the finished query of the current stage */
-template<bool COUNT, int SPECTRAL>
+template<bool COUNT, int SPECTRAL, int FEAT>
 __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u)
 {
   /* the stages of the other spectral domain never occur: compiled out */
@@ -901,8 +936,8 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
       for(int a = 0; a < 3; ++a) L.pos[a] = L.pos[a] + L.dir[a] * dst;
       bool specular = false;
       if(L.surface) {
-        ground_normalf(S, LC(gh_prim), N);
-        if(S.gmat) {
+        ground_normalf<FEAT>(S, LC(gh_prim), N);
+        if(has_gmat<FEAT>(S)) {
           /* the hit side's material and its BRDF at the wavelength,
            * ..._sw.c:403-411 (the canonical of the phase choice) */
           const int32_t m = interface_mtl(S.ifcs[LC(gh_mtl)], S.mtls, dot3f(N, L.dir) > 0.f);
@@ -949,8 +984,8 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
       bool shadowed = LC(R) <= 0.f;
       if(!shadowed) {
         float wp[3];
-        world_posf(S, L.pos, wp);
-        const GroundF g = ground_tracef(S, wp, sun_dir, FLT_MAX, LC(prev_prim), L.prev_edge, true);
+        world_posf<FEAT>(S, L.pos, wp);
+        const GroundF g = ground_tracef<FEAT>(S, wp, sun_dir, FLT_MAX, LC(prev_prim), L.prev_edge, true);
         count_ground<COUNT>(L, g);
         shadowed = g.hit;
       }
@@ -989,10 +1024,10 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
         L.prev_edge = false;
       } else {
         float N[3];
-        ground_normalf(S, LC(gh_prim), N);
+        ground_normalf<FEAT>(S, LC(gh_prim), N);
         float refl, T;
         bool specular = false;
-        if(S.gmat) { /* ..._lw.c:249-252 */
+        if(has_gmat<FEAT>(S)) { /* ..._lw.c:249-252 */
           const int32_t m = interface_mtl(S.ifcs[LC(gh_mtl)], S.mtls, dot3f(N, L.dir) > 0.f);
           const DevBrdf& b = brdf_fetch(S.mtls[m], S.brdfs, (double)LC(wlen), (double)u[4]);
           refl = (float)b.refl;
@@ -1028,9 +1063,10 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
 
 /* Sensor ray, wavelength, band and k-point, then the first walk
  * (..._draw_map.c:348-400 and :233-302) */
-template<int SENSOR, int SPECTRAL, bool COUNT, bool RARE>
+template<int SENSOR, int SPECTRAL, bool COUNT, int FEAT>
 __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lane& L, const float* u)
 {
+  constexpr bool RARE = (FEAT & kFeatRare) != 0;
   const uint32_t px = L.pixel % M.width, py = L.pixel / M.width;
   float org[3], dir[3];
   if(SENSOR == HTGX_SENSOR_CAMERA) {
@@ -1038,7 +1074,7 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
      * htgx_device.h) */
     const float fx = ((float)px + u[0]) / (float)M.width;
     const float fy = ((float)py + u[1]) / (float)M.height;
-    if(M.ortho) {
+    if(RARE && M.ortho) {
       const float sx = (2.f * fx - 1.f) * (float)(M.ortho_half_h * M.aspect);
       const float sy = (1.f - 2.f * fy) * (float)M.ortho_half_h;
 #pragma unroll
@@ -1054,7 +1090,7 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
         dir[a] = (float)M.z[a] + (float)M.x[a] * sx + (float)M.y[a] * sy;
         org[a] = (float)M.pos[a];
       }
-      if(M.lens_radius > 0) {
+      if(RARE && M.lens_radius > 0) {
         const float r = (float)M.lens_radius * sqrtf(u[2]), phi = 2.f * kPif * u[3];
         const float lx = r * cosf(phi), ly = r * sinf(phi);
 #pragma unroll
@@ -1078,16 +1114,16 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
     const float up[3] = {0.f, 0.f, 1.f};
     /* a sample under the ground (the up ray meets the ground's sky side from
      * below, ..._draw_map.c:75-100) is rejected */
-    const GroundF gu = ground_tracef(S, org, up, INFINITY, -1, false, false);
+    const GroundF gu = ground_tracef<FEAT>(S, org, up, INFINITY, -1, false, false);
     count_ground<COUNT>(L, gu);
     if(gu.hit) {
       float N[3];
-      ground_normalf(S, gu.prim, N);
+      ground_normalf<FEAT>(S, gu.prim, N);
       /* with interfaces: the material of the side the up ray travels in
        * (front if cos(up, -N) < 0) must be the sky's; else the ray must not
        * meet the side N points to from below */
       bool under;
-      if(S.explicit_ifc) {
+      if(RARE && S.explicit_ifc) {
         const DevIfc& f = S.ifcs[gu.mtl];
         under = (N[2] > 0.f ? f.front : f.back) != S.sky_mtl;
       } else {
@@ -1130,7 +1166,7 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
     request_ground(L, MODE_LW, HTGX_Kext);
   } else if(SENSOR == HTGX_SENSOR_CAMERA) {
     LC(phase) = 0;
-    sw_begin<COUNT>(S, L, HTGX_RADIANCE_ALL, org, dir);
+    sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_ALL, org, dir);
   } else {
     float sun_dir[3];
     local_to_worldf(S.sun_dir, 1.f - u[7] * (1.f - S.sun_cos_half), 2.f * kPif * u[8], sun_dir);
@@ -1139,12 +1175,12 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
     LC(Ld) = 0.f;
 #pragma unroll
     for(int a = 0; a < 3; ++a) { LCA(org, a) = org[a]; LCA(dir0, a) = dir[a]; }
-    if(LC(cosN) > 0.f) { LC(phase) = 1; sw_begin<COUNT>(S, L, HTGX_RADIANCE_DIRECT, org, sun_dir); }
-    else { LC(phase) = 2; sw_begin<COUNT>(S, L, HTGX_RADIANCE_DIFFUSE, org, dir); }
+    if(LC(cosN) > 0.f) { LC(phase) = 1; sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_DIRECT, org, sun_dir); }
+    else { LC(phase) = 2; sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_DIFFUSE, org, dir); }
   }
 }
 
-template<int SENSOR, int SPECTRAL, bool COUNT>
+template<int SENSOR, int SPECTRAL, bool COUNT, int FEAT>
 __device__ __forceinline__ void walk_done(const SceneF& S, Lane& L)
 {
   if(SENSOR == HTGX_SENSOR_CAMERA) {
@@ -1159,27 +1195,41 @@ __device__ __forceinline__ void walk_done(const SceneF& S, Lane& L)
     float o[3], d[3];
 #pragma unroll
     for(int a = 0; a < 3; ++a) { o[a] = LCA(org, a); d[a] = LCA(dir0, a); }
-    sw_begin<COUNT>(S, L, HTGX_RADIANCE_DIFFUSE, o, d);
+    sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_DIFFUSE, o, d);
   } else {
     LC(stage) = ST_REAL_DONE;
     LC(w) = (LC(cosN) * S.sun_solid_angle * LC(Ld) + kPif * LC(w)) / LC(pdf);
   }
 }
 
-/* Next chunk from this XCD's tile range, else from the others */
-__device__ __forceinline__ bool fetch_chunk(const Launch& P, uint32_t xcd, uint32_t* chunk)
+/* Chunks for the lanes with `need', from this XCD's tile range, else from the
+ * others: one atomic per wavefront and range, the lanes sharing what it
+ * reserved in lane order. `tried' counts the ranges the wavefront has found
+ * empty; it does not ask them again. Returns false for a lane that finds no
+ * chunk left anywhere. The whole wavefront calls this together. */
+__device__ __forceinline__ bool fetch_chunks(const Launch& P, uint32_t xcd, uint32_t* tried, bool need,
+                                             uint32_t* chunk)
 {
   const uint32_t per_tile = P.nsub * 64u;
-  for(uint32_t k = 0; k < (uint32_t)kXcds; ++k) {
-    const uint32_t x = (xcd + k) % (uint32_t)kXcds;
-    const uint32_t t0 = x * P.xcd_tiles;
-    const uint32_t t1 = min(t0 + P.xcd_tiles, P.ntiles);
-    if(t0 >= t1) continue;
+  bool got = false;
+  uint64_t mask = __ballot(need);
+  while(mask && *tried < (uint32_t)kXcds) {
+    const uint32_t x = (xcd + *tried) % (uint32_t)kXcds;
+    const uint32_t t0 = min(x * P.xcd_tiles, P.ntiles), t1 = min(t0 + P.xcd_tiles, P.ntiles);
     const uint32_t n = (t1 - t0) * per_tile;
-    const uint32_t c = atomicAdd(P.counters + x, 1u);
-    if(c < n) { *chunk = t0 * per_tile + c; return true; }
+    if(n) {
+      const int leader = __ffsll((unsigned long long)mask) - 1;
+      uint32_t c = 0;
+      if((int)(threadIdx.x & 63u) == leader) c = atomicAdd(P.counters + x, (uint32_t)__popcll(mask));
+      c = (uint32_t)__builtin_amdgcn_readlane((int)c, leader) +
+          (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                              __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+      if(need && !got && c < n) { *chunk = t0 * per_tile + c; got = true; }
+    }
+    mask = __ballot(need && !got);
+    if(mask) ++*tried;
   }
-  return false;
+  return got;
 }
 
 __device__ __forceinline__ uint64_t wave_sum64(uint64_t v)
@@ -1188,31 +1238,10 @@ __device__ __forceinline__ uint64_t wave_sum64(uint64_t v)
   return v;
 }
 
-/* Kernel features: without kFeatRare, the features that few maps use (cloud
- * and ground repetition, spectral BRDFs and interfaces, orthographic and
- * thin-lens cameras, CIE XYZ wavelength sampling, Planck wavelength sampling
- * over a continuous range) are compiled out; without kFeatMesh, the mesh
- * ground (its BVH casts, its deferred casts). Their flags become constants,
- * so that their code and registers do not weigh on the kernels of the maps
- * that do without them. */
-enum { kFeatRare = 1, kFeatMesh = 2 };
-
-/* The persistent loop of one wavefront over the chunks of one map */
 /* A pointer to constant memory: the kernel argument segment, or a table in
  * device memory that no kernel writes while it is read */
 template<class T>
 using KPtr = const __attribute__((address_space(4))) T*;
-
-/* The same address, opaque to the optimiser (an empty asm statement in a
- * scalar register): loads through it stay where they are written, in the
- * loop, instead of being hoisted out of it */
-template<class T>
-__device__ __forceinline__ KPtr<T> launder(KPtr<T> p)
-{
-  uint64_t a = (uint64_t)p;
-  asm volatile("" : "+s"(a));
-  return (KPtr<T>)a;
-}
 
 /* A copy of a constant-memory struct (scalar loads; the host compilation
  * pass, which only needs the declaration, gets an empty value) */
@@ -1227,37 +1256,39 @@ __device__ __forceinline__ T kload(KPtr<T> p)
 #endif
 }
 
-/* The scene and map of a kernel instance: the features it was not compiled
- * for (FEAT) read as constant zeros, so that their code folds away */
-template<int FEAT>
-__device__ __forceinline__ void fold_features(SceneF& S, DevMap& M)
-{
-  /* no mesh: the ground type is NONE or PLANE (0 or 1), so that every test
-   * for HTGX_GROUND_MESH (2) folds to false */
-  if(!(FEAT & kFeatMesh)) S.ground_type &= 1;
-  if(!(FEAT & kFeatRare)) {
-    S.repeat = 0;
-    S.ground_repeat = 0;
-    S.gmat = 0;
-    S.explicit_ifc = 0;
-    M.ortho = 0;
-    M.lens_radius = 0.0;
-  }
-}
+/* The arguments of the map each wavefront of the block works on (of a batch,
+ * the wavefronts may be at different maps). The event step reads its scene,
+ * map and launch constants from here: 60-odd of them, in scalar registers
+ * they would be live across the tracking steps, and loaded by scalar loads at
+ * each event they cost ten dependent waits on the kernel argument segment,
+ * 1800-3200 cycles per event step. An LDS broadcast read answers in about
+ * 100 cycles. */
+__shared__ KArgs g_args[kBlock / 64];
 
+/* The persistent loop of one wavefront over the chunks of one map */
 template<int SENSOR, int SPECTRAL, bool COUNT, int FEAT, bool LIST = false>
-__device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr<Launch> pP)
+__device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
 {
   constexpr bool RARE = (FEAT & kFeatRare) != 0;
   constexpr bool kLW = SPECTRAL == HTGX_SPECTRAL_LW;
-  SceneF S = kload(pS);
-  DevMap M = kload(pM);
-  const Launch P = kload(pP);
-  fold_features<FEAT>(S, M);
+  const SceneF S = kload(&pK->S);
+  const Launch P = kload(&pK->P);
+  const uint64_t seed = kload(&pK->M.seed);
+  /* this wavefront's copy of the arguments, for the event step */
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  {
+    static_assert(sizeof(KArgs) % 4 == 0, "copied by dwords");
+    const KPtr<uint32_t> src = (KPtr<uint32_t>)pK;
+    uint32_t* dst = (uint32_t*)&g_args[wave];
+    for(uint32_t i = threadIdx.x & 63u; i < sizeof(KArgs) / 4; i += 64u) dst[i] = kload(src + i);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
   /* canonicals per event: 8, plus 2 for the sun of a SW flux map */
   constexpr int NP = (SENSOR == HTGX_SENSOR_RECTANGLE && SPECTRAL == HTGX_SPECTRAL_SW) ? 5 : 4;
   Lane L;
-  L.lstate = LS_EVENT;
+  L.lstate = (threadIdx.x & 63u) < P.lanes ? LS_EVENT : LS_DONE;
   LC(stage) = ST_FETCH;
   L.pending = false;
   L.nq = false;
@@ -1268,8 +1299,9 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
   LC(tsum) = LC(tsum2) = 0.f;
   L.pixel = L.r = 0;
   const uint32_t xcd = blockIdx.x % (uint32_t)kXcds;
+  uint32_t tried = 0; /* chunk ranges found empty */
   const TrackRegs G =
-      track_regs<!RARE>(S, (uint32_t)M.seed ^ (uint32_t)(M.seed >> 32), P.max_steps);
+      track_regs<!RARE>(S, (uint32_t)seed ^ (uint32_t)(seed >> 32), P.max_steps);
   const uint32_t key = G.key;
   uint64_t d_it = 0, d_ce = 0, d_cl = 0, d_se = 0, d_sl = 0, d_ee = 0, d_el = 0;
   /* shader clock cycles per phase (counting build only) */
@@ -1282,13 +1314,18 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
     const uint64_t want0 = __ballot(L.lstate == LS_EVENT);
     const uint64_t busy0 = __ballot(L.lstate == LS_SEG || L.lstate == LS_COLL);
     if(!(busy0 | want0)) break;
+    /* the thresholds count on a full wavefront: with lanes out of work they
+     * shrink with the lanes left, so that the last paths do not wait for
+     * company that cannot come */
+    const uint32_t alive = (uint32_t)__popcll(busy0 | want0);
+    const uint32_t ev_min = (P.ev_thresh * alive) >> 6, seg_min = (P.seg_thresh * alive) >> 6;
     if(COUNT) tk = clock64();
 
     /* next segment of the query, and the first tentative collision in it:
      * while some lanes can take a collision step, the segment step waits
      * until seg_thresh lanes need it */
     const uint64_t bs = __ballot(L.lstate == LS_SEG);
-    const bool run_seg = bs && (__popcll(bs) >= P.seg_thresh || !__ballot(L.lstate == LS_COLL));
+    const bool run_seg = bs && (__popcll(bs) >= seg_min || !__ballot(L.lstate == LS_COLL));
     if(COUNT) {
       d_it++;
       d_se += run_seg;
@@ -1299,7 +1336,7 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
       /* longwave kernels run MODE_LW queries only, shortwave ones MODE_SC
        * and MODE_TR: the other modes' code is compiled out */
       const int sprop = kLW ? HTGX_Kext : L.mode == MODE_SC ? HTGX_Ks : L.prop;
-      if(iter_next<COUNT>(S, G, L, sprop, &t0, !kLW && L.mode == MODE_TR)) {
+      if(iter_next<COUNT, FEAT>(S, G, L, sprop, &t0, !kLW && L.mode == MODE_TR)) {
         const float len = L.s_t1 - t0;
         if(!kLW && L.mode == MODE_TR) L.Tmin += (double)len * (double)L.s_kmin;
         if(!kLW && L.mode == MODE_SC) {
@@ -1421,24 +1458,18 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
     /* events, when enough lanes need them or nothing else is left */
     const uint64_t want = __ballot(L.lstate == LS_EVENT);
     const uint64_t other = __ballot(L.lstate == LS_SEG || L.lstate == LS_COLL);
-    if(want && (__popcll(want) >= P.ev_thresh || !other)) {
-      /* the shortwave event step reads its constants afresh: the many
-       * fields it uses then hold scalar registers only while it runs, not
-       * across the tracking steps (fewer scalar spills there). The
-       * longwave one, which runs twice as often per realisation, keeps the
-       * values computed before the loop: recomputing them at each event
-       * measured slower there */
-      constexpr bool kReload = SPECTRAL != HTGX_SPECTRAL_LW, kReloadP = kReload;
-      const SceneF& S_h = S;
-      const DevMap& M_h = M;
-      const Launch& P_h = P;
-      SceneF S = kReload ? kload(launder(pS)) : S_h;
-      DevMap M = kReload ? kload(launder(pM)) : M_h;
-      const Launch P = kReloadP ? kload(launder(pP)) : P_h;
-      if(kReload) fold_features<FEAT>(S, M);
+    if(want && (__popcll(want) >= ev_min || !other)) {
+      /* the index is opaque to the optimiser (an empty asm statement), so
+       * that the reads stay where they are written */
+      uint32_t wv = wave;
+      asm volatile("" : "+s"(wv));
+      const SceneF& S = g_args[wv].S;
+      const DevMap& M = g_args[wv].M;
+      const Launch& P = g_args[wv].P;
       if(COUNT) { d_ee++; d_el += __popcll(want); }
-      if(L.lstate == LS_EVENT) {
-        if(LIST && LC(stage) == ST_FETCH) {
+      const bool fetch = L.lstate == LS_EVENT && LC(stage) == ST_FETCH;
+      if(LIST) {
+        if(fetch) {
           /* the next (pixel, realisation) pair of the list, one realisation */
           const uint32_t c = atomicAdd(P.counters, 1u);
           if(c >= P.nvalid) {
@@ -1453,27 +1484,28 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
             LC(tsum) = LC(tsum2) = 0.f;
             LC(stage) = ST_BEGIN;
           }
-        } else if(LC(stage) == ST_FETCH) {
-          uint32_t c;
-          if(!fetch_chunk(P, xcd, &c)) {
-            L.lstate = LS_DONE;
-            if(P.exhausted) atomicExch(P.exhausted, 1u);
-          } else {
-            LC(chunk) = c;
-            const uint32_t m = c & 63u, rest = c >> 6;
-            const uint32_t s = rest % P.nsub, t = rest / P.nsub;
-            const uint32_t x = (t % P.ntx) * 8u + ((m & 1u) | ((m >> 1) & 2u) | ((m >> 2) & 4u));
-            const uint32_t y = (t / P.ntx) * 8u + (((m >> 1) & 1u) | ((m >> 2) & 2u) | ((m >> 3) & 4u));
-            if(x < P.width && y < P.height) {
-              L.pixel = y * P.width + x;
-              L.r = (P.spp_offset_dev ? *P.spp_offset_dev : P.spp_offset) + s * P.K;
-              LC(r_end) = L.r + P.K;
-              LC(n) = LC(nfail) = 0;
-              LC(sum) = LC(sum2) = 0.0;
-              LC(tsum) = LC(tsum2) = 0.f;
-              LC(stage) = ST_BEGIN;
-            } /* else: outside the image, fetch again next time */
-          }
+        }
+      } else if(__ballot(fetch)) {
+        uint32_t c = 0;
+        const bool got = fetch_chunks(P, xcd, &tried, fetch, &c);
+        if(fetch && !got) {
+          L.lstate = LS_DONE;
+          if(P.exhausted) atomicExch(P.exhausted, 1u);
+        } else if(fetch) {
+          LC(chunk) = c;
+          const uint32_t m = c & 63u, rest = c >> 6;
+          const uint32_t s = rest % P.nsub, t = rest / P.nsub;
+          const uint32_t x = (t % P.ntx) * 8u + ((m & 1u) | ((m >> 1) & 2u) | ((m >> 2) & 4u));
+          const uint32_t y = (t / P.ntx) * 8u + (((m >> 1) & 1u) | ((m >> 2) & 2u) | ((m >> 3) & 4u));
+          if(x < P.width && y < P.height) {
+            L.pixel = y * P.width + x;
+            L.r = (P.spp_offset_dev ? *P.spp_offset_dev : P.spp_offset) + s * P.K;
+            LC(r_end) = L.r + P.K;
+            LC(n) = LC(nfail) = 0;
+            LC(sum) = LC(sum2) = 0.0;
+            LC(tsum) = LC(tsum2) = 0.f;
+            LC(stage) = ST_BEGIN;
+          } /* else: outside the image, fetch again next time */
         }
       }
       WF_TICK(2)
@@ -1490,15 +1522,15 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
         for(int i = 0; i < NP; ++i) { const float2 v = draw2(L, key); u[2 * i] = v.x; u[2 * i + 1] = v.y; }
         WF_TICK(3)
         if(begin) {
-          real_begin<SENSOR, SPECTRAL, COUNT, RARE>(S, M, L, u);
+          real_begin<SENSOR, SPECTRAL, COUNT, FEAT>(S, M, L, u);
         }
         WF_TICK(4)
         if(!begin && L.pending) {
           L.pending = false;
-          consume<COUNT, SPECTRAL>(S, L, u);
+          consume<COUNT, SPECTRAL, FEAT>(S, L, u);
         }
         WF_TICK(5)
-        while(LC(stage) == ST_WALK_DONE) walk_done<SENSOR, SPECTRAL, COUNT>(S, L);
+        while(LC(stage) == ST_WALK_DONE) walk_done<SENSOR, SPECTRAL, COUNT, FEAT>(S, L);
         WF_TICK(6)
         if(LC(stage) == ST_REAL_DONE) {
           const uint64_t t1 = wall_clock64();
@@ -1532,8 +1564,8 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
           L.lazy = false; /* a query that ended in the medium leaves no cast pending */
           if(L.nq_ground) {
             float wp[3];
-            world_posf(S, L.pos, wp);
-            if(S.ground_type == HTGX_GROUND_MESH && !resume && wp[2] > S.ghi[2] && L.dir[2] < 0.f) {
+            world_posf<FEAT>(S, L.pos, wp);
+            if(is_mesh<FEAT>(S) && !resume && wp[2] > S.ghi[2] && L.dir[2] < 0.f) {
               /* from above the mesh, downwards: the tracking runs up to the
                * mesh's top first, and most queries end in the medium before
                * it; the cast waits until the tracking gets there */
@@ -1541,7 +1573,7 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
               L.gh_hit = false;
               L.qr = (S.ghi[2] - wp[2]) / L.dir[2];
             } else {
-              const GroundF gh = ground_tracef(S, wp, L.dir, INFINITY, LC(prev_prim), L.prev_edge,
+              const GroundF gh = ground_tracef<FEAT>(S, wp, L.dir, INFINITY, LC(prev_prim), L.prev_edge,
                                                false);
               count_ground<COUNT>(L, gh);
               L.gh_hit = gh.hit;
@@ -1561,7 +1593,7 @@ __device__ __forceinline__ void run_scene(KPtr<SceneF> pS, KPtr<DevMap> pM, KPtr
             L.Tmin = 0.0;
             L.pending = false;
             if(!kLW && L.mode == MODE_SC) L.Ts_a = exp1f(draw2(L, key).x);
-            iter_init(S, L);
+            iter_init<FEAT>(S, L);
           }
           L.tc = L.tc_a = INFINITY;
           L.lstate = LS_SEG;
@@ -1605,7 +1637,7 @@ wavefront_kernel(KArgs A)
 {
   (void)A;
   const KPtr<KArgs> k = (KPtr<KArgs>)__builtin_amdgcn_kernarg_segment_ptr();
-  run_scene<SENSOR, SPECTRAL, COUNT, FEAT>(&k->S, &k->M, &k->P);
+  run_scene<SENSOR, SPECTRAL, COUNT, FEAT>(k);
 }
 
 /* Given (pixel, realisation) pairs of one map, one realisation each (the
@@ -1618,7 +1650,7 @@ wavefront_list_kernel(KArgs A)
 {
   (void)A;
   const KPtr<KArgs> k = (KPtr<KArgs>)__builtin_amdgcn_kernarg_segment_ptr();
-  run_scene<SENSOR, SPECTRAL, false, kFeatRare | kFeatMesh, true>(&k->S, &k->M, &k->P);
+  run_scene<SENSOR, SPECTRAL, false, kFeatRare | kFeatMesh, true>(k);
 }
 
 /* The FP32 segment iterator on given rays over [0, range[1]] (a debug
@@ -1640,11 +1672,11 @@ wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop,
   L.cka = S.has_clouds ? S.cka[iband] : 0.f;
   L.cks = S.has_clouds ? S.cks[iband] : 0.f;
   LCA(shift, 0) = LCA(shift, 1) = 0.f;
-  iter_init(S, L);
+  iter_init<kFeatRare>(S, L);
   uint32_t n = 0;
   float t0;
   const TrackRegs G = track_regs<false>(S, 0u, 0u);
-  while(iter_next<false>(S, G, L, prop, &t0)) {
+  while(iter_next<false, kFeatRare>(S, G, L, prop, &t0)) {
     if(n < max_segs) {
       htgx_segment& o = segs[(size_t)i * max_segs + n];
       o.t0 = t0;
@@ -1666,9 +1698,7 @@ wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop,
 
 /* One map of a batched launch */
 struct BatchScene {
-  SceneF S;
-  DevMap M;
-  Launch P;
+  KArgs A;
   htgx_mc_accum* accum; /* the map's pixel accumulators */
 };
 
@@ -1683,10 +1713,10 @@ wavefront_batch_kernel(const BatchScene* __restrict__ scenes, uint32_t nscenes)
 {
   for(uint32_t s = 0; s < nscenes; ++s) {
     const BatchScene& B = scenes[s];
-    const unsigned int ex = __hip_atomic_load(B.P.exhausted, __ATOMIC_RELAXED,
+    const unsigned int ex = __hip_atomic_load(B.A.P.exhausted, __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT);
     if(__builtin_amdgcn_readfirstlane(ex)) continue;
-    run_scene<SENSOR, SPECTRAL, false, FEAT>((KPtr<SceneF>)&B.S, (KPtr<DevMap>)&B.M, (KPtr<Launch>)&B.P);
+    run_scene<SENSOR, SPECTRAL, false, FEAT>((KPtr<KArgs>)&B.A);
   }
 }
 
@@ -1707,8 +1737,8 @@ batch_advance_kernel(BatchScene* scenes, uint32_t n, unsigned int* step)
 {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i < n) {
-    scenes[i].P.spp_offset += scenes[i].M.spp;
-    scenes[i].M.spp_offset += scenes[i].M.spp;
+    scenes[i].A.P.spp_offset += scenes[i].A.M.spp;
+    scenes[i].A.M.spp_offset += scenes[i].A.M.spp;
   }
   if(i == 0) *step += 1u;
 }
@@ -1752,8 +1782,8 @@ batch_merge_kernel(const BatchScene* scenes)
 {
   const BatchScene& B = scenes[blockIdx.y];
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if(p < B.M.width * B.M.height)
-    merge_pixel(B.P.partials, B.M.width, B.P.ntx, B.P.nsub, B.accum, p);
+  const Launch& P = B.A.P;
+  if(p < P.width * P.height) merge_pixel(P.partials, P.width, P.ntx, P.nsub, B.accum, p);
 }
 
 __global__ void
@@ -2094,6 +2124,8 @@ wavefront_build(htgx_ctx* ctx, htgx_wavefront_state* st)
   return HTGX_OK;
 }
 
+constexpr uint32_t kChunksPerLane = 4;
+
 /* Launch parameters of one map, its partials and counters aside */
 static int
 fill_launch(htgx_ctx* ctx, const DevMap& M, Launch* P)
@@ -2104,8 +2136,16 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, Launch* P)
   P->height = M.height;
   P->ntx = (M.width + 7) / 8;
   P->ntiles = P->ntx * ((M.height + 7) / 8);
-  /* chunk size: the largest divisor of spp not above K */
-  uint32_t K = std::min(st->K, M.spp);
+  /* chunk size: the largest divisor of spp not above K that leaves at least
+   * kChunksPerLane chunks per resident lane. A chunk's realisations run one
+   * after the other, so on a small map whole chunks would leave lanes idle
+   * and put up to K walks in a row at the end of the launch; the price of
+   * small chunks is 128 B of partial sums moved per chunk. The rule knows the
+   * device's grid and not the caller's, so that the sums do not depend on
+   * the launch parameters other than the chunk size. */
+  const uint64_t nreal = (uint64_t)P->ntiles * 64u * M.spp;
+  const uint64_t most = nreal / ((uint64_t)kChunksPerLane * st->grid_max * kBlock);
+  uint32_t K = (uint32_t)std::min<uint64_t>(std::min(st->K, M.spp), std::max<uint64_t>(1, most));
   while(M.spp % K) --K;
   P->K = K;
   P->nsub = M.spp / K;
@@ -2114,12 +2154,26 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, Launch* P)
   P->ev_thresh = st->ev_thresh;
   P->seg_thresh = st->seg_thresh;
   P->max_steps = 1u << 20;
+  P->lanes = 64;
   const uint64_t nchunks = (uint64_t)P->ntiles * P->nsub * 64u;
   if(nchunks > 0xFFFFFFFFull) return HTGX_BAD_ARG;
   P->nvalid = (uint32_t)((uint64_t)M.width * M.height * P->nsub);
   P->stats = ctx->d_counters;
   P->trunc = st->d_trunc;
   return HTGX_OK;
+}
+
+/* Grid of a launch of its own, at most `grid' blocks: with fewer chunks than
+ * lanes, the chunks spread evenly over all wavefronts (one to a wavefront if
+ * there are that few) instead of filling the first ones: a lane that shares
+ * its wavefront waits for the steps of the others. */
+static uint32_t
+spread_launch(uint32_t grid, Launch* P)
+{
+  const uint64_t nchunks = (uint64_t)P->ntiles * P->nsub * 64u, nw = kBlock / 64;
+  const uint32_t g = (uint32_t)std::min<uint64_t>(grid, (nchunks + nw - 1) / nw);
+  P->lanes = (uint32_t)std::min<uint64_t>(64, (nchunks + nw * g - 1) / (nw * g));
+  return g;
 }
 
 /* Launch parameters of one map; sizes the chunk partials of the context */
@@ -2158,14 +2212,15 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, 
   htgx_wavefront_state* st = ctx->wf;
   Launch P;
   if((res = setup_launch(ctx, M, &P)) != HTGX_OK) return res;
+  const uint32_t grid = spread_launch(st->grid, &P);
   zero_u32_kernel<<<1, 64, 0, stream>>>(st->d_counters, kXcds);
   HIP_OK(hipGetLastError());
   if(ctx->counting) {
     zero_u64_kernel<<<1, 64, 0, stream>>>(ctx->d_counters, HTGX_NSTATS);
     HIP_OK(hipGetLastError());
-    if((res = launch<true>(st->S, M, P, st->grid, stream))) return res;
+    if((res = launch<true>(st->S, M, P, grid, stream))) return res;
   } else {
-    if((res = launch<false>(st->S, M, P, st->grid, stream))) return res;
+    if((res = launch<false>(st->S, M, P, grid, stream))) return res;
   }
   const uint32_t npix = M.width * M.height;
   wf_merge_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(
@@ -2187,7 +2242,16 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum*
   if(!base) return HTGX_BAD_OP;
   Launch P;
   if((res = fill_launch(ctx, M, &P)) != HTGX_OK) return res;
-  const uint64_t need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
+  uint64_t need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
+  if(need > kScratchBytes - kScratchHead && P.K < st->K) {
+    /* small chunks were preferred: the full ones need less scratch */
+    uint32_t K = std::min(st->K, M.spp);
+    while(M.spp % K) --K;
+    P.K = K;
+    P.nsub = M.spp / K;
+    P.nvalid = (uint32_t)((uint64_t)M.width * M.height * P.nsub);
+    need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
+  }
   if(need > kScratchBytes - kScratchHead) {
     fprintf(stderr, "htgx: htgx_render_accum_noalloc: %llu chunk partials of %zu B exceed the "
             "%zu MiB scratch (fewer pixels, fewer realisations per call, or a larger chunk)\n",
@@ -2195,6 +2259,7 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum*
             kScratchBytes >> 20);
     return HTGX_BAD_ARG;
   }
+  const uint32_t grid = spread_launch(st->grid, &P);
   P.counters = (unsigned int*)base;
   P.partials = (htgx_mc_accum*)(base + kScratchHead);
   /* fill kernels, no memset: the call may be captured in a graph */
@@ -2203,9 +2268,9 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum*
   if(ctx->counting) {
     zero_u64_kernel<<<1, 64, 0, stream>>>(ctx->d_counters, HTGX_NSTATS);
     HIP_OK(hipGetLastError());
-    if((res = launch<true>(st->S, M, P, st->grid, stream))) return res;
+    if((res = launch<true>(st->S, M, P, grid, stream))) return res;
   } else {
-    if((res = launch<false>(st->S, M, P, st->grid, stream))) return res;
+    if((res = launch<false>(st->S, M, P, grid, stream))) return res;
   }
   const uint32_t npix = M.width * M.height;
   wf_merge_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P.partials, M.width, M.height, P.ntx,
@@ -2314,7 +2379,7 @@ static int plan_launch_step(htgx_batch_plan* p, hipStream_t stream)
   if(p->single) {
     const BatchScene& e = p->table_h[0];
     int res;
-    if((res = launch<false>(e.S, e.M, e.P, p->grid, stream)) != HTGX_OK) return res;
+    if((res = launch<false>(e.A.S, e.A.M, e.A.P, p->grid, stream)) != HTGX_OK) return res;
   } else switch(p->feat) {
     case 0: launch_batch<0>(p, stream); break;
     case kFeatRare: launch_batch<kFeatRare>(p, stream); break;
@@ -2362,32 +2427,32 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
   for(uint32_t k = 0; k < n; ++k) {
     const uint32_t i = p->order[k];
     BatchScene& e = p->table_h[k];
-    e.S = ctxs[i]->wf->S;
-    e.M = Ms[i];
+    e.A.S = ctxs[i]->wf->S;
+    e.A.M = Ms[i];
     e.accum = accums[i];
-    if((res = setup_launch(ctxs[i], Ms[i], &e.P)) != HTGX_OK) return res;
-    e.P.stats = nullptr;
-    e.P.counters = p->queues + (size_t)k * kXcds;
-    e.P.exhausted = p->flags + k;
-    e.P.done_count = p->flags + n + k;
-    e.P.done_tick = p->ticks + k;
+    if((res = setup_launch(ctxs[i], Ms[i], &e.A.P)) != HTGX_OK) return res;
+    e.A.P.stats = nullptr;
+    e.A.P.counters = p->queues + (size_t)k * kXcds;
+    e.A.P.exhausted = p->flags + k;
+    e.A.P.done_count = p->flags + n + k;
+    e.A.P.done_tick = p->ticks + k;
     if(own_partials) {
       /* the context's partials and wavelength tables may be reallocated by
        * its next map: the plan keeps copies of its own */
-      const size_t np = (size_t)e.P.ntiles * e.P.nsub * 64u;
-      if((res = plan_alloc(p, np, &e.P.partials))) return res;
-      if(e.M.nwbands) {
+      const size_t np = (size_t)e.A.P.ntiles * e.A.P.nsub * 64u;
+      if((res = plan_alloc(p, np, &e.A.P.partials))) return res;
+      if(e.A.M.nwbands) {
         double *cdf = nullptr, *pdf = nullptr;
-        if((res = plan_alloc(p, e.M.nwbands, &cdf)) || (res = plan_alloc(p, e.M.nwbands, &pdf)))
+        if((res = plan_alloc(p, e.A.M.nwbands, &cdf)) || (res = plan_alloc(p, e.A.M.nwbands, &pdf)))
           return res;
-        HIP_OK(hipMemcpy(cdf, e.M.wcdf, e.M.nwbands * sizeof(double), hipMemcpyDeviceToDevice));
-        HIP_OK(hipMemcpy(pdf, e.M.wpdf, e.M.nwbands * sizeof(double), hipMemcpyDeviceToDevice));
-        e.M.wcdf = cdf;
-        e.M.wpdf = pdf;
+        HIP_OK(hipMemcpy(cdf, e.A.M.wcdf, e.A.M.nwbands * sizeof(double), hipMemcpyDeviceToDevice));
+        HIP_OK(hipMemcpy(pdf, e.A.M.wpdf, e.A.M.nwbands * sizeof(double), hipMemcpyDeviceToDevice));
+        e.A.M.wcdf = cdf;
+        e.A.M.wpdf = pdf;
       }
     }
     p->maxpix = std::max(p->maxpix, Ms[i].width * Ms[i].height);
-    p->feat |= features(e.S, e.M);
+    p->feat |= features(e.A.S, e.A.M);
     p->us_per_tick[k] = ctxs[i]->us_per_tick;
   }
   if(n == 1) {
@@ -2396,8 +2461,9 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
      * where batch_advance_kernel moves it on after each step */
     p->single = true;
     BatchScene& e = p->table_h[0];
-    e.P.spp_offset_dev = (const uint32_t*)((const char*)p->table + offsetof(BatchScene, P) +
-                                           offsetof(Launch, spp_offset));
+    p->grid = spread_launch(p->grid, &e.A.P);
+    e.A.P.spp_offset_dev = (const uint32_t*)((const char*)p->table + offsetof(BatchScene, A) +
+                                             offsetof(KArgs, P) + offsetof(Launch, spp_offset));
   }
   HIP_OK(hipMemcpy(p->table, p->table_h.data(), n * sizeof(BatchScene), hipMemcpyHostToDevice));
   HIP_OK(hipMemset(p->flags, 0, (2 * n + 1) * sizeof(unsigned int)));
@@ -2681,6 +2747,7 @@ int htgx_debug_realisations_fp32(htgx_ctx* ctx, const htgx_map_desc* desc, const
     P.ev_thresh = st->ev_thresh;
     P.seg_thresh = st->seg_thresh;
     P.max_steps = 1u << 20;
+    P.lanes = 64;
     P.counters = st->d_counters;
     P.partials = d_acc.p;
     P.nvalid = m;
