@@ -249,7 +249,7 @@ struct Lane {
   uint32_t nsteps;
   /* segment iterator */
   float tit, tnext;    /* iterator position; grid entry or leaf exit */
-  uint32_t lohi[3];    /* leaf block range lo | hi << 16 */
+  float flo[3], fhi[3]; /* leaf range [flo, fhi[ in blocks: whole numbers below 2^16 */
   float lmn, lmx;       /* LWC bounds of the current leaf */
   int32_t j;
   /* current segment */
@@ -491,7 +491,8 @@ __device__ __forceinline__ void face_forwardf(float N[3], const float dir[3])
  * one then spills 8 bytes per lane and still runs faster. */
 struct TrackRegs {
   float lower[3], inv_cs[3];
-  uint32_t def0, def1, B, key, max_steps;
+  float B;               /* cells per block, exact */
+  uint32_t def0, def1, key, max_steps;
   const float* lwc;
   const uint2* leafrec; /* the leaf records and their LWC scale */
   float lwc_scale;
@@ -508,7 +509,7 @@ __device__ __forceinline__ TrackRegs track_regs(const SceneF& S, uint32_t key, u
   }
   g.def0 = S.def[0];
   g.def1 = S.def[1];
-  g.B = S.B;
+  g.B = (float)S.B;
   g.key = key;
   g.max_steps = max_steps;
   g.lwc = S.lwc;
@@ -536,12 +537,30 @@ __device__ __forceinline__ float planef(const SceneF& S, int a, uint32_t k)
   return S.lower[a] + (float)k * S.bs[a];
 }
 
-template<bool COUNT>
+/* Index of element (x, y, z) of a grid of d0 x d1 x .. elements. A 32-bit
+ * multiply takes four times the issue cycles of a 24-bit one: the kernels
+ * without the rare features use the latter, which features() allows for grids
+ * of fewer than 2^24 rows of fewer than 2^24 elements. */
+template<int FEAT>
+__device__ __forceinline__ uint32_t grid_index(uint32_t x, uint32_t y, uint32_t z, uint32_t d0, uint32_t d1)
+{
+  if(FEAT & kFeatRare) return (z * d1 + y) * d0 + x;
+  return __umul24(__umul24(z, d1) + y, d0) + x;
+}
+
+/* f clamped into [lo, hi], all whole but f: the same whole number as clamping
+ * floor(f), with one median instruction and the conversion's truncation */
+__device__ __forceinline__ uint32_t clamp_cell(float f, float lo, float hi)
+{
+  return (uint32_t)__builtin_amdgcn_fmed3f(f, lo, hi);
+}
+
+template<bool COUNT, int FEAT>
 __device__ __forceinline__ void load_leaf(const SceneF& S, const TrackRegs& G, Lane& L, uint32_t cx,
                                           uint32_t cy, uint32_t cz)
 {
   /* one 8-byte load: the leaf's level and its LWC bounds */
-  const uint2 rec = G.leafrec[(cz * S.dims0[1] + cy) * S.dims0[0] + cx];
+  const uint2 rec = G.leafrec[grid_index<FEAT>(cx, cy, cz, S.dims0[0], S.dims0[1])];
   const uint32_t lvl = rec.x >> kLeafIdBits;
   L.lmn = half_bits_to_float(rec.y & 0xFFFFu) * G.lwc_scale;
   L.lmx = half_bits_to_float(rec.y >> 16) * G.lwc_scale;
@@ -552,8 +571,10 @@ __device__ __forceinline__ void load_leaf(const SceneF& S, const TrackRegs& G, L
   for(int a = 0; a < 3; ++a) {
     const uint32_t lo = (c[a] >> lvl) << lvl;
     const uint32_t hi = min(lo + (1u << lvl), S.dims0[a]);
-    L.lohi[a] = lo | (hi << 16);
-    const float ta0 = (planef(S, a, L.dir[a] > 0.f ? hi : lo) - L.pos[a]) * L.inv_dir[a];
+    L.flo[a] = (float)lo;
+    L.fhi[a] = (float)hi;
+    const float plane = S.lower[a] + (L.dir[a] > 0.f ? L.fhi[a] : L.flo[a]) * S.bs[a];
+    const float ta0 = (plane - L.pos[a]) * L.inv_dir[a];
     const float ta = L.dir[a] != 0.f ? ta0 : INFINITY;
     const bool better = ta < best;
     best = better ? ta : best;
@@ -577,16 +598,17 @@ __device__ __forceinline__ bool next_cell(const SceneF& S, Lane& L, uint32_t c[3
   int oa = 0;
 #pragma unroll
   for(int a = 0; a < 3; ++a) {
-    const uint32_t lo = step ? L.lohi[a] & 0xFFFFu : 0u;
-    const uint32_t hi = step ? L.lohi[a] >> 16 : S.dims0[a];
+    const float n = (float)S.dims0[a];
+    const float lo = step ? L.flo[a] : 0.f;
+    const float hi = step ? L.fhi[a] : n;
     const bool pos_dir = L.dir[a] > 0.f;
     const bool across = step && a == L.exit_axis;
-    const bool out_a = across && (pos_dir ? hi >= S.dims0[a] : lo == 0);
+    const bool out_a = across && (pos_dir ? hi >= n : lo == 0.f);
     const float p = L.pos[a] + L.tit * L.dir[a];
-    const float f = floorf((p - S.lower[a]) * S.inv_bs[a]);
-    const uint32_t cl = f < (float)lo ? lo : f > (float)(hi - 1) ? hi - 1 : (uint32_t)f;
-    const uint32_t cs = pos_dir ? hi : lo - 1;
-    c[a] = across ? cs : cl;
+    const float f = (p - S.lower[a]) * S.inv_bs[a];
+    const float cs = pos_dir ? hi : lo - 1.f;
+    const float cl = __builtin_amdgcn_fmed3f(f, lo, hi - 1.f);
+    c[a] = (uint32_t)(across ? cs : cl);
     out = out || out_a;
     oa = out_a ? a : oa;
   }
@@ -700,7 +722,9 @@ __device__ __forceinline__ float gas_depth(const SceneF& S, const Lane& L, int p
   return fabsf(d);
 }
 
-/* Next segment holding some medium into L.s_*; false at the end of the range.
+/* One pass of the segment iterator: the next segment holding some medium into
+ * L.s_* (ITER_SEGMENT), a boundary crossed without one (ITER_AGAIN: call
+ * again), or the end of the range (ITER_END).
  * With `runs' (transmissivity queries, whose gas segments have k_min = k_max
  * and so no collisions), a stretch of the ray outside the cloud grid is one
  * segment over all the gas layers it crosses, up to the grid's entry, the
@@ -709,9 +733,12 @@ __device__ __forceinline__ float gas_depth(const SceneF& S, const Lane& L, int p
  * column of the gas (gas_depth) instead of a sum over its layers.
  * The iterator only moves past an emitted segment at the next call, so that
  * the leaf range used to clamp the cells of its collisions stays the one of
- * the segment. Each pass of the loop loads at most one leaf, at one site. */
+ * the segment. A pass loads at most one leaf, at one site, and the gas
+ * coefficients of its layer ahead of it, so that the two loads overlap: a
+ * wavefront that waits for them alone waited 250 cycles more. */
+enum { ITER_END = 0, ITER_SEGMENT = 1, ITER_AGAIN = 2 };
 template<bool COUNT, int FEAT>
-__device__ __forceinline__ bool iter_next(const SceneF& S, const TrackRegs& G, Lane& L, int prop,
+__device__ __forceinline__ int iter_next(const SceneF& S, const TrackRegs& G, Lane& L, int prop,
                                           float* t0, bool runs = false)
 {
   if(L.adv) {
@@ -719,101 +746,98 @@ __device__ __forceinline__ bool iter_next(const SceneF& S, const TrackRegs& G, L
     iter_advance(L, L.s_t1, L.adv_g, L.adv_c, L.adv_end);
   }
   const float tmax = L.qr;
-  for(;;) {
-    if(L.itdone || !(L.tit < tmax)) return false;
-    if(L.cstate >= 3) {
-      uint32_t c[3];
-      if(next_cell<FEAT>(S, L, c)) { load_leaf<COUNT>(S, G, L, c[0], c[1], c[2]); L.cstate = 1; }
-      else L.cstate = 2;
-    }
-    const float t = L.tit;
-    const float tc = L.cstate == 0 ? L.tnext : L.cstate == 1 ? fmaxf(L.tnext, t) : INFINITY;
-    if(runs && L.cstate != 1 && L.j >= 0 && L.j < (int32_t)S.nlayers && L.dir[2] != 0.f) {
-      /* a gas run: up to the grid's entry, the range's end or the edge of
-       * the gas, whichever comes first */
-      const float ze = L.dir[2] > 0.f ? S.zb + (float)S.nlayers * S.dzl : S.zb;
-      const float tx = fmaxf((ze - L.pos[2]) * L.inv_dir[2], t);
-      const float t1 = fminf(fminf(tc, tx), tmax);
-      if(t1 > t) {
-        const float dcol = gas_depth(S, L, prop, L.pos[2] + t * L.dir[2], L.pos[2] + t1 * L.dir[2]);
-        const float k = dcol * fabsf(L.inv_dir[2]) / (t1 - t);
-        *t0 = t;
-        L.s_t1 = t1;
-        L.s_kmin = L.s_kmax = k;
-        L.s_gka = L.s_gks = 0.f;
-        L.s_cloud = false;
-        L.s_layer = L.j;
-        /* past the run: the layer the ray is in just beyond t1 (or out of
-         * the gas), the grid entered if the run ended there */
-        const float zf = (L.pos[2] + t1 * L.dir[2] - S.zb) * S.inv_dzl;
-        int32_t j1 = L.dir[2] > 0.f ? (int32_t)floorf(zf) : (int32_t)ceilf(zf) - 1;
-        if(t1 == tx) j1 = L.dir[2] > 0.f ? (int32_t)S.nlayers : -1;
-        L.j = j1 < -1 ? -1 : j1 > (int32_t)S.nlayers ? (int32_t)S.nlayers : j1;
-        L.adv = true;
-        L.adv_g = false;
-        L.adv_c = tc == t1;
-        L.adv_end = tc == INFINITY && t1 == tx;
-        L.nsteps &= kCollMask;
-        if(COUNT) L.c_seg++;
-        return true;
-      }
-    }
-    float tg;
-    if(L.dir[2] > 0.f && L.j < (int32_t)S.nlayers) tg = (S.zb + (float)(L.j + 1) * S.dzl - L.pos[2]) * L.inv_dir[2];
-    else if(L.dir[2] < 0.f && L.j >= 0) tg = (S.zb + (float)L.j * S.dzl - L.pos[2]) * L.inv_dir[2];
-    else tg = INFINITY;
-    tg = fmaxf(tg, t);
-    const float t1 = fminf(fminf(tc, tg), tmax);
-    const bool at_end = tg == INFINITY && tc == INFINITY;
-    const bool in_gas = L.j >= 0 && L.j < (int32_t)S.nlayers;
-    const bool in_cloud = L.cstate == 1;
-    if(t1 > t && (in_gas || in_cloud)) {
-      float gka = 0.f, gks = 0.f, cmn = 0.f, cmx = 0.f;
-      if(in_gas) {
-        gka = S.gas_ka[L.gka_off + (uint32_t)L.j];
-        gks = S.gas_ks[L.gks_off + (uint32_t)L.j];
-      }
-      if(in_cloud) {
-        const float c = prop == HTGX_Ka ? L.cka : prop == HTGX_Ks ? L.cks : L.cka + L.cks;
-        cmn = c * L.lmn;
-        cmx = c * L.lmx;
-      }
-      const float gk = prop == HTGX_Ka ? gka : prop == HTGX_Ks ? gks : gka + gks;
+  if(L.itdone || !(L.tit < tmax)) return ITER_END;
+  const bool in_gas = L.j >= 0 && L.j < (int32_t)S.nlayers;
+  float gka = 0.f, gks = 0.f;
+  if(in_gas) {
+    gka = S.gas_ka[L.gka_off + (uint32_t)L.j];
+    gks = S.gas_ks[L.gks_off + (uint32_t)L.j];
+  }
+  if(L.cstate >= 3) {
+    uint32_t c[3];
+    if(next_cell<FEAT>(S, L, c)) { load_leaf<COUNT, FEAT>(S, G, L, c[0], c[1], c[2]); L.cstate = 1; }
+    else L.cstate = 2;
+  }
+  const float t = L.tit;
+  const float tc = L.cstate == 0 ? L.tnext : L.cstate == 1 ? fmaxf(L.tnext, t) : INFINITY;
+  if(runs && L.cstate != 1 && in_gas && L.dir[2] != 0.f) {
+    /* a gas run: up to the grid's entry, the range's end or the edge of
+     * the gas, whichever comes first */
+    const float ze = L.dir[2] > 0.f ? S.zb + (float)S.nlayers * S.dzl : S.zb;
+    const float tx = fmaxf((ze - L.pos[2]) * L.inv_dir[2], t);
+    const float t1 = fminf(fminf(tc, tx), tmax);
+    if(t1 > t) {
+      const float dcol = gas_depth(S, L, prop, L.pos[2] + t * L.dir[2], L.pos[2] + t1 * L.dir[2]);
+      const float k = dcol * fabsf(L.inv_dir[2]) / (t1 - t);
       *t0 = t;
       L.s_t1 = t1;
-      L.s_kmin = gk + cmn;
-      L.s_kmax = gk + cmx;
-      L.s_gka = gka;
-      L.s_gks = gks;
-      L.s_cloud = in_cloud;
-      L.s_layer = in_gas ? L.j : -1;
+      L.s_kmin = L.s_kmax = k;
+      L.s_gka = L.s_gks = 0.f;
+      L.s_cloud = false;
+      L.s_layer = L.j;
+      /* past the run: the layer the ray is in just beyond t1 (or out of
+       * the gas), the grid entered if the run ended there */
+      const float zf = (L.pos[2] + t1 * L.dir[2] - S.zb) * S.inv_dzl;
+      int32_t j1 = L.dir[2] > 0.f ? (int32_t)floorf(zf) : (int32_t)ceilf(zf) - 1;
+      if(t1 == tx) j1 = L.dir[2] > 0.f ? (int32_t)S.nlayers : -1;
+      L.j = j1 < -1 ? -1 : j1 > (int32_t)S.nlayers ? (int32_t)S.nlayers : j1;
       L.adv = true;
-      L.adv_g = tg == t1;
+      L.adv_g = false;
       L.adv_c = tc == t1;
-      L.adv_end = at_end;
+      L.adv_end = tc == INFINITY && t1 == tx;
       L.nsteps &= kCollMask;
       if(COUNT) L.c_seg++;
-      return true;
+      return ITER_SEGMENT;
     }
-    iter_advance(L, t1, tg == t1, tc == t1, at_end);
-    if((L.nsteps >> kCollBits) >= kMaxEmptyPasses) { L.itdone = true; return false; }
-    L.nsteps += 1u << kCollBits;
   }
+  float tg;
+  if(L.dir[2] > 0.f && L.j < (int32_t)S.nlayers) tg = (S.zb + (float)(L.j + 1) * S.dzl - L.pos[2]) * L.inv_dir[2];
+  else if(L.dir[2] < 0.f && L.j >= 0) tg = (S.zb + (float)L.j * S.dzl - L.pos[2]) * L.inv_dir[2];
+  else tg = INFINITY;
+  tg = fmaxf(tg, t);
+  const float t1 = fminf(fminf(tc, tg), tmax);
+  const bool at_end = tg == INFINITY && tc == INFINITY;
+  const bool in_cloud = L.cstate == 1;
+  if(t1 > t && (in_gas || in_cloud)) {
+    float cmn = 0.f, cmx = 0.f;
+    if(in_cloud) {
+      const float c = prop == HTGX_Ka ? L.cka : prop == HTGX_Ks ? L.cks : L.cka + L.cks;
+      cmn = c * L.lmn;
+      cmx = c * L.lmx;
+    }
+    const float gk = prop == HTGX_Ka ? gka : prop == HTGX_Ks ? gks : gka + gks;
+    *t0 = t;
+    L.s_t1 = t1;
+    L.s_kmin = gk + cmn;
+    L.s_kmax = gk + cmx;
+    L.s_gka = gka;
+    L.s_gks = gks;
+    L.s_cloud = in_cloud;
+    L.s_layer = in_gas ? L.j : -1;
+    L.adv = true;
+    L.adv_g = tg == t1;
+    L.adv_c = tc == t1;
+    L.adv_end = at_end;
+    L.nsteps &= kCollMask;
+    if(COUNT) L.c_seg++;
+    return ITER_SEGMENT;
+  }
+  iter_advance(L, t1, tg == t1, tc == t1, at_end);
+  if((L.nsteps >> kCollBits) >= kMaxEmptyPasses) { L.itdone = true; return ITER_END; }
+  L.nsteps += 1u << kCollBits;
+  return ITER_AGAIN;
 }
 
 /* LWC of the cell holding x, clamped into the current segment's leaf */
-template<bool COUNT>
+template<bool COUNT, int FEAT>
 __device__ __forceinline__ float seg_lwcf(const TrackRegs& G, Lane& L, const float x[3])
 {
   uint32_t ci[3];
 #pragma unroll
-  for(int a = 0; a < 3; ++a) {
-    const uint32_t lo = (L.lohi[a] & 0xFFFFu) * G.B, hi = (L.lohi[a] >> 16) * G.B - 1;
-    const float f = floorf((x[a] - G.lower[a]) * G.inv_cs[a]);
-    ci[a] = f < (float)lo ? lo : f > (float)hi ? hi : (uint32_t)f;
-  }
+  for(int a = 0; a < 3; ++a)
+    ci[a] = clamp_cell((x[a] - G.lower[a]) * G.inv_cs[a], L.flo[a] * G.B, L.fhi[a] * G.B - 1.f);
   if(COUNT) L.c_lwc++;
-  return G.lwc[(ci[2] * G.def1 + ci[1]) * G.def0 + ci[0]];
+  return G.lwc[grid_index<FEAT>(ci[0], ci[1], ci[2], G.def0, G.def1)];
 }
 
 /*******************************************************************************
@@ -1336,7 +1360,8 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
       /* longwave kernels run MODE_LW queries only, shortwave ones MODE_SC
        * and MODE_TR: the other modes' code is compiled out */
       const int sprop = kLW ? HTGX_Kext : L.mode == MODE_SC ? HTGX_Ks : L.prop;
-      if(iter_next<COUNT, FEAT>(S, G, L, sprop, &t0, !kLW && L.mode == MODE_TR)) {
+      const int it = iter_next<COUNT, FEAT>(S, G, L, sprop, &t0, !kLW && L.mode == MODE_TR);
+      if(it == ITER_SEGMENT) {
         const float len = L.s_t1 - t0;
         if(!kLW && L.mode == MODE_TR) L.Tmin += (double)len * (double)L.s_kmin;
         if(!kLW && L.mode == MODE_SC) {
@@ -1365,6 +1390,8 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
           L.tc = t0 + L.Ts * L.inv_maj;
           L.lstate = LS_COLL;
         }
+      } else if(it == ITER_AGAIN) {
+        /* the next pass with the next segment step */
       } else if(L.lazy) {
         /* the query reached the top of the mesh ground without an event:
          * cast the ray on the ground now, then go on up to the hit */
@@ -1399,7 +1426,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
         float x[3];
 #pragma unroll
         for(int a = 0; a < 3; ++a) x[a] = L.pos[a] + tx * L.dir[a];
-        const float v = L.s_cloud ? seg_lwcf<COUNT>(G, L, x) : 0.f;
+        const float v = L.s_cloud ? seg_lwcf<COUNT, FEAT>(G, L, x) : 0.f;
         /* the draw does not depend on the LWC: written before the LWC's
          * first use, its Threefry rounds run while the load is in flight */
         const float2 uu = draw2(L, key);
@@ -1676,7 +1703,10 @@ wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop,
   uint32_t n = 0;
   float t0;
   const TrackRegs G = track_regs<false>(S, 0u, 0u);
-  while(iter_next<false, kFeatRare>(S, G, L, prop, &t0)) {
+  for(;;) {
+    const int it = iter_next<false, kFeatRare>(S, G, L, prop, &t0);
+    if(it == ITER_END) break;
+    if(it == ITER_AGAIN) continue;
     if(n < max_segs) {
       htgx_segment& o = segs[(size_t)i * max_segs + n];
       o.t0 = t0;
@@ -1685,7 +1715,7 @@ wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop,
       o.kmax = L.s_kmax;
       o.leaf = -1;
       if(L.s_cloud) {
-        const uint32_t c[3] = {L.lohi[0] & 0xFFFFu, L.lohi[1] & 0xFFFFu, L.lohi[2] & 0xFFFFu};
+        const uint32_t c[3] = {(uint32_t)L.flo[0], (uint32_t)L.flo[1], (uint32_t)L.flo[2]};
         o.leaf = S.leafrec[(c[2] * S.dims0[1] + c[1]) * S.dims0[0] + c[0]].x & kLeafIdMask;
       }
       o.layer = L.s_layer;
@@ -1839,8 +1869,10 @@ int launch_variant(F kernel, const SceneF& S, const DevMap& M, const Launch& P, 
 /* The kernel features a map needs (kFeatRare, kFeatMesh) */
 int features(const SceneF& S, const DevMap& M)
 {
+  /* (also grids too large for the 24-bit index arithmetic, grid_index) */
   const bool rare = S.repeat || S.ground_repeat || S.gmat || M.ortho || M.lens_radius > 0 ||
-                    M.wmode == 3 || M.wmode == 2;
+                    M.wmode == 3 || M.wmode == 2 ||
+                    (uint64_t)S.def[1] * S.def[2] >= (1u << 24) || S.def[0] >= (1u << 24);
   return (rare ? kFeatRare : 0) | (S.ground_type == HTGX_GROUND_MESH ? kFeatMesh : 0);
 }
 
