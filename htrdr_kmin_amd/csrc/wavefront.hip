@@ -299,14 +299,43 @@ constexpr uint32_t kMaxEmptyPasses = 2000;
  * with counter (pair index, seed) under the key (pixel, realisation). The
  * numbers of a realisation depend only on its key and on how many pairs it
  * drew before, not on the lanes it shares a wavefront with. */
-__device__ __forceinline__ float2 draw2(Lane& L, uint32_t key)
+__device__ __forceinline__ float2 draw_at(const Lane& L, uint32_t pair, uint32_t key)
 {
-  const uint32_t ctr[2] = {L.pair, key};
+  const uint32_t ctr[2] = {pair, key};
   const uint32_t k[2] = {L.pixel, L.r};
   uint32_t out[2];
   threefry2x32_20(ctr, k, out);
-  L.pair += 1;
   return make_float2((float)(out[0] >> 8) * 0x1.0p-24f, (float)(out[1] >> 8) * 0x1.0p-24f);
+}
+
+__device__ __forceinline__ float2 draw2(Lane& L, uint32_t key)
+{
+  return draw_at(L, L.pair++, key);
+}
+
+/* Which blocks of its event's draws a lane has a use for: 0 and 1 (u[0..3],
+ * directions and films), 2 (u[4..5], phase choice, roulette). Every event takes
+ * the same number of blocks from its stream, used or not. */
+struct EventDraws {
+  bool d0, d1, d2;
+};
+template<int SPECTRAL, int FEAT>
+__device__ __forceinline__ EventDraws event_draws(const SceneF& S, const Lane& L, int stage)
+{
+  const bool begin = stage == ST_BEGIN;
+  EventDraws d;
+  if(SPECTRAL == HTGX_SPECTRAL_LW) {
+    const bool surface = L.pending && L.ev == EV_NONE && L.gh_hit;
+    d.d0 = begin || surface || (L.pending && L.ev == EV_SCA);
+    d.d1 = begin;
+    /* a BRDF list picks its entry with u[4] */
+    d.d2 = begin || (has_gmat<FEAT>(S) && surface);
+  } else {
+    const bool walk = L.pending && stage == ST_SCATTER && L.ev != EV_ABS && (L.gh_hit || L.ev == EV_HIT);
+    d.d0 = d.d1 = begin || walk;
+    d.d2 = begin || walk || (L.pending && stage == ST_SUN && L.surface);
+  }
+  return d;
 }
 
 /* Exp(1) sample from a canonical, ssp_ran_exp(rng, 1) */
@@ -480,25 +509,24 @@ __device__ __forceinline__ void face_forwardf(float N[3], const float dir[3])
   }
 }
 
-/* What the tracking steps read of the scene at every step (the cloud grid's
- * addressing, the leaf records, the random-stream key, the collision
- * budget). With VREG they are held in vector registers for the whole launch
- * (the empty asm statements make them lane values): in scalar registers
- * they stay live across the whole loop, where the kernel runs out of scalar
- * registers, and are reloaded from their spill slots at every step. The
- * kernels with the rare features have no vector registers to spare and keep
- * them in scalar ones. The mesh kernels keep the copy: the shortwave flux
- * one then spills 8 bytes per lane and still runs faster. */
+using GlobalF = const __attribute__((address_space(1))) float*;
+using GlobalU64 = const __attribute__((address_space(1))) uint64_t*;
+
+/* What the tracking steps read of the scene at every step: the cloud grid's
+ * addressing, the leaf records, the random-stream key, the collision budget.
+ * In scalar registers: the event step's constants are in LDS (g_args), which
+ * leaves room for these. Vector copies of them measured no faster on the
+ * image (296 against 298 ms) and cost the terrain map's kernel 52 bytes of
+ * spills a lane (228 against 194 ms). */
 struct TrackRegs {
   float lower[3], inv_cs[3];
   float B;               /* cells per block, exact */
   uint32_t def0, def1, key, max_steps;
-  const float* lwc;
-  const uint2* leafrec; /* the leaf records and their LWC scale */
+  GlobalF lwc;
+  GlobalU64 leafrec;    /* the leaf records and their LWC scale */
   float lwc_scale;
 };
 
-template<bool VREG>
 __device__ __forceinline__ TrackRegs track_regs(const SceneF& S, uint32_t key, uint32_t max_steps)
 {
   TrackRegs g;
@@ -512,15 +540,9 @@ __device__ __forceinline__ TrackRegs track_regs(const SceneF& S, uint32_t key, u
   g.B = (float)S.B;
   g.key = key;
   g.max_steps = max_steps;
-  g.lwc = S.lwc;
-  g.leafrec = S.leafrec;
+  g.lwc = (GlobalF)S.lwc;
+  g.leafrec = (GlobalU64)S.leafrec;
   g.lwc_scale = S.lwc_scale;
-  if(VREG) {
-    asm volatile("" : "+v"(g.lower[0]), "+v"(g.lower[1]), "+v"(g.lower[2]), "+v"(g.inv_cs[0]),
-                      "+v"(g.inv_cs[1]), "+v"(g.inv_cs[2]));
-    asm volatile("" : "+v"(g.def0), "+v"(g.def1), "+v"(g.B), "+v"(g.key), "+v"(g.max_steps),
-                      "+v"(g.lwc), "+v"(g.leafrec), "+v"(g.lwc_scale));
-  }
   return g;
 }
 
@@ -560,10 +582,10 @@ __device__ __forceinline__ void load_leaf(const SceneF& S, const TrackRegs& G, L
                                           uint32_t cy, uint32_t cz)
 {
   /* one 8-byte load: the leaf's level and its LWC bounds */
-  const uint2 rec = G.leafrec[grid_index<FEAT>(cx, cy, cz, S.dims0[0], S.dims0[1])];
-  const uint32_t lvl = rec.x >> kLeafIdBits;
-  L.lmn = half_bits_to_float(rec.y & 0xFFFFu) * G.lwc_scale;
-  L.lmx = half_bits_to_float(rec.y >> 16) * G.lwc_scale;
+  const uint64_t rec = G.leafrec[grid_index<FEAT>(cx, cy, cz, S.dims0[0], S.dims0[1])];
+  const uint32_t lvl = (uint32_t)rec >> kLeafIdBits, bnd = (uint32_t)(rec >> 32);
+  L.lmn = half_bits_to_float(bnd & 0xFFFFu) * G.lwc_scale;
+  L.lmx = half_bits_to_float(bnd >> 16) * G.lwc_scale;
   const uint32_t c[3] = {cx, cy, cz};
   float best = INFINITY;
   int ax = 0;
@@ -681,20 +703,21 @@ __device__ __forceinline__ void iter_init(const SceneF& S, Lane& L)
   L.j = fj < -1.f ? -1 : fj > (float)S.nlayers ? (int32_t)S.nlayers : (int32_t)fj;
 }
 
-/* Move the iterator past a boundary at t1 (gas layer if adv_g, leaf or grid
- * entry if adv_c). No memory access: a leaf boundary only marks the leaf to
- * load next (state 3 or 4). */
-__device__ __forceinline__ void iter_advance(Lane& L, float t1, bool adv_g, bool adv_c,
-                                             bool at_end)
+/* Move the iterator past the boundary its last pass stopped at, s_t1 (gas
+ * layer if adv_g, leaf or grid entry if adv_c; the end of the range ends it).
+ * No memory access: a leaf boundary only marks the leaf to load next (state 3
+ * or 4). Selects, not branches: a wavefront of few lanes pays more for the
+ * jumps than for the instructions. */
+__device__ __forceinline__ void iter_advance(Lane& L)
 {
-  if(t1 >= L.qr) { L.itdone = true; return; }
-  L.tit = t1;
-  if(adv_g) L.j += L.dir[2] > 0.f ? 1 : -1;
-  if(adv_c) {
-    if(L.cstate == 0) L.cstate = 3;
-    else if(L.cstate == 1) L.cstate = 4;
-  }
-  if(at_end) L.itdone = true;
+  const bool end = L.s_t1 >= L.qr;
+  const bool move = L.adv && !end;
+  L.itdone = L.itdone || (L.adv && (end || L.adv_end));
+  L.tit = move ? L.s_t1 : L.tit;
+  const int32_t dj = L.dir[2] > 0.f ? 1 : -1;
+  L.j += move && L.adv_g ? dj : 0;
+  L.cstate += move && L.adv_c && L.cstate < 2 ? 3 : 0;
+  L.adv = false;
 }
 
 /* Vertical optical depth of the gas between heights za and zb (clamped into
@@ -741,12 +764,9 @@ template<bool COUNT, int FEAT>
 __device__ __forceinline__ int iter_next(const SceneF& S, const TrackRegs& G, Lane& L, int prop,
                                           float* t0, bool runs = false)
 {
-  if(L.adv) {
-    L.adv = false;
-    iter_advance(L, L.s_t1, L.adv_g, L.adv_c, L.adv_end);
-  }
+  iter_advance(L);
   const float tmax = L.qr;
-  if(L.itdone || !(L.tit < tmax)) return ITER_END;
+  if(L.itdone || !(L.tit < tmax) || (L.nsteps >> kCollBits) > kMaxEmptyPasses) return ITER_END;
   const bool in_gas = L.j >= 0 && L.j < (int32_t)S.nlayers;
   float gka = 0.f, gks = 0.f;
   if(in_gas) {
@@ -798,34 +818,29 @@ __device__ __forceinline__ int iter_next(const SceneF& S, const TrackRegs& G, La
   const float t1 = fminf(fminf(tc, tg), tmax);
   const bool at_end = tg == INFINITY && tc == INFINITY;
   const bool in_cloud = L.cstate == 1;
-  if(t1 > t && (in_gas || in_cloud)) {
-    float cmn = 0.f, cmx = 0.f;
-    if(in_cloud) {
-      const float c = prop == HTGX_Ka ? L.cka : prop == HTGX_Ks ? L.cks : L.cka + L.cks;
-      cmn = c * L.lmn;
-      cmx = c * L.lmx;
-    }
-    const float gk = prop == HTGX_Ka ? gka : prop == HTGX_Ks ? gks : gka + gks;
-    *t0 = t;
-    L.s_t1 = t1;
-    L.s_kmin = gk + cmn;
-    L.s_kmax = gk + cmx;
-    L.s_gka = gka;
-    L.s_gks = gks;
-    L.s_cloud = in_cloud;
-    L.s_layer = in_gas ? L.j : -1;
-    L.adv = true;
-    L.adv_g = tg == t1;
-    L.adv_c = tc == t1;
-    L.adv_end = at_end;
-    L.nsteps &= kCollMask;
-    if(COUNT) L.c_seg++;
-    return ITER_SEGMENT;
+  const float c = !in_cloud ? 0.f : prop == HTGX_Ka ? L.cka : prop == HTGX_Ks ? L.cks : L.cka + L.cks;
+  const float cmn = in_cloud ? c * L.lmn : 0.f, cmx = in_cloud ? c * L.lmx : 0.f;
+  const float gk = prop == HTGX_Ka ? gka : prop == HTGX_Ks ? gks : gka + gks;
+  /* the iterator moves past this boundary at the next pass */
+  L.s_t1 = t1;
+  L.adv = true;
+  L.adv_g = tg == t1;
+  L.adv_c = tc == t1;
+  L.adv_end = at_end;
+  if(!(t1 > t && (in_gas || in_cloud))) {
+    L.nsteps += 1u << kCollBits;
+    return ITER_AGAIN;
   }
-  iter_advance(L, t1, tg == t1, tc == t1, at_end);
-  if((L.nsteps >> kCollBits) >= kMaxEmptyPasses) { L.itdone = true; return ITER_END; }
-  L.nsteps += 1u << kCollBits;
-  return ITER_AGAIN;
+  *t0 = t;
+  L.s_kmin = gk + cmn;
+  L.s_kmax = gk + cmx;
+  L.s_gka = gka;
+  L.s_gks = gks;
+  L.s_cloud = in_cloud;
+  L.s_layer = in_gas ? L.j : -1;
+  L.nsteps &= kCollMask;
+  if(COUNT) L.c_seg++;
+  return ITER_SEGMENT;
 }
 
 /* LWC of the cell holding x, clamped into the current segment's leaf */
@@ -1293,7 +1308,6 @@ __shared__ KArgs g_args[kBlock / 64];
 template<int SENSOR, int SPECTRAL, bool COUNT, int FEAT, bool LIST = false>
 __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
 {
-  constexpr bool RARE = (FEAT & kFeatRare) != 0;
   constexpr bool kLW = SPECTRAL == HTGX_SPECTRAL_LW;
   const SceneF S = kload(&pK->S);
   const Launch P = kload(&pK->P);
@@ -1325,7 +1339,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
   const uint32_t xcd = blockIdx.x % (uint32_t)kXcds;
   uint32_t tried = 0; /* chunk ranges found empty */
   const TrackRegs G =
-      track_regs<!RARE>(S, (uint32_t)seed ^ (uint32_t)(seed >> 32), P.max_steps);
+      track_regs(S, (uint32_t)seed ^ (uint32_t)(seed >> 32), P.max_steps);
   const uint32_t key = G.key;
   uint64_t d_it = 0, d_ce = 0, d_cl = 0, d_se = 0, d_sl = 0, d_ee = 0, d_el = 0;
   /* shader clock cycles per phase (counting build only) */
@@ -1400,7 +1414,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
         L.nq_ground = 2;
         L.lstate = LS_EVENT;
       } else {
-        if(P.trunc && (L.nsteps >> kCollBits) >= kMaxEmptyPasses) atomicAdd(P.trunc + 1, 1ull);
+        if(P.trunc && (L.nsteps >> kCollBits) > kMaxEmptyPasses) atomicAdd(P.trunc + 1, 1ull);
         L.ev = EV_NONE;
         L.pending = true;
         L.lstate = LS_EVENT;
@@ -1488,6 +1502,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
     if(want && (__popcll(want) >= ev_min || !other)) {
       /* the index is opaque to the optimiser (an empty asm statement), so
        * that the reads stay where they are written */
+      const SceneF& S_t = S; /* what the tracking steps keep in registers */
       uint32_t wv = wave;
       asm volatile("" : "+s"(wv));
       const SceneF& S = g_args[wv].S;
@@ -1546,7 +1561,35 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
         /* one set of canonicals per event, drawn at a single site */
         float u[2 * NP];
 #pragma unroll
-        for(int i = 0; i < NP; ++i) { const float2 v = draw2(L, key); u[2 * i] = v.x; u[2 * i + 1] = v.y; }
+        for(int i = 0; i < 2 * NP; ++i) u[i] = 0.f;
+        const EventDraws need = event_draws<SPECTRAL, FEAT>(S, L, LC(stage));
+        /* two blocks side by side: a block is a chain of 50 dependent
+         * instructions, and a wavefront alone on its SIMD waits 8 cycles for
+         * each where two chains fill the gaps. The last block (the optical
+         * thickness of the next query) is every event's; beside it runs block
+         * 0 or, for a lane with no use for that, the block after the event's
+         * own, which gives a shortwave scattering query its second optical
+         * thickness. Blocks 1 and 2 follow for the lanes that use them. */
+        const float2 vl = draw_at(L, L.pair + (uint32_t)(NP - 1), key);
+        const float2 v0 = draw_at(L, L.pair + (need.d0 ? 0u : (uint32_t)NP), key);
+        u[2 * NP - 2] = vl.x;
+        u[2 * NP - 1] = vl.y;
+        u[0] = v0.x;
+        u[1] = v0.y;
+        const bool have_a = !need.d0;
+        if(need.d1 || need.d2) {
+          const float2 v1 = draw_at(L, L.pair + 1u, key), v2 = draw_at(L, L.pair + 2u, key);
+          u[2] = v1.x;
+          u[3] = v1.y;
+          u[4] = v2.x;
+          u[5] = v2.y;
+        }
+        if(NP > 4 && begin) {
+          const float2 v3 = draw_at(L, L.pair + 3u, key);
+          u[6] = v3.x;
+          u[7] = v3.y;
+        }
+        L.pair += NP;
         WF_TICK(3)
         if(begin) {
           real_begin<SENSOR, SPECTRAL, COUNT, FEAT>(S, M, L, u);
@@ -1619,8 +1662,13 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
             L.Ts = exp1f(u[2 * NP - 1]);
             L.Tmin = 0.0;
             L.pending = false;
-            if(!kLW && L.mode == MODE_SC) L.Ts_a = exp1f(draw2(L, key).x);
-            iter_init<FEAT>(S, L);
+            if(!kLW && L.mode == MODE_SC) {
+              float ua = v0.x;
+              if(!have_a) ua = draw_at(L, L.pair, key).x;
+              L.pair++;
+              L.Ts_a = exp1f(ua);
+            }
+            iter_init<FEAT>(S_t, L);
           }
           L.tc = L.tc_a = INFINITY;
           L.lstate = LS_SEG;
@@ -1702,7 +1750,7 @@ wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop,
   iter_init<kFeatRare>(S, L);
   uint32_t n = 0;
   float t0;
-  const TrackRegs G = track_regs<false>(S, 0u, 0u);
+  const TrackRegs G = track_regs(S, 0u, 0u);
   for(;;) {
     const int it = iter_next<false, kFeatRare>(S, G, L, prop, &t0);
     if(it == ITER_END) break;
