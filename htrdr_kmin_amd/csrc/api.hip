@@ -38,128 +38,6 @@ using namespace htgx;
  ******************************************************************************/
 namespace {
 
-/* Pixel of item i of a realisation slice: 8x8 tiles (one wavefront per tile,
- * the tile size of src/core/htrdr_draw_map.c:45), pixels of a tile in Morton
- * order like draw_tile (src/core/htrdr_draw_map.c:301-319). */
-__device__ __forceinline__ void
-tile_pixel(uint32_t i, uint32_t ntx, uint32_t* x, uint32_t* y)
-{
-  const uint32_t tile = i >> 6, m = i & 63u;
-  *x = (tile % ntx) * 8u + ((m & 1u) | ((m >> 1) & 2u) | ((m >> 2) & 4u));
-  *y = (tile / ntx) * 8u + (((m >> 1) & 1u) | ((m >> 2) & 2u) | ((m >> 3) & 4u));
-}
-
-__device__ __forceinline__ uint64_t
-wave_sum(uint64_t v)
-{
-  for(int off = 32; off > 0; off >>= 1)
-    v += (uint64_t)__shfl_xor((unsigned long long)v, off, 64);
-  return v;
-}
-
-__device__ __forceinline__ void
-flush_counters(const Counters& c, unsigned long long* counters)
-{
-  const uint64_t a = wave_sum(c.nleaf), b = wave_sum(c.nseg), d = wave_sum(c.ncoll),
-                 e = wave_sum(c.ncell), f = wave_sum(c.nev);
-  if((threadIdx.x & 63u) == 0) {
-    atomicAdd(counters + 1, (unsigned long long)a);
-    atomicAdd(counters + 2, (unsigned long long)b);
-    atomicAdd(counters + 3, (unsigned long long)d);
-    atomicAdd(counters + 4, (unsigned long long)e);
-    atomicAdd(counters + 5, (unsigned long long)f);
-  }
-}
-
-/* One thread = one pixel x one slice of its realisations, one path at a
- * time, FP64 throughout: the "plain" solver and the FP64 GPU oracle. It is
- * the device counterpart of draw_pixel_xwave / draw_pixel_flux
- * (src/atmosphere/htrdr_atmosphere_draw_map.c:210-436) driven by the tile
- * loop of draw_map (src/core/htrdr_draw_map.c:324-491). */
-template<bool COUNT>
-__global__ void __launch_bounds__(256)
-plain_kernel(DevScene S, DevMap M, uint32_t ntx, uint32_t items_per_slice,
-             uint32_t nslices, uint32_t spt, htgx_mc_accum* partials,
-             unsigned long long* counters)
-{
-  const uint64_t item = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  Counters cnt = {0, 0, 0, 0, 0};
-  uint32_t x = 0, y = 0, slice = 0;
-  bool active = item < (uint64_t)items_per_slice * nslices;
-  if(active) {
-    slice = (uint32_t)(item / items_per_slice);
-    tile_pixel((uint32_t)(item % items_per_slice), ntx, &x, &y);
-    active = x < M.width && y < M.height;
-  }
-  if(active) {
-    const uint64_t npix = (uint64_t)M.width * M.height;
-    const uint64_t pixel = (uint64_t)y * M.width + x;
-    const uint32_t rb = slice * spt;
-    const uint32_t re = min(rb + spt, M.spp);
-    Counters* pc = COUNT ? &cnt : nullptr;
-    htgx_mc_accum a;
-    a.sum = a.sum_c = a.sum2 = a.sum2_c = a.tsum = a.tsum2 = 0;
-    a.n = a.nfail = 0;
-    Path P;
-    Stream rng;
-    TrackOut out;
-    uint32_t r = rb;
-    uint64_t t0 = wall_clock64();
-    real_begin(S, M, P, rng, pixel, (uint64_t)M.spp_offset + r);
-    /* Flat loop: a lane whose realisation ends starts its next one at once
-     * instead of waiting at a per-realisation barrier for the other lanes. */
-    while(r < re) {
-      while(P.stage == ST_WALK_DONE) walk_done(S, M, P);
-      if(P.stage == ST_REAL_DONE) {
-        const uint64_t t1 = wall_clock64();
-        if(P.rejected) {
-          a.nfail++;
-        } else {
-          const double us = (double)(t1 - t0) * M.us_per_tick;
-          nsum(a.sum, a.sum_c, P.weight);
-          nsum(a.sum2, a.sum2_c, P.weight * P.weight);
-          a.tsum += us;
-          a.tsum2 += us * us;
-          a.n++;
-        }
-        if(++r >= re) break;
-        t0 = t1;
-        real_begin(S, M, P, rng, pixel, (uint64_t)M.spp_offset + r);
-        continue;
-      }
-      int mode, prop;
-      double o[3], d[3], r1;
-      stage_query(P, &mode, &prop, o, d, &r1);
-      track(S, rng, mode, prop, P.iband, P.iquad, o, d, r1, out, pc);
-      stage_consume(S, P, rng, out, pc);
-    }
-    partials[(size_t)slice * npix + pixel] = a;
-  }
-  if(COUNT) flush_counters(cnt, counters);
-}
-
-/* Fold the slices of each pixel, in slice order, into its accumulator */
-__global__ void __launch_bounds__(256)
-merge_kernel(const htgx_mc_accum* partials, uint32_t nslices, uint64_t npix,
-             htgx_mc_accum* accum)
-{
-  const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if(p >= npix) return;
-  htgx_mc_accum a = accum[p];
-  for(uint32_t s = 0; s < nslices; ++s) {
-    const htgx_mc_accum q = partials[(size_t)s * npix + p];
-    nsum(a.sum, a.sum_c, q.sum);
-    a.sum_c += q.sum_c;
-    nsum(a.sum2, a.sum2_c, q.sum2);
-    a.sum2_c += q.sum2_c;
-    a.tsum += q.tsum;
-    a.tsum2 += q.tsum2;
-    a.n += q.n;
-    a.nfail += q.nfail;
-  }
-  accum[p] = a;
-}
-
 __global__ void
 trace_segments_kernel(DevScene S, const double* rays, uint32_t nrays, int prop,
                       uint32_t iband, uint32_t iquad, htgx_segment* segs,
@@ -889,6 +767,7 @@ htgx_ctx_destroy(htgx_ctx* ctx)
   if(!ctx) return HTGX_BAD_ARG;
   for(void* p : ctx->bufs) (void)hipFree(p);
   if(ctx->d_partials) (void)hipFree(ctx->d_partials);
+  if(ctx->d_plain_queue) (void)hipFree(ctx->d_plain_queue);
   if(ctx->d_wcdf) (void)hipFree(ctx->d_wcdf);
   if(ctx->d_wpdf) (void)hipFree(ctx->d_wpdf);
   if(ctx->d_cie_cdf) (void)hipFree(ctx->d_cie_cdf);
@@ -1112,45 +991,6 @@ DevMap htgx_cie_channel_map(const htgx_ctx* ctx, const DevMap& M, int c)
 /*******************************************************************************
  * Rendering
  ******************************************************************************/
-static int
-render_plain(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, hipStream_t stream)
-{
-  const uint64_t npix = (uint64_t)M.width * M.height;
-  const uint32_t ntx = (M.width + 7) / 8, nty = (M.height + 7) / 8;
-  const uint64_t items_per_slice = (uint64_t)ntx * nty * 64;
-  /* Enough threads to fill the 256 CUs several times over, each running as
-   * many consecutive realisations of its pixel as possible. */
-  const uint64_t target = 1ull << 21;
-  uint32_t nslices = (uint32_t)std::min<uint64_t>(M.spp,
-    std::max<uint64_t>(1, (target + items_per_slice - 1) / items_per_slice));
-  const uint32_t spt = (M.spp + nslices - 1) / nslices;
-  nslices = (M.spp + spt - 1) / spt;
-  if(items_per_slice * nslices > 0xFFFFFFFFull) return HTGX_BAD_ARG;
-
-  const size_t need = (size_t)nslices * npix * sizeof(htgx_mc_accum);
-  if(need > ctx->partials_cap) {
-    if(ctx->d_partials) { HIP_OK(hipFree(ctx->d_partials)); ctx->d_partials = nullptr; }
-    HIP_OK(hipMalloc(&ctx->d_partials, need));
-    ctx->partials_cap = need;
-  }
-  const uint64_t nthreads = items_per_slice * nslices;
-  const uint32_t nblocks = (uint32_t)((nthreads + 255) / 256);
-  if(ctx->counting) {
-    HIP_OK(hipMemsetAsync(ctx->d_counters, 0, HTGX_NSTATS * sizeof(unsigned long long), stream));
-    plain_kernel<true><<<nblocks, 256, 0, stream>>>(ctx->S, M, ntx, (uint32_t)items_per_slice,
-      nslices, spt, (htgx_mc_accum*)ctx->d_partials, ctx->d_counters);
-  } else {
-    plain_kernel<false><<<nblocks, 256, 0, stream>>>(ctx->S, M, ntx, (uint32_t)items_per_slice,
-      nslices, spt, (htgx_mc_accum*)ctx->d_partials, ctx->d_counters);
-  }
-  HIP_OK(hipGetLastError());
-  merge_kernel<<<(uint32_t)((npix + 255) / 256), 256, 0, stream>>>(
-    (const htgx_mc_accum*)ctx->d_partials, nslices, npix, accum);
-  HIP_OK(hipGetLastError());
-  ctx->last_nrealisations = npix * M.spp;
-  return HTGX_OK;
-}
-
 extern "C" int
 htgx_render_accum(htgx_ctx* ctx, const htgx_map_desc* desc, htgx_mc_accum* accum, void* stream)
 {
@@ -1168,7 +1008,7 @@ htgx_render_accum(htgx_ctx* ctx, const htgx_map_desc* desc, htgx_mc_accum* accum
     htgx_mc_accum* a = accum + (size_t)c * npix;
     res = desc->solver == HTGX_SOLVER_WAVEFRONT_FP32
       ? htgx_render_wavefront(ctx, Mc, a, (hipStream_t)stream)
-      : render_plain(ctx, Mc, a, (hipStream_t)stream);
+      : htgx_render_plain(ctx, Mc, a, (hipStream_t)stream);
     if(res != HTGX_OK) return res;
     nreal += ctx->last_nrealisations;
   }

@@ -31,9 +31,11 @@ struct htgx_ctx {
   bool cache_loaded = false;
   std::string cache_err;
   double us_per_tick = 0.01;
-  /* per-slice partial accumulators of the plain solver */
+  /* the plain solver's chunk partials, chunk counters and resident blocks */
   void* d_partials = nullptr;
   size_t partials_cap = 0;
+  unsigned int* d_plain_queue = nullptr;
+  uint32_t plain_grid = 0;
   /* wavelength CDF of the last map (cached by range and Tref) */
   double* d_wcdf = nullptr;
   double* d_wpdf = nullptr;
@@ -62,6 +64,7 @@ int htgx_map_setup(htgx_ctx* ctx, const htgx_map_desc* desc, htgx::DevMap* map,
 /* The map of channel c (0 X, 1 Y, 2 Z) of a CIE XYZ image set up by
  * htgx_map_setup: the channel's wavelength CDF and its own random streams */
 htgx::DevMap htgx_cie_channel_map(const htgx_ctx* ctx, const htgx::DevMap& M, int c);
+int htgx_render_plain(htgx_ctx* ctx, const htgx::DevMap& map, htgx_mc_accum* accum, hipStream_t stream);
 int htgx_render_wavefront(htgx_ctx* ctx, const htgx::DevMap& map, htgx_mc_accum* accum,
                           hipStream_t stream);
 /* Several maps of distinct contexts (same device, same sensor and spectral

@@ -35,6 +35,7 @@
 #pragma clang fp contract(on)
 
 #include "htgx_internal.h"
+#include "htgx_queue.h"
 
 #include <hip/hip_runtime.h>
 
@@ -63,7 +64,6 @@ using namespace htgx;
 namespace {
 
 constexpr float kPif = 3.14159265358979323846f;
-constexpr int kXcds = 8;
 
 /* FP32 copy of the scene constants (device arrays shared with the FP64
  * solver where the layout is the same) */
@@ -342,14 +342,6 @@ __device__ __forceinline__ EventDraws event_draws(const SceneF& S, const Lane& L
 __device__ __forceinline__ float exp1f(float u)
 {
   return -__logf(1.0f - u);
-}
-
-__device__ __forceinline__ void nsum(double& sum, double& c, double x)
-{
-  const double t = sum + x;
-  if(fabs(sum) >= fabs(x)) c += (sum - t) + x;
-  else c += (x - t) + sum;
-  sum = t;
 }
 
 /* Planck's law in W/m^2/sr/m (src/core/htrdr_spectral.h:102-116) in FP32 */
@@ -1241,60 +1233,6 @@ __device__ __forceinline__ void walk_done(const SceneF& S, Lane& L)
   }
 }
 
-/* Chunks for the lanes with `need', from this XCD's tile range, else from the
- * others: one atomic per wavefront and range, the lanes sharing what it
- * reserved in lane order. `tried' counts the ranges the wavefront has found
- * empty; it does not ask them again. Returns false for a lane that finds no
- * chunk left anywhere. The whole wavefront calls this together. */
-__device__ __forceinline__ bool fetch_chunks(const Launch& P, uint32_t xcd, uint32_t* tried, bool need,
-                                             uint32_t* chunk)
-{
-  const uint32_t per_tile = P.nsub * 64u;
-  bool got = false;
-  uint64_t mask = __ballot(need);
-  while(mask && *tried < (uint32_t)kXcds) {
-    const uint32_t x = (xcd + *tried) % (uint32_t)kXcds;
-    const uint32_t t0 = min(x * P.xcd_tiles, P.ntiles), t1 = min(t0 + P.xcd_tiles, P.ntiles);
-    const uint32_t n = (t1 - t0) * per_tile;
-    if(n) {
-      const int leader = __ffsll((unsigned long long)mask) - 1;
-      uint32_t c = 0;
-      if((int)(threadIdx.x & 63u) == leader) c = atomicAdd(P.counters + x, (uint32_t)__popcll(mask));
-      c = (uint32_t)__builtin_amdgcn_readlane((int)c, leader) +
-          (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                              __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-      if(need && !got && c < n) { *chunk = t0 * per_tile + c; got = true; }
-    }
-    mask = __ballot(need && !got);
-    if(mask) ++*tried;
-  }
-  return got;
-}
-
-__device__ __forceinline__ uint64_t wave_sum64(uint64_t v)
-{
-  for(int off = 32; off > 0; off >>= 1) v += (uint64_t)__shfl_xor((unsigned long long)v, off, 64);
-  return v;
-}
-
-/* A pointer to constant memory: the kernel argument segment, or a table in
- * device memory that no kernel writes while it is read */
-template<class T>
-using KPtr = const __attribute__((address_space(4))) T*;
-
-/* A copy of a constant-memory struct (scalar loads; the host compilation
- * pass, which only needs the declaration, gets an empty value) */
-template<class T>
-__device__ __forceinline__ T kload(KPtr<T> p)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-  return *p;
-#else
-  (void)p;
-  return T{};
-#endif
-}
-
 /* The arguments of the map each wavefront of the block works on (of a batch,
  * the wavefronts may be at different maps). The event step reads its scene,
  * map and launch constants from here: 60-odd of them, in scalar registers
@@ -1314,15 +1252,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
   const uint64_t seed = kload(&pK->M.seed);
   /* this wavefront's copy of the arguments, for the event step */
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  {
-    static_assert(sizeof(KArgs) % 4 == 0, "copied by dwords");
-    const KPtr<uint32_t> src = (KPtr<uint32_t>)pK;
-    uint32_t* dst = (uint32_t*)&g_args[wave];
-    for(uint32_t i = threadIdx.x & 63u; i < sizeof(KArgs) / 4; i += 64u) dst[i] = kload(src + i);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
+  copy_to_lds(pK, &g_args[wave]);
   /* canonicals per event: 8, plus 2 for the sun of a SW flux map */
   constexpr int NP = (SENSOR == HTGX_SENSOR_RECTANGLE && SPECTRAL == HTGX_SPECTRAL_SW) ? 5 : 4;
   Lane L;
@@ -1535,12 +1465,9 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
           if(P.exhausted) atomicExch(P.exhausted, 1u);
         } else if(fetch) {
           LC(chunk) = c;
-          const uint32_t m = c & 63u, rest = c >> 6;
-          const uint32_t s = rest % P.nsub, t = rest / P.nsub;
-          const uint32_t x = (t % P.ntx) * 8u + ((m & 1u) | ((m >> 1) & 2u) | ((m >> 2) & 4u));
-          const uint32_t y = (t / P.ntx) * 8u + (((m >> 1) & 1u) | ((m >> 2) & 2u) | ((m >> 3) & 4u));
-          if(x < P.width && y < P.height) {
-            L.pixel = y * P.width + x;
+          uint32_t pixel, s;
+          if(chunk_pixel(P, c, &pixel, &s)) {
+            L.pixel = pixel;
             L.r = (P.spp_offset_dev ? *P.spp_offset_dev : P.spp_offset) + s * P.K;
             LC(r_end) = L.r + P.K;
             LC(n) = LC(nfail) = 0;
@@ -1821,39 +1748,6 @@ batch_advance_kernel(BatchScene* scenes, uint32_t n, unsigned int* step)
   if(i == 0) *step += 1u;
 }
 
-/* Fold the chunks of pixel p, in chunk order, into its accumulator */
-__device__ __forceinline__ void
-merge_pixel(const htgx_mc_accum* partials, uint32_t width, uint32_t ntx, uint32_t nsub,
-            htgx_mc_accum* accum, uint32_t p)
-{
-  const uint32_t x = p % width, y = p / width;
-  const uint32_t t = (y / 8u) * ntx + (x / 8u);
-  const uint32_t ix = x & 7u, iy = y & 7u;
-  const uint32_t m = (ix & 1u) | ((iy & 1u) << 1) | ((ix & 2u) << 1) | ((iy & 2u) << 2)
-                   | ((ix & 4u) << 2) | ((iy & 4u) << 3);
-  htgx_mc_accum a = accum[p];
-  for(uint32_t s = 0; s < nsub; ++s) {
-    const htgx_mc_accum q = partials[((size_t)t * nsub + s) * 64u + m];
-    nsum(a.sum, a.sum_c, q.sum);
-    a.sum_c += q.sum_c;
-    nsum(a.sum2, a.sum2_c, q.sum2);
-    a.sum2_c += q.sum2_c;
-    a.tsum += q.tsum;
-    a.tsum2 += q.tsum2;
-    a.n += q.n;
-    a.nfail += q.nfail;
-  }
-  accum[p] = a;
-}
-
-__global__ void __launch_bounds__(256)
-wf_merge_kernel(const htgx_mc_accum* partials, uint32_t width, uint32_t height, uint32_t ntx,
-                uint32_t nsub, htgx_mc_accum* accum)
-{
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if(p < width * height) merge_pixel(partials, width, ntx, nsub, accum, p);
-}
-
 /* The merges of every map of a batch: blockIdx.y is the table slot */
 __global__ void __launch_bounds__(256)
 batch_merge_kernel(const BatchScene* scenes)
@@ -1862,20 +1756,6 @@ batch_merge_kernel(const BatchScene* scenes)
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   const Launch& P = B.A.P;
   if(p < P.width * P.height) merge_pixel(P.partials, P.width, P.ntx, P.nsub, B.accum, p);
-}
-
-__global__ void
-zero_u32_kernel(unsigned int* p, uint32_t n)
-{
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if(i < n) p[i] = 0u;
-}
-
-__global__ void
-zero_u64_kernel(unsigned long long* p, uint32_t n)
-{
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if(i < n) p[i] = 0ull;
 }
 
 /* FP16 bits of a bound of v >= 0 in units of scale >= v, rounded down (lower
@@ -2303,7 +2183,7 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, 
     if((res = launch<false>(st->S, M, P, grid, stream))) return res;
   }
   const uint32_t npix = M.width * M.height;
-  wf_merge_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(
+  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(
     (const htgx_mc_accum*)st->d_partials, M.width, M.height, P.ntx, P.nsub, accum);
   HIP_OK(hipGetLastError());
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
@@ -2353,7 +2233,7 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum*
     if((res = launch<false>(st->S, M, P, grid, stream))) return res;
   }
   const uint32_t npix = M.width * M.height;
-  wf_merge_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P.partials, M.width, M.height, P.ntx,
+  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P.partials, M.width, M.height, P.ntx,
                                                            P.nsub, accum);
   HIP_OK(hipGetLastError());
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
