@@ -981,7 +981,7 @@ DevMap htgx_cie_channel_map(const htgx_ctx* ctx, const DevMap& M, int c)
 {
   DevMap C = M;
   C.cie_channel = c;
-  C.cie_rcp = ctx->cie_rcp[c];
+  for(int k = 0; k < 3; ++k) C.cie_rcp[k] = ctx->cie_rcp[std::min(c + k, 2)];
   C.wcdf = ctx->d_cie_cdf + (size_t)c * ctx->cie_nbands;
   C.wpdf = nullptr;
   C.seed = M.seed ^ ((uint64_t)(c + 1) << 56);
@@ -991,6 +991,21 @@ DevMap htgx_cie_channel_map(const htgx_ctx* ctx, const DevMap& M, int c)
 /*******************************************************************************
  * Rendering
  ******************************************************************************/
+int
+htgx_render_channels(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_mc_accum* accum,
+                     hipStream_t stream, htgx_render_fn render)
+{
+  const size_t npix = (size_t)M.width * M.height;
+  uint64_t nreal = 0;
+  for(uint32_t c = 0; c < planes; ++c) {
+    const int res = render(ctx, htgx_cie_channel_map(ctx, M, (int)c), 1, accum + c * npix, stream);
+    if(res != HTGX_OK) return res;
+    nreal += ctx->last_nrealisations;
+  }
+  ctx->last_nrealisations = nreal;
+  return HTGX_OK;
+}
+
 extern "C" int
 htgx_render_accum(htgx_ctx* ctx, const htgx_map_desc* desc, htgx_mc_accum* accum, void* stream)
 {
@@ -999,21 +1014,12 @@ htgx_render_accum(htgx_ctx* ctx, const htgx_map_desc* desc, htgx_mc_accum* accum
   if(!ctx || !desc || !accum) return HTGX_BAD_ARG;
   if((res = htgx_map_setup(ctx, desc, &M)) != HTGX_OK) return res;
   /* a CIE XYZ image is 3 maps, one per channel, into 3 accumulator planes
-   * (draw_pixel_image, src/atmosphere/htrdr_atmosphere_draw_map.c:134-199) */
-  const int nch = desc->spectral_type == HTGX_SPECTRAL_SW_CIE_XYZ ? 3 : 1;
-  const size_t npix = (size_t)desc->width * desc->height;
-  uint64_t nreal = 0;
-  for(int c = 0; c < nch; ++c) {
-    const DevMap Mc = nch == 3 ? htgx_cie_channel_map(ctx, M, c) : M;
-    htgx_mc_accum* a = accum + (size_t)c * npix;
-    res = desc->solver == HTGX_SOLVER_WAVEFRONT_FP32
-      ? htgx_render_wavefront(ctx, Mc, a, (hipStream_t)stream)
-      : htgx_render_plain(ctx, Mc, a, (hipStream_t)stream);
-    if(res != HTGX_OK) return res;
-    nreal += ctx->last_nrealisations;
-  }
-  ctx->last_nrealisations = nreal;
-  return HTGX_OK;
+   * (draw_pixel_image, src/atmosphere/htrdr_atmosphere_draw_map.c:134-199),
+   * in one launch */
+  const uint32_t planes = desc->spectral_type == HTGX_SPECTRAL_SW_CIE_XYZ ? 3 : 1;
+  return desc->solver == HTGX_SOLVER_WAVEFRONT_FP32
+    ? htgx_render_wavefront(ctx, M, planes, accum, (hipStream_t)stream)
+    : htgx_render_plain(ctx, M, planes, accum, (hipStream_t)stream);
 }
 
 extern "C" int
@@ -1025,18 +1031,8 @@ htgx_render_accum_noalloc(htgx_ctx* ctx, const htgx_map_desc* desc, htgx_mc_accu
   if(!ctx || !desc || !accum) return HTGX_BAD_ARG;
   if(desc->solver != HTGX_SOLVER_WAVEFRONT_FP32) return HTGX_BAD_ARG;
   if((res = htgx_map_setup(ctx, desc, &M, false)) != HTGX_OK) return res;
-  const int nch = desc->spectral_type == HTGX_SPECTRAL_SW_CIE_XYZ ? 3 : 1;
-  const size_t npix = (size_t)desc->width * desc->height;
-  uint64_t nreal = 0;
-  for(int c = 0; c < nch; ++c) {
-    const DevMap Mc = nch == 3 ? htgx_cie_channel_map(ctx, M, c) : M;
-    if((res = htgx_render_wavefront_noalloc(ctx, Mc, accum + (size_t)c * npix,
-                                            (hipStream_t)stream)) != HTGX_OK)
-      return res;
-    nreal += ctx->last_nrealisations;
-  }
-  ctx->last_nrealisations = nreal;
-  return HTGX_OK;
+  const uint32_t planes = desc->spectral_type == HTGX_SPECTRAL_SW_CIE_XYZ ? 3 : 1;
+  return htgx_render_wavefront_noalloc(ctx, M, planes, accum, (hipStream_t)stream);
 }
 
 extern "C" int

@@ -130,8 +130,11 @@ struct DevMap {
   const double* wcdf;
   const double* wpdf;
   double Tref;
-  int cie_channel;  /* wmode 3: 0 X, 1 Y, 2 Z */
-  double cie_rcp;   /* wmode 3: 1 / integral of the channel's fit, nm^-1 */
+  /* wmode 3: the channel of the map's first plane (0 X, 1 Y, 2 Z), and per
+   * plane 1 / integral of its channel's fit, nm^-1; wcdf holds the planes'
+   * CDFs one after the other */
+  int cie_channel;
+  double cie_rcp[3];
   double us_per_tick; /* wall clock period in microseconds */
 };
 
@@ -285,18 +288,20 @@ HTGX_HD double cie_band_sample(int channel, double lmin, double len, double r1)
  * The pdf is in nm^-1; for a CIE channel it is the constant 1 / integral of
  * the channel, as the reference returns it. Without RARE, the modes that few
  * maps use (3, CIE channels, and 2, Planck over a continuous range) are
- * compiled out: the caller guarantees the mode is 0 or 1. */
+ * compiled out: the caller guarantees the mode is 0 or 1. plane: of a map of
+ * several channels, the one to sample. */
 template<bool RARE = true>
-HTGX_D double sample_wavelength(const DevMap& M, double r0, double r1, double* pdf)
+HTGX_D double sample_wavelength(const DevMap& M, double r0, double r1, double* pdf, uint32_t plane = 0)
 {
   if(RARE && M.wmode == 3) {
+    const double* cdf = M.wcdf + (size_t)plane * M.nwbands;
     uint32_t lo = 0, hi = M.nwbands - 1;
     while(lo < hi) {
       const uint32_t mid = (lo + hi) >> 1;
-      if(M.wcdf[mid] > r0) hi = mid; else lo = mid + 1;
+      if(cdf[mid] > r0) hi = mid; else lo = mid + 1;
     }
-    *pdf = M.cie_rcp;
-    return cie_band_sample(M.cie_channel, M.range[0] + (double)lo * M.band_len, M.band_len, r1);
+    *pdf = M.cie_rcp[plane];
+    return cie_band_sample(M.cie_channel + (int)plane, M.range[0] + (double)lo * M.band_len, M.band_len, r1);
   }
   if(M.wmode == 1) {
     uint32_t lo = 0, hi = M.nwbands - 1;

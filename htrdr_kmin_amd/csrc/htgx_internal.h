@@ -64,8 +64,11 @@ int htgx_map_setup(htgx_ctx* ctx, const htgx_map_desc* desc, htgx::DevMap* map,
 /* The map of channel c (0 X, 1 Y, 2 Z) of a CIE XYZ image set up by
  * htgx_map_setup: the channel's wavelength CDF and its own random streams */
 htgx::DevMap htgx_cie_channel_map(const htgx_ctx* ctx, const htgx::DevMap& M, int c);
-int htgx_render_plain(htgx_ctx* ctx, const htgx::DevMap& map, htgx_mc_accum* accum, hipStream_t stream);
-int htgx_render_wavefront(htgx_ctx* ctx, const htgx::DevMap& map, htgx_mc_accum* accum,
+/* A map on either solver; planes: accumulator planes, 3 for a CIE XYZ image
+ * (map its first channel's, with the image's seed), else 1 */
+int htgx_render_plain(htgx_ctx* ctx, const htgx::DevMap& map, uint32_t planes, htgx_mc_accum* accum,
+                      hipStream_t stream);
+int htgx_render_wavefront(htgx_ctx* ctx, const htgx::DevMap& map, uint32_t planes, htgx_mc_accum* accum,
                           hipStream_t stream);
 /* Several maps of distinct contexts (same device, same sensor and spectral
  * type) in one persistent FP32 launch; synchronous. scene_ms[i] (optional):
@@ -100,10 +103,17 @@ int htgx_debug_trace_segments_fp32_impl(htgx_ctx* ctx, const double* rays, uint3
  * [0] by the tentative-collision budget, [1] by the segment iterator's bound
  * on passes without a segment */
 int htgx_wavefront_truncations(htgx_ctx* ctx, uint64_t out[2]);
-/* htgx_render_accum_noalloc of one map (channel) on the FP32 solver: the
- * chunk counters and partials in the library's static scratch array */
-int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const htgx::DevMap& map, htgx_mc_accum* accum,
-                                  hipStream_t stream);
+/* The planes of a CIE XYZ image rendered one after the other, each as a map of
+ * its own, by one of the functions around; for images whose planes together
+ * need more than kMaxPlanePartials bytes of partial sums */
+constexpr uint64_t kMaxPlanePartials = 4ull << 30;
+typedef int (*htgx_render_fn)(htgx_ctx*, const htgx::DevMap&, uint32_t, htgx_mc_accum*, hipStream_t);
+int htgx_render_channels(htgx_ctx* ctx, const htgx::DevMap& map, uint32_t planes, htgx_mc_accum* accum,
+                         hipStream_t stream, htgx_render_fn render);
+/* htgx_render_accum_noalloc of one map on the FP32 solver: the chunk counters
+ * and partials in the library's static scratch array */
+int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const htgx::DevMap& map, uint32_t planes,
+                                  htgx_mc_accum* accum, hipStream_t stream);
 void htgx_wavefront_release(htgx_ctx* ctx);
 
 #endif /* HTGX_INTERNAL_H */

@@ -9,8 +9,12 @@
  * partial accumulator of its own and the merge folds them per pixel in chunk
  * order, so a map does not depend on the schedule.
  *
- * The queue is any struct with the fields width, height, ntx, K, nsub, ntiles,
- * xcd_tiles and counters.
+ * A map may have several planes (the channels of a CIE XYZ image) that follow
+ * each other in the queue: one launch, so that the longest walks of a plane,
+ * which end alone, overlap with the others.
+ *
+ * The queue is any struct with the fields width, height, ntx, K, nsub, planes,
+ * plane_tiles (tiles of a plane), ntiles (of all), xcd_tiles and counters.
  */
 #ifndef HTGX_QUEUE_H
 #define HTGX_QUEUE_H
@@ -56,13 +60,15 @@ __device__ __forceinline__ bool fetch_chunks(const Q& P, uint32_t xcd, uint32_t*
   return got;
 }
 
-/* Pixel and slice of a chunk; false if the pixel lies outside the image */
+/* Pixel, slice and plane of a chunk; false if the pixel lies outside the image */
 template<class Q>
-__device__ __forceinline__ bool chunk_pixel(const Q& P, uint32_t c, uint32_t* pixel, uint32_t* sub)
+__device__ __forceinline__ bool chunk_pixel(const Q& P, uint32_t c, uint32_t* pixel, uint32_t* sub,
+                                            uint32_t* plane)
 {
   const uint32_t m = c & 63u, rest = c >> 6;
-  const uint32_t t = rest / P.nsub;
+  const uint32_t tt = rest / P.nsub, t = tt % P.plane_tiles;
   *sub = rest % P.nsub;
+  *plane = tt / P.plane_tiles;
   const uint32_t x = (t % P.ntx) * 8u + ((m & 1u) | ((m >> 1) & 2u) | ((m >> 2) & 4u));
   const uint32_t y = (t / P.ntx) * 8u + (((m >> 1) & 1u) | ((m >> 2) & 2u) | ((m >> 3) & 4u));
   *pixel = y * P.width + x;
@@ -78,19 +84,21 @@ __device__ __forceinline__ void neumaier(double& sum, double& c, double x)
   sum = t;
 }
 
-/* Fold the chunks of pixel p, in chunk order, into its accumulator */
+/* Fold the chunks of pixel i (of all planes), in chunk order, into its
+ * accumulator */
+template<class Q>
 __device__ __forceinline__ void
-merge_pixel(const htgx_mc_accum* partials, uint32_t width, uint32_t ntx, uint32_t nsub,
-            htgx_mc_accum* accum, uint32_t p)
+merge_pixel(const Q& P, htgx_mc_accum* accum, uint32_t i)
 {
-  const uint32_t x = p % width, y = p / width;
-  const uint32_t t = (y / 8u) * ntx + (x / 8u);
+  const uint32_t npix = P.width * P.height, p = i % npix, nsub = P.nsub;
+  const uint32_t x = p % P.width, y = p / P.width;
+  const uint32_t t = (i / npix) * P.plane_tiles + (y / 8u) * P.ntx + (x / 8u);
   const uint32_t ix = x & 7u, iy = y & 7u;
   const uint32_t m = (ix & 1u) | ((iy & 1u) << 1) | ((ix & 2u) << 1) | ((iy & 2u) << 2)
                    | ((ix & 4u) << 2) | ((iy & 4u) << 3);
-  htgx_mc_accum a = accum[p];
+  htgx_mc_accum a = accum[i];
   for(uint32_t s = 0; s < nsub; ++s) {
-    const htgx_mc_accum q = partials[((size_t)t * nsub + s) * 64u + m];
+    const htgx_mc_accum q = P.partials[((size_t)t * nsub + s) * 64u + m];
     neumaier(a.sum, a.sum_c, q.sum);
     a.sum_c += q.sum_c;
     neumaier(a.sum2, a.sum2_c, q.sum2);
@@ -100,15 +108,28 @@ merge_pixel(const htgx_mc_accum* partials, uint32_t width, uint32_t ntx, uint32_
     a.n += q.n;
     a.nfail += q.nfail;
   }
-  accum[p] = a;
+  accum[i] = a;
 }
 
+template<class Q>
 __global__ void __launch_bounds__(256)
-merge_chunks_kernel(const htgx_mc_accum* partials, uint32_t width, uint32_t height, uint32_t ntx,
-                    uint32_t nsub, htgx_mc_accum* accum)
+merge_chunks_kernel(Q P, htgx_mc_accum* accum)
 {
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if(p < width * height) merge_pixel(partials, width, ntx, nsub, accum, p);
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if(i < P.width * P.height * P.planes) merge_pixel(P, accum, i);
+}
+
+/* The queue's sizes for a map of width x height pixels */
+template<class Q>
+inline void set_queue_size(Q& P, uint32_t width, uint32_t height, uint32_t planes)
+{
+  P.width = width;
+  P.height = height;
+  P.ntx = (width + 7) / 8;
+  P.planes = planes;
+  P.plane_tiles = P.ntx * ((height + 7) / 8);
+  P.ntiles = P.plane_tiles * planes;
+  P.xcd_tiles = (P.ntiles + kXcds - 1) / kXcds;
 }
 
 __global__ void

@@ -52,7 +52,8 @@ struct Launch {
   uint32_t width, height, ntx;
   uint32_t K;         /* realisations per chunk (the last of a pixel may be shorter) */
   uint32_t nsub;      /* chunks per pixel */
-  uint32_t ntiles, xcd_tiles;
+  uint32_t planes;    /* 3 for the channels of a CIE XYZ image, else 1 */
+  uint32_t plane_tiles, ntiles, xcd_tiles;
   uint32_t lanes;     /* lanes of each wavefront that take work */
   unsigned int* counters;   /* [kXcds] next chunk of each XCD range */
   htgx_mc_accum* partials;  /* [ntiles * nsub * 64] */
@@ -76,6 +77,7 @@ struct Lane {
   uint32_t draw;        /* next draw of its stream */
   uint64_t buf[4];      /* the Threefry block holding it, unless draw % 4 == 0 */
   uint32_t iband, kquad; /* band, k-point row */
+  uint32_t channel;     /* of an image of several channels: 1 + the lane's, else 0 */
   uint32_t surface : 1, rayleigh : 1, gh_hit : 1, specular : 1, prev_edge : 1, gh_edge : 1;
   uint32_t pending : 1, nq : 1, nq_ground : 1;
   uint32_t done : 1, adv : 1, adv_g : 1, adv_c : 1, s_cloud : 1;
@@ -108,7 +110,7 @@ struct LaneCold {
   double org[3][kBlock], dir0[3][kBlock], cosN[kBlock], Ld[kBlock]; /* shortwave flux */
   uint32_t stage[kBlock], mask[kBlock], phase[kBlock], t0[kBlock];
   int32_t prev_prim[kBlock], gh_prim[kBlock];
-  uint32_t n[kBlock], nfail[kBlock], chunk[kBlock], r_end[kBlock];
+  uint32_t n[kBlock], nfail[kBlock], chunk[kBlock], r_end[kBlock], plane[kBlock];
 };
 __shared__ LaneCold g_cold;
 /* The arguments, one copy per wavefront, for the event step */
@@ -123,7 +125,7 @@ __device__ __forceinline__ void stream_block(const Lane& L, uint64_t seed, uint3
                                              uint64_t out[4])
 {
   const uint64_t ctr[4] = {b, 0, 0, 0};
-  const uint64_t key[4] = {seed, L.pixel, (uint64_t)spp_offset + L.r, 0};
+  const uint64_t key[4] = {seed ^ ((uint64_t)L.channel << 56), L.pixel, (uint64_t)spp_offset + L.r, 0};
   threefry4x64_20(ctr, key, out);
 }
 
@@ -636,7 +638,7 @@ __device__ __forceinline__ void real_begin(const DevScene& S, const DevMap& M, L
   }
   const double r0 = u.next(), r1 = u.next(), r2 = u.next();
   double pdf;
-  const double wlen = sample_wavelength<GEN>(M, r0, r1, &pdf);
+  const double wlen = sample_wavelength<GEN>(M, r0, r1, &pdf, GEN ? LC(plane) : 0u);
   pdf *= 1e9;
   LC(pdf) = pdf;
   LC(wlen) = wlen;
@@ -720,7 +722,7 @@ plain_kernel(KArgs A)
   L.lstate = (threadIdx.x & 63u) < lanes ? LS_EVENT : LS_DONE;
   LC(stage) = ST_FETCH;
   L.pending = L.nq = false;
-  L.pixel = L.r = L.draw = 0;
+  L.pixel = L.r = L.draw = L.channel = 0;
   if(COUNT) L.n_leaf = L.n_seg = L.n_coll = L.n_cell = L.n_ev = 0;
   const uint32_t xcd = blockIdx.x % (uint32_t)kXcds;
   uint32_t tried = 0;
@@ -822,9 +824,13 @@ plain_kernel(KArgs A)
         if(fetch && !got) {
           L.lstate = LS_DONE;
         } else if(fetch) {
-          uint32_t pixel, sub;
-          if(chunk_pixel(P, c, &pixel, &sub)) {
+          uint32_t pixel, sub, plane;
+          if(chunk_pixel(P, c, &pixel, &sub, &plane)) {
             LC(chunk) = c;
+            if(GEN) {
+              LC(plane) = plane;
+              L.channel = P.planes > 1 ? plane + 1u : 0u;
+            }
             L.pixel = pixel;
             L.r = sub * P.K;
             LC(r_end) = min(L.r + P.K, M.spp);
@@ -943,7 +949,8 @@ int launch(const KArgs& A, uint32_t grid, hipStream_t stream)
 
 } /* namespace */
 
-int htgx_render_plain(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, hipStream_t stream)
+int htgx_render_plain(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_mc_accum* accum,
+                      hipStream_t stream)
 {
   int res;
   if(!ctx->plain_grid) {
@@ -958,12 +965,8 @@ int htgx_render_plain(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, hipS
   A.S = ctx->S;
   A.M = M;
   Launch& P = A.P;
-  const uint64_t npix = (uint64_t)M.width * M.height;
-  P.width = M.width;
-  P.height = M.height;
-  P.ntx = (M.width + 7) / 8;
-  P.ntiles = P.ntx * ((M.height + 7) / 8);
-  P.xcd_tiles = (P.ntiles + kXcds - 1) / kXcds;
+  const uint64_t npix = (uint64_t)M.width * M.height * planes;
+  set_queue_size(P, M.width, M.height, planes);
   /* chunks as large as leaves 4 to each resident lane: a lane runs its
    * chunk's realisations one after the other, and a chunk moves 128 B of
    * partial sums whatever its length */
@@ -971,6 +974,8 @@ int htgx_render_plain(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, hipS
   P.K = (uint32_t)std::min<uint64_t>(M.spp, std::max<uint64_t>(1, items * M.spp / (4 * lanes)));
   P.nsub = (M.spp + P.K - 1) / P.K;
   const uint64_t nchunks = items * P.nsub;
+  if(planes > 1 && nchunks * sizeof(htgx_mc_accum) > kMaxPlanePartials)
+    return htgx_render_channels(ctx, M, planes, accum, stream, htgx_render_plain);
   if(nchunks > 0xFFFFFFFFull) return HTGX_BAD_ARG;
   /* fewer chunks than lanes: spread over all the wavefronts */
   const uint64_t nw = kBlock / 64;
@@ -999,8 +1004,7 @@ int htgx_render_plain(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, hipS
     res = gen ? launch<true, false>(A, grid, stream) : launch<false, false>(A, grid, stream);
   }
   if(res != HTGX_OK) return res;
-  merge_chunks_kernel<<<(uint32_t)((npix + 255) / 256), 256, 0, stream>>>(
-    P.partials, M.width, M.height, P.ntx, P.nsub, accum);
+  merge_chunks_kernel<<<(uint32_t)((npix + 255) / 256), 256, 0, stream>>>(P, accum);
   HIP_OK(hipGetLastError());
   ctx->last_nrealisations = npix * M.spp;
   return HTGX_OK;

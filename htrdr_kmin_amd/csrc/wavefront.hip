@@ -127,7 +127,8 @@ struct Launch {
   uint32_t width, height, ntx;
   uint32_t K;            /* realisations per chunk */
   uint32_t nsub;         /* chunks per pixel in this launch */
-  uint32_t ntiles;
+  uint32_t planes;       /* 3 for the channels of a CIE XYZ image, else 1 */
+  uint32_t plane_tiles, ntiles; /* tiles of a plane, of all */
   uint32_t xcd_tiles;    /* tiles per XCD range */
   uint32_t spp_offset;
   uint32_t ev_thresh;    /* min #lanes needing the EVENT branch */
@@ -210,6 +211,7 @@ struct Lane {
   /* work */
   uint32_t pixel, r;    /* key of the realisation's random stream */
   uint32_t pair;        /* next Threefry-2x32 block of the realisation */
+  uint32_t key;         /* the map's seed, folded (of its plane's channel) */
   /* realisation */
   uint32_t gka_off, gks_off; /* rows of gas ka (band, k-point) and ks (band) */
   float cka, cks;       /* particle absorption / scattering per LWC of the band */
@@ -277,7 +279,7 @@ struct LaneCold {
   int32_t prev_prim[kBlock], gh_prim[kBlock]; /* previous surface hit (-1: none), current hit */
   uint32_t gh_mtl[kBlock];
   float tsum[kBlock], tsum2[kBlock];
-  uint32_t n[kBlock], nfail[kBlock], chunk[kBlock], r_end[kBlock];
+  uint32_t n[kBlock], nfail[kBlock], chunk[kBlock], r_end[kBlock], plane[kBlock];
   float shift[2][kBlock]; /* -r: world X/Y of the origin of the lane's frame */
   uint32_t ntiles[kBlock]; /* -r: copies of the grid the query has crossed */
 };
@@ -299,18 +301,18 @@ constexpr uint32_t kMaxEmptyPasses = 2000;
  * with counter (pair index, seed) under the key (pixel, realisation). The
  * numbers of a realisation depend only on its key and on how many pairs it
  * drew before, not on the lanes it shares a wavefront with. */
-__device__ __forceinline__ float2 draw_at(const Lane& L, uint32_t pair, uint32_t key)
+__device__ __forceinline__ float2 draw_at(const Lane& L, uint32_t pair)
 {
-  const uint32_t ctr[2] = {pair, key};
+  const uint32_t ctr[2] = {pair, L.key};
   const uint32_t k[2] = {L.pixel, L.r};
   uint32_t out[2];
   threefry2x32_20(ctr, k, out);
   return make_float2((float)(out[0] >> 8) * 0x1.0p-24f, (float)(out[1] >> 8) * 0x1.0p-24f);
 }
 
-__device__ __forceinline__ float2 draw2(Lane& L, uint32_t key)
+__device__ __forceinline__ float2 draw2(Lane& L)
 {
-  return draw_at(L, L.pair++, key);
+  return draw_at(L, L.pair++);
 }
 
 /* Which blocks of its event's draws a lane has a use for: 0 and 1 (u[0..3],
@@ -513,13 +515,13 @@ using GlobalU64 = const __attribute__((address_space(1))) uint64_t*;
 struct TrackRegs {
   float lower[3], inv_cs[3];
   float B;               /* cells per block, exact */
-  uint32_t def0, def1, key, max_steps;
+  uint32_t def0, def1, max_steps;
   GlobalF lwc;
   GlobalU64 leafrec;    /* the leaf records and their LWC scale */
   float lwc_scale;
 };
 
-__device__ __forceinline__ TrackRegs track_regs(const SceneF& S, uint32_t key, uint32_t max_steps)
+__device__ __forceinline__ TrackRegs track_regs(const SceneF& S, uint32_t max_steps)
 {
   TrackRegs g;
 #pragma unroll
@@ -530,7 +532,6 @@ __device__ __forceinline__ TrackRegs track_regs(const SceneF& S, uint32_t key, u
   g.def0 = S.def[0];
   g.def1 = S.def[1];
   g.B = (float)S.B;
-  g.key = key;
   g.max_steps = max_steps;
   g.lwc = (GlobalF)S.lwc;
   g.leafrec = (GlobalU64)S.leafrec;
@@ -1167,7 +1168,7 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
   }
 
   double pdf;
-  const double wlen = sample_wavelength<RARE>(M, (double)u[4], (double)u[5], &pdf);
+  const double wlen = sample_wavelength<RARE>(M, (double)u[4], (double)u[5], &pdf, RARE ? LC(plane) : 0u);
   LC(pdf) = (float)(pdf * 1e9);
   LC(wlen) = (float)wlen;
   uint32_t band;
@@ -1268,9 +1269,10 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
   L.pixel = L.r = 0;
   const uint32_t xcd = blockIdx.x % (uint32_t)kXcds;
   uint32_t tried = 0; /* chunk ranges found empty */
-  const TrackRegs G =
-      track_regs(S, (uint32_t)seed ^ (uint32_t)(seed >> 32), P.max_steps);
-  const uint32_t key = G.key;
+  const TrackRegs G = track_regs(S, P.max_steps);
+  /* only an image of several channels changes the key from lane to lane */
+  const uint32_t key = (uint32_t)seed ^ (uint32_t)(seed >> 32);
+  L.key = key;
   uint64_t d_it = 0, d_ce = 0, d_cl = 0, d_se = 0, d_sl = 0, d_ee = 0, d_el = 0;
   /* shader clock cycles per phase (counting build only) */
   uint64_t cy[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -1373,7 +1375,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
         const float v = L.s_cloud ? seg_lwcf<COUNT, FEAT>(G, L, x) : 0.f;
         /* the draw does not depend on the LWC: written before the LWC's
          * first use, its Threefry rounds run while the load is in flight */
-        const float2 uu = draw2(L, key);
+        const float2 uu = draw2(L);
         const float gka = L.s_gka, gks = L.s_gks;
         const float ka = gka + L.cka * v;
         const float ks = gks + L.cks * v;
@@ -1451,6 +1453,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
             L.pixel = P.list[2 * c];
             L.r = P.list[2 * c + 1];
             LC(r_end) = L.r + 1u;
+            LC(plane) = 0;
             LC(n) = LC(nfail) = 0;
             LC(sum) = LC(sum2) = 0.0;
             LC(tsum) = LC(tsum2) = 0.f;
@@ -1465,9 +1468,14 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
           if(P.exhausted) atomicExch(P.exhausted, 1u);
         } else if(fetch) {
           LC(chunk) = c;
-          uint32_t pixel, s;
-          if(chunk_pixel(P, c, &pixel, &s)) {
+          uint32_t pixel, s, plane;
+          if(chunk_pixel(P, c, &pixel, &s, &plane)) {
             L.pixel = pixel;
+            if(FEAT & kFeatRare) {
+              /* the channel's seed is the map's ^ (channel + 1) << 56 */
+              LC(plane) = plane;
+              L.key = P.planes > 1 ? key ^ ((plane + 1u) << 24) : key;
+            }
             L.r = (P.spp_offset_dev ? *P.spp_offset_dev : P.spp_offset) + s * P.K;
             LC(r_end) = L.r + P.K;
             LC(n) = LC(nfail) = 0;
@@ -1497,22 +1505,22 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
          * 0 or, for a lane with no use for that, the block after the event's
          * own, which gives a shortwave scattering query its second optical
          * thickness. Blocks 1 and 2 follow for the lanes that use them. */
-        const float2 vl = draw_at(L, L.pair + (uint32_t)(NP - 1), key);
-        const float2 v0 = draw_at(L, L.pair + (need.d0 ? 0u : (uint32_t)NP), key);
+        const float2 vl = draw_at(L, L.pair + (uint32_t)(NP - 1));
+        const float2 v0 = draw_at(L, L.pair + (need.d0 ? 0u : (uint32_t)NP));
         u[2 * NP - 2] = vl.x;
         u[2 * NP - 1] = vl.y;
         u[0] = v0.x;
         u[1] = v0.y;
         const bool have_a = !need.d0;
         if(need.d1 || need.d2) {
-          const float2 v1 = draw_at(L, L.pair + 1u, key), v2 = draw_at(L, L.pair + 2u, key);
+          const float2 v1 = draw_at(L, L.pair + 1u), v2 = draw_at(L, L.pair + 2u);
           u[2] = v1.x;
           u[3] = v1.y;
           u[4] = v2.x;
           u[5] = v2.y;
         }
         if(NP > 4 && begin) {
-          const float2 v3 = draw_at(L, L.pair + 3u, key);
+          const float2 v3 = draw_at(L, L.pair + 3u);
           u[6] = v3.x;
           u[7] = v3.y;
         }
@@ -1591,7 +1599,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
             L.pending = false;
             if(!kLW && L.mode == MODE_SC) {
               float ua = v0.x;
-              if(!have_a) ua = draw_at(L, L.pair, key).x;
+              if(!have_a) ua = draw_at(L, L.pair).x;
               L.pair++;
               L.Ts_a = exp1f(ua);
             }
@@ -1677,7 +1685,7 @@ wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop,
   iter_init<kFeatRare>(S, L);
   uint32_t n = 0;
   float t0;
-  const TrackRegs G = track_regs(S, 0u, 0u);
+  const TrackRegs G = track_regs(S, 0u);
   for(;;) {
     const int it = iter_next<false, kFeatRare>(S, G, L, prop, &t0);
     if(it == ITER_END) break;
@@ -1755,7 +1763,7 @@ batch_merge_kernel(const BatchScene* scenes)
   const BatchScene& B = scenes[blockIdx.y];
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   const Launch& P = B.A.P;
-  if(p < P.width * P.height) merge_pixel(P.partials, P.width, P.ntx, P.nsub, B.accum, p);
+  if(p < P.width * P.height) merge_pixel(P, B.accum, p);
 }
 
 /* FP16 bits of a bound of v >= 0 in units of scale >= v, rounded down (lower
@@ -2088,14 +2096,11 @@ constexpr uint32_t kChunksPerLane = 4;
 
 /* Launch parameters of one map, its partials and counters aside */
 static int
-fill_launch(htgx_ctx* ctx, const DevMap& M, Launch* P)
+fill_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
 {
   htgx_wavefront_state* st = ctx->wf;
   std::memset(P, 0, sizeof(*P));
-  P->width = M.width;
-  P->height = M.height;
-  P->ntx = (M.width + 7) / 8;
-  P->ntiles = P->ntx * ((M.height + 7) / 8);
+  set_queue_size(*P, M.width, M.height, planes);
   /* chunk size: the largest divisor of spp not above K that leaves at least
    * kChunksPerLane chunks per resident lane. A chunk's realisations run one
    * after the other, so on a small map whole chunks would leave lanes idle
@@ -2109,7 +2114,6 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, Launch* P)
   while(M.spp % K) --K;
   P->K = K;
   P->nsub = M.spp / K;
-  P->xcd_tiles = (P->ntiles + kXcds - 1) / kXcds;
   P->spp_offset = M.spp_offset;
   P->ev_thresh = st->ev_thresh;
   P->seg_thresh = st->seg_thresh;
@@ -2117,7 +2121,7 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, Launch* P)
   P->lanes = 64;
   const uint64_t nchunks = (uint64_t)P->ntiles * P->nsub * 64u;
   if(nchunks > 0xFFFFFFFFull) return HTGX_BAD_ARG;
-  P->nvalid = (uint32_t)((uint64_t)M.width * M.height * P->nsub);
+  P->nvalid = (uint32_t)((uint64_t)M.width * M.height * planes * P->nsub);
   P->stats = ctx->d_counters;
   P->trunc = st->d_trunc;
   return HTGX_OK;
@@ -2138,11 +2142,11 @@ spread_launch(uint32_t grid, Launch* P)
 
 /* Launch parameters of one map; sizes the chunk partials of the context */
 static int
-setup_launch(htgx_ctx* ctx, const DevMap& M, Launch* P)
+setup_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
 {
   htgx_wavefront_state* st = ctx->wf;
   int res;
-  if((res = fill_launch(ctx, M, P)) != HTGX_OK) return res;
+  if((res = fill_launch(ctx, M, planes, P)) != HTGX_OK) return res;
   const size_t need = (size_t)P->ntiles * P->nsub * 64u * sizeof(htgx_mc_accum);
   if(need > st->partials_cap) {
     if(st->d_partials) { HIP_OK(hipFree(st->d_partials)); st->d_partials = nullptr; }
@@ -2165,13 +2169,21 @@ int htgx_wavefront_truncations(htgx_ctx* ctx, uint64_t out[2])
   return HTGX_OK;
 }
 
-int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, hipStream_t stream)
+int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_mc_accum* accum,
+                          hipStream_t stream)
 {
   int res;
   if((res = wavefront_prepare(ctx)) != HTGX_OK) return res;
   htgx_wavefront_state* st = ctx->wf;
   Launch P;
-  if((res = setup_launch(ctx, M, &P)) != HTGX_OK) return res;
+  if(planes > 1) {
+    /* a large image's channels one after the other, as they need a third of
+     * the partial sums then and have no use for a common tail */
+    res = fill_launch(ctx, M, planes, &P);
+    if(res != HTGX_OK || (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum) > kMaxPlanePartials)
+      return htgx_render_channels(ctx, M, planes, accum, stream, htgx_render_wavefront);
+  }
+  if((res = setup_launch(ctx, M, planes, &P)) != HTGX_OK) return res;
   const uint32_t grid = spread_launch(st->grid, &P);
   zero_u32_kernel<<<1, 64, 0, stream>>>(st->d_counters, kXcds);
   HIP_OK(hipGetLastError());
@@ -2182,15 +2194,14 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum, 
   } else {
     if((res = launch<false>(st->S, M, P, grid, stream))) return res;
   }
-  const uint32_t npix = M.width * M.height;
-  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(
-    (const htgx_mc_accum*)st->d_partials, M.width, M.height, P.ntx, P.nsub, accum);
+  const uint32_t npix = M.width * M.height * planes;
+  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P, accum);
   HIP_OK(hipGetLastError());
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
   return HTGX_OK;
 }
 
-int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum* accum,
+int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_mc_accum* accum,
                                   hipStream_t stream)
 {
   htgx_wavefront_state* st = ctx->wf;
@@ -2201,7 +2212,7 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum*
   unsigned char* base = (unsigned char*)scratch_of(dev);
   if(!base) return HTGX_BAD_OP;
   Launch P;
-  if((res = fill_launch(ctx, M, &P)) != HTGX_OK) return res;
+  if((res = fill_launch(ctx, M, planes, &P)) != HTGX_OK) return res;
   uint64_t need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
   if(need > kScratchBytes - kScratchHead && P.K < st->K) {
     /* small chunks were preferred: the full ones need less scratch */
@@ -2209,8 +2220,12 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum*
     while(M.spp % K) --K;
     P.K = K;
     P.nsub = M.spp / K;
-    P.nvalid = (uint32_t)((uint64_t)M.width * M.height * P.nsub);
+    P.nvalid = (uint32_t)((uint64_t)M.width * M.height * planes * P.nsub);
     need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
+  }
+  if(need > kScratchBytes - kScratchHead && planes > 1) {
+    /* the channels one after the other, each in the whole scratch */
+    return htgx_render_channels(ctx, M, planes, accum, stream, htgx_render_wavefront_noalloc);
   }
   if(need > kScratchBytes - kScratchHead) {
     fprintf(stderr, "htgx: htgx_render_accum_noalloc: %llu chunk partials of %zu B exceed the "
@@ -2232,9 +2247,8 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, htgx_mc_accum*
   } else {
     if((res = launch<false>(st->S, M, P, grid, stream))) return res;
   }
-  const uint32_t npix = M.width * M.height;
-  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P.partials, M.width, M.height, P.ntx,
-                                                           P.nsub, accum);
+  const uint32_t npix = M.width * M.height * planes;
+  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P, accum);
   HIP_OK(hipGetLastError());
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
   return HTGX_OK;
@@ -2390,7 +2404,7 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
     e.A.S = ctxs[i]->wf->S;
     e.A.M = Ms[i];
     e.accum = accums[i];
-    if((res = setup_launch(ctxs[i], Ms[i], &e.A.P)) != HTGX_OK) return res;
+    if((res = setup_launch(ctxs[i], Ms[i], 1, &e.A.P)) != HTGX_OK) return res;
     e.A.P.stats = nullptr;
     e.A.P.counters = p->queues + (size_t)k * kXcds;
     e.A.P.exhausted = p->flags + k;
@@ -2616,7 +2630,7 @@ int htgx_wavefront_autotune(htgx_ctx* ctx, const DevMap& M, double budget_ms,
   uint32_t n = 0;
   res = tune_search([&](const htgx_wf_params& p, double* t) {
     set_params(st, p);
-    return clk.time([&] { return htgx_render_wavefront(ctx, M, acc.p, clk.stream); }, t);
+    return clk.time([&] { return htgx_render_wavefront(ctx, M, 1, acc.p, clk.stream); }, t);
   }, budget_ms, st->grid_max, &cur, &ms, &n);
   ctx->counting = counting;
   set_params(st, cur); /* kept for the maps that follow */
