@@ -286,14 +286,14 @@ HTGX_HD double cie_band_sample(int channel, double lmin, double len, double r1)
 /* htrdr_ran_wlen_planck_sample, src/core/htrdr_ran_wlen_planck.c:359-376,
  * and htrdr_ran_wlen_cie_xyz_sample_X/Y/Z, htrdr_ran_wlen_cie_xyz.c:346-397.
  * The pdf is in nm^-1; for a CIE channel it is the constant 1 / integral of
- * the channel, as the reference returns it. Without RARE, the modes that few
- * maps use (3, CIE channels, and 2, Planck over a continuous range) are
- * compiled out: the caller guarantees the mode is 0 or 1. plane: of a map of
- * several channels, the one to sample. */
-template<bool RARE = true>
+ * the channel, as the reference returns it. CIE and CONT compile in the modes
+ * that not every kernel needs (3, CIE channels, and 2, Planck over a
+ * continuous range): without them the caller guarantees another mode. plane:
+ * of a map of several channels, the one to sample. */
+template<bool CIE = true, bool CONT = true>
 HTGX_D double sample_wavelength(const DevMap& M, double r0, double r1, double* pdf, uint32_t plane = 0)
 {
-  if(RARE && M.wmode == 3) {
+  if(CIE && M.wmode == 3) {
     const double* cdf = M.wcdf + (size_t)plane * M.nwbands;
     uint32_t lo = 0, hi = M.nwbands - 1;
     while(lo < hi) {
@@ -311,7 +311,7 @@ HTGX_D double sample_wavelength(const DevMap& M, double r0, double r1, double* p
     }
     *pdf = M.wpdf[lo] * (1.0 / M.band_len);
     return M.range[0] + (double)lo * M.band_len + M.band_len * r1;
-  } else if(!RARE || M.wmode == 0) {
+  } else if(!CONT || M.wmode == 0) {
     *pdf = 1.0;
     return M.range[0];
   } else {

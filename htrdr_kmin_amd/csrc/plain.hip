@@ -638,7 +638,7 @@ __device__ __forceinline__ void real_begin(const DevScene& S, const DevMap& M, L
   }
   const double r0 = u.next(), r1 = u.next(), r2 = u.next();
   double pdf;
-  const double wlen = sample_wavelength<GEN>(M, r0, r1, &pdf, GEN ? LC(plane) : 0u);
+  const double wlen = sample_wavelength<GEN, GEN>(M, r0, r1, &pdf, GEN ? LC(plane) : 0u);
   pdf *= 1e9;
   LC(pdf) = pdf;
   LC(wlen) = wlen;

@@ -172,8 +172,12 @@ struct KArgs {
  * over a continuous range) are compiled out; without kFeatMesh, the mesh
  * ground (its BVH casts, its deferred casts). Their tests below are constants
  * then, so that their code and registers do not weigh on the kernels of the
- * maps that do without them. */
-enum { kFeatRare = 1, kFeatMesh = 2 };
+ * maps that do without them. A map whose one rare feature is its CIE XYZ
+ * wavelengths, the command line's default image, has a kernel of its own
+ * (kFeatCie): with the rare features' 45 KB of code and 88 bytes of spills a
+ * lane it took 117 ms instead of 88 (256x256 pixels x 16 realisations). */
+enum { kFeatRare = 1, kFeatMesh = 2, kFeatCie = 4 };
+constexpr bool has_cie(int feat) { return (feat & (kFeatRare | kFeatCie)) != 0; }
 
 template<int FEAT>
 __device__ __forceinline__ bool is_mesh(const SceneF& S)
@@ -1168,7 +1172,8 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
   }
 
   double pdf;
-  const double wlen = sample_wavelength<RARE>(M, (double)u[4], (double)u[5], &pdf, RARE ? LC(plane) : 0u);
+  const double wlen = sample_wavelength<has_cie(FEAT), RARE>(M, (double)u[4], (double)u[5], &pdf,
+                                                              has_cie(FEAT) ? LC(plane) : 0u);
   LC(pdf) = (float)(pdf * 1e9);
   LC(wlen) = (float)wlen;
   uint32_t band;
@@ -1471,7 +1476,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
           uint32_t pixel, s, plane;
           if(chunk_pixel(P, c, &pixel, &s, &plane)) {
             L.pixel = pixel;
-            if(FEAT & kFeatRare) {
+            if(has_cie(FEAT)) {
               /* the channel's seed is the map's ^ (channel + 1) << 56 */
               LC(plane) = plane;
               L.key = P.planes > 1 ? key ^ ((plane + 1u) << 24) : key;
@@ -1802,14 +1807,16 @@ int launch_variant(F kernel, const SceneF& S, const DevMap& M, const Launch& P, 
   return HTGX_OK;
 }
 
-/* The kernel features a map needs (kFeatRare, kFeatMesh) */
+/* The kernel features a map needs */
 int features(const SceneF& S, const DevMap& M)
 {
   /* (also grids too large for the 24-bit index arithmetic, grid_index) */
   const bool rare = S.repeat || S.ground_repeat || S.gmat || M.ortho || M.lens_radius > 0 ||
-                    M.wmode == 3 || M.wmode == 2 ||
+                    M.wmode == 2 ||
                     (uint64_t)S.def[1] * S.def[2] >= (1u << 24) || S.def[0] >= (1u << 24);
-  return (rare ? kFeatRare : 0) | (S.ground_type == HTGX_GROUND_MESH ? kFeatMesh : 0);
+  const bool mesh = S.ground_type == HTGX_GROUND_MESH;
+  if(M.wmode == 3) return rare || mesh ? kFeatRare | (mesh ? kFeatMesh : 0) : kFeatCie;
+  return (rare ? kFeatRare : 0) | (mesh ? kFeatMesh : 0);
 }
 
 template<bool COUNT, int FEAT>
@@ -1828,7 +1835,11 @@ int launch_full(const SceneF& S, const DevMap& M, const Launch& P, uint32_t grid
 template<bool COUNT>
 int launch(const SceneF& S, const DevMap& M, const Launch& P, uint32_t grid, hipStream_t stream)
 {
-  switch(features(S, M)) {
+  const int feat = features(S, M);
+  if(feat == kFeatCie) /* camera images only */
+    return launch_variant(wavefront_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_SW, COUNT, kFeatCie>, S, M, P,
+                          grid, stream);
+  switch(feat) {
     case 0: return launch_full<COUNT, 0>(S, M, P, grid, stream);
     case kFeatRare: return launch_full<COUNT, kFeatRare>(S, M, P, grid, stream);
     case kFeatMesh: return launch_full<COUNT, kFeatMesh>(S, M, P, grid, stream);
