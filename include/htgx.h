@@ -413,15 +413,20 @@ int htgx_render_accum_noalloc
  * hence the last bits of the accumulators. */
 struct htgx_wf_params {
   uint32_t ev_thresh; /* lanes of a 64-lane wavefront that must wait for the
-                         event step before it runs (1-64; 0 = default 24) */
-  uint32_t chunk;     /* realisations per work-queue chunk (1-16; 0 = default 4) */
+                         event step before it runs (1-64; 0 = default 24), fewer
+                         in proportion when lanes are out of work; with
+                         seg_thresh 0 also no fewer than wait for either other
+                         step */
+  uint32_t chunk;     /* realisations per work-queue chunk at most (1-16; 0 =
+                         default 4; small maps take smaller ones) */
   uint32_t grid;      /* blocks of 256 lanes of the persistent launch
                          (1-grid_max; 0 = grid_max) */
   uint32_t grid_max;  /* read only: blocks resident on the device at once */
   uint32_t seg_thresh; /* lanes of a 64-lane wavefront that must wait for the
                           segment step before it runs while other lanes can
-                          take a collision step (0-64; 0 = run it whenever a
-                          lane needs it) */
+                          take a collision step (1-64, 1: run it whenever a
+                          lane needs it; 0 = default: no fewer than wait for
+                          the collision step) */
 };
 
 int htgx_get_wavefront_params(struct htgx_ctx* ctx, struct htgx_wf_params* params);
