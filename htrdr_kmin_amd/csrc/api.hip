@@ -264,7 +264,8 @@ check_scene(const htgx_scene_desc* s)
       if(!(c.ssa[b] >= 0 && c.ssa[b] <= 1) || !(c.hg_g[b] > -1 && c.hg_g[b] < 1)) return HTGX_BAD_ARG;
     const size_t ncells = (size_t)c.def[0] * c.def[1] * c.def[2];
     bool ok = true;
-    for(size_t i = 0; i < ncells; ++i) ok &= c.lwc[i] >= 0.f && c.lwc[i] <= FLT_MAX;
+    #pragma omp parallel for schedule(static) reduction(&& : ok) if(ncells >= 1u << 20)
+    for(int64_t i = 0; i < (int64_t)ncells; ++i) ok = ok && (c.lwc[i] >= 0.f && c.lwc[i] <= FLT_MAX);
     if(!ok) return HTGX_BAD_ARG;
   }
   if(s->ground.type == HTGX_GROUND_PLANE || s->ground.type == HTGX_GROUND_MESH) {
@@ -276,10 +277,14 @@ check_scene(const htgx_scene_desc* s)
       if(g.plane_mtl >= nsurf) return HTGX_BAD_ARG;
     } else {
       if(!g.nverts || !g.ntris || !g.verts || !g.tris || !g.tri_mtl) return HTGX_BAD_ARG;
-      for(uint32_t t = 0; t < g.ntris; ++t) {
-        if(g.tri_mtl[t] >= nsurf) return HTGX_BAD_ARG;
-        for(int k = 0; k < 3; ++k) if(g.tris[3 * (size_t)t + k] >= g.nverts) return HTGX_BAD_ARG;
+      bool ok = true;
+      #pragma omp parallel for schedule(static) reduction(&& : ok) if(g.ntris >= 1u << 16)
+      for(int64_t t = 0; t < (int64_t)g.ntris; ++t) {
+        bool v = g.tri_mtl[t] < nsurf;
+        for(int k = 0; k < 3; ++k) v = v && g.tris[3 * (size_t)t + k] < g.nverts;
+        ok = ok && v;
       }
+      if(!ok) return HTGX_BAD_ARG;
     }
   } else if(s->ground.type != HTGX_GROUND_NONE) {
     return HTGX_BAD_ARG;
