@@ -129,20 +129,18 @@ __device__ __forceinline__ void stream_block(const Lane& L, uint64_t seed, uint3
   threefry4x64_20(ctr, key, out);
 }
 
-/* The draws of one event, in stream order */
+/* The draws of one event, in stream order, and how many it takes before the
+ * optical thickness of its next query, which is the draw `ts'. Every index is a
+ * constant where it is used: an index that varies over the lanes would put the
+ * array in scratch memory, a load of several hundred cycles each. */
 constexpr int kMaxDraws = 10;
 struct Draws {
   uint64_t w[kMaxDraws];
-  int n = 0; /* taken so far */
+  uint64_t ts;
+  uint32_t n;
 
-  __device__ __forceinline__ double next()
-  {
-    uint64_t v = w[kMaxDraws - 1];
-#pragma unroll
-    for(int i = kMaxDraws - 2; i >= 0; --i) v = n == i ? w[i] : v;
-    ++n;
-    return canonical(v);
-  }
+  __device__ __forceinline__ double at(int i) const { return canonical(w[i]); }
+  __device__ __forceinline__ void end(int i) { ts = w[i]; n = (uint32_t)i; }
 };
 
 /* Kernels without GEN: a plane ground or none, grey materials, no repetition,
@@ -413,16 +411,18 @@ __device__ __forceinline__ void sw_begin(const DevScene& S, Lane& L, int mask, c
   else LC(stage) = ST_WALK_DONE;
 }
 
-/* Next-event estimate and Russian roulette closing a SW event, ..._sw.c:494-504;
- * the lane's origin is the event */
-__device__ __forceinline__ void sw_accumulate(const DevScene& S, Lane& L, Draws& u, double Tr)
+/* Next-event estimate and Russian roulette (the draw `rr' of a surface event)
+ * closing a SW event, ..._sw.c:494-504; the lane's origin is the event. False
+ * if the walk ends. */
+__device__ __forceinline__ bool sw_accumulate(const DevScene& S, Lane& L, double rr, double Tr)
 {
   const double sun_pdf = L.specular ? 1.0 : 1.0 / S.sun_solid_angle;
   LC(w) += LC(ksi) * LC(L_sun) * Tr * LC(R) / sun_pdf;
-  if(L.surface && u.next() >= LC(refl)) { LC(stage) = ST_WALK_DONE; return; }
+  if(L.surface && rr >= LC(refl)) { LC(stage) = ST_WALK_DONE; return false; }
 #pragma unroll
   for(int a = 0; a < 3; ++a) L.d[a] = LCA(dir_next, a);
   request_scatter(L);
+  return true;
 }
 
 /* Draws the event of a lane takes at most, the optical thickness of the next
@@ -445,6 +445,7 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
   const int stage = (int)LC(stage);
   if(kLW) {
     if(stage != ST_LW) return;
+    u.n = 0;
     if(!L.gh_hit && L.ev == EV_NONE) { LC(w) = 0; LC(stage) = ST_WALK_DONE; return; }
     if(COUNT) L.n_ev++;
     if(L.ev == EV_ABS) {
@@ -457,8 +458,8 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
 #pragma unroll
     for(int a = 0; a < 3; ++a) pn[a] = (GEN && a < 2 ? L.ow[a] : L.o[a]) + L.d[a] * dst;
     if(L.ev == EV_SCA) {
-      const double u0 = u.next(), u1 = u.next();
-      local_to_world(L.d, hg_cos_sample(LC(g), u0), 2.0 * kPi * u1, dn);
+      local_to_world(L.d, hg_cos_sample(LC(g), u.at(0)), 2.0 * kPi * u.at(1), dn);
+      u.end(2);
       LC(prev_prim) = -1; /* ..._lw.c:236 */
       L.prev_edge = false;
     } else {
@@ -467,7 +468,7 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
       const uint32_t mtl = ground_surface<GEN>(S, LC(gh_prim), N);
       if(GEN && S.gmat) { /* ..._lw.c:249-252 */
         const int32_t m = interface_mtl(S.ifcs[mtl], S.mtls, dot3(N, L.d) > 0);
-        const DevBrdf& b = brdf_fetch(S.mtls[m], S.brdfs, LC(wlen), u.next());
+        const DevBrdf& b = brdf_fetch(S.mtls[m], S.brdfs, LC(wlen), u.at(0));
         refl = b.refl;
         specular = b.type == HTGX_BRDF_SPECULAR;
         T = S.mtls[m].T;
@@ -478,13 +479,15 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
       if(-(L.d[0]*N[0] + L.d[1]*N[1] + L.d[2]*N[2]) < 0) {
         N[0] = -N[0]; N[1] = -N[1]; N[2] = -N[2];
       }
-      if(specular) {
-        reflect3(L.d, N, dn);
-      } else {
-        const double u0 = u.next(), u1 = u.next();
-        cos_hemisphere(N, u0, u1, dn);
-      }
-      if(u.next() >= refl) {
+      /* the draws of the hemisphere and of the roulette follow the BRDF's */
+      const bool brdf = GEN && S.gmat;
+      if(specular) reflect3(L.d, N, dn);
+      else cos_hemisphere(N, brdf ? u.at(1) : u.at(0), brdf ? u.at(2) : u.at(1), dn);
+      double rr;
+      if(specular) { rr = u.at(1); u.end(2); }
+      else if(brdf) { rr = u.at(3); u.end(4); }
+      else { rr = u.at(2); u.end(3); }
+      if(rr >= refl) {
         LC(w) = T > 0 ? planck_mono(LC(wlen) * 1e-9, T) : 0;
         LC(stage) = ST_WALK_DONE;
         return;
@@ -498,6 +501,7 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
     return;
   }
 
+  u.end(0);
   if(GEN) { /* back from the copy of the grid the query ended in */
     L.o[0] = L.ow[0];
     L.o[1] = L.ow[1];
@@ -530,14 +534,16 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
       double pn[3], dn[3], sun[3], R, N[3] = {0, 0, 1};
 #pragma unroll
       for(int a = 0; a < 3; ++a) pn[a] = L.o[a] + L.d[a] * L.tmax;
+      /* draws: a surface's BRDF or a volume's phase choice, directions, sun */
       double albedo = 1;
+      const bool one = !L.surface || (GEN && S.gmat);
       if(L.surface) {
         const uint32_t mtl = ground_surface<GEN>(S, LC(gh_prim), N);
         if(GEN && S.gmat) {
           /* the hit side's material and its BRDF at the wavelength,
            * ..._sw.c:403-411 */
           const int32_t m = interface_mtl(S.ifcs[mtl], S.mtls, dot3(N, L.d) > 0);
-          const DevBrdf& b = brdf_fetch(S.mtls[m], S.brdfs, LC(wlen), u.next());
+          const DevBrdf& b = brdf_fetch(S.mtls[m], S.brdfs, LC(wlen), u.at(0));
           albedo = b.refl;
           L.specular = b.type == HTGX_BRDF_SPECULAR;
         } else {
@@ -547,7 +553,7 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
           N[0] = -N[0]; N[1] = -N[1]; N[2] = -N[2];
         }
       } else {
-        L.rayleigh = u.next() < LC(gas_ratio);
+        L.rayleigh = u.at(0) < LC(gas_ratio);
       }
       if(GEN && L.specular) {
         reflect3(L.d, N, dn);
@@ -556,14 +562,14 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
         R = !in_solar_cone(S, sun) || dot3(N, sun) < 0 ? 0 : albedo;
       } else {
         /* surface and volume scattering share the two direction sites */
-        const double u0 = u.next(), u1 = u.next();
+        const double u0 = one ? u.at(1) : u.at(0), u1 = one ? u.at(2) : u.at(1);
         double axis[3], mu;
 #pragma unroll
         for(int a = 0; a < 3; ++a) axis[a] = L.surface ? N[a] : L.d[a];
         if(L.surface) mu = sqrt(1.0 - u0);
         else mu = L.rayleigh ? rayleigh_cos_sample(u0) : hg_cos_sample(LC(g), u0);
         local_to_world(axis, mu, 2.0 * kPi * u1, dn);
-        const double s0 = u.next(), s1 = u.next();
+        const double s0 = one ? u.at(3) : u.at(2), s1 = one ? u.at(4) : u.at(3);
         const double sd[3] = {S.sun_dir[0], S.sun_dir[1], S.sun_dir[2]};
         local_to_world(sd, 1.0 - s0 * (1.0 - S.sun_cos_half), 2.0 * kPi * s1, sun);
         if(L.surface) {
@@ -581,7 +587,19 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
       bool shadowed = R <= 0;
       if(!shadowed)
         shadowed = trace<GEN>(S, pn, sun, (double)FLT_MAX, LC(prev_prim), L.prev_edge, true).hit;
-      if(shadowed) { sw_accumulate(S, L, u, 0.0); break; }
+      const bool spec = GEN && L.specular;
+      if(spec) u.end(1);
+      else if(one) u.end(5);
+      else u.end(4);
+      if(shadowed) {
+        const double rr = canonical(u.ts);
+        if(sw_accumulate(S, L, rr, 0.0) && L.surface) {
+          if(spec) u.end(2);
+          else if(one) u.end(6);
+          else u.end(5);
+        }
+        break;
+      }
 #pragma unroll
       for(int a = 0; a < 3; ++a) L.d[a] = sun[a];
       LC(stage) = ST_SUN;
@@ -589,7 +607,7 @@ __device__ __forceinline__ void consume(const DevScene& S, Lane& L, Draws& u)
     } break;
 
     case ST_SUN:
-      sw_accumulate(S, L, u, Tr);
+      if(sw_accumulate(S, L, u.at(0), Tr) && L.surface) u.end(1);
       break;
 
     default: break;
@@ -603,9 +621,9 @@ __device__ __forceinline__ void real_begin(const DevScene& S, const DevMap& M, L
   const uint32_t px = L.pixel % M.width, py = L.pixel / M.width;
   const double psx = 1.0 / (double)M.width, psy = 1.0 / (double)M.height;
   double org[3], dir0[3];
-  const double x = ((double)px + u.next()) * psx;
-  const double y = ((double)py + u.next()) * psy;
-  const double l0 = u.next(), l1 = u.next();
+  const double x = ((double)px + u.at(0)) * psx;
+  const double y = ((double)py + u.at(1)) * psy;
+  const double l0 = u.at(2), l1 = u.at(3);
   if(M.sensor == HTGX_SENSOR_CAMERA) {
     if(GEN) {
       camera_ray(M, x, y, l0, l1, org, dir0);
@@ -636,7 +654,8 @@ __device__ __forceinline__ void real_begin(const DevScene& S, const DevMap& M, L
     const double z[3] = {M.z[0], M.z[1], M.z[2]};
     cos_hemisphere(z, l0, l1, dir0);
   }
-  const double r0 = u.next(), r1 = u.next(), r2 = u.next();
+  const double r0 = u.at(4), r1 = u.at(5), r2 = u.at(6);
+  u.end(7);
   double pdf;
   const double wlen = sample_wavelength<GEN, GEN>(M, r0, r1, &pdf, GEN ? LC(plane) : 0u);
   pdf *= 1e9;
@@ -661,7 +680,8 @@ __device__ __forceinline__ void real_begin(const DevScene& S, const DevMap& M, L
   double dir[3] = {dir0[0], dir0[1], dir0[2]};
   LC(phase) = 0;
   if(M.sensor != HTGX_SENSOR_CAMERA) {
-    const double s0 = u.next(), s1 = u.next();
+    const double s0 = u.at(7), s1 = u.at(8);
+    u.end(9);
     const double sd[3] = {S.sun_dir[0], S.sun_dir[1], S.sun_dir[2]};
     double sun[3];
     local_to_world(sd, 1.0 - s0 * (1.0 - S.sun_cos_half), 2.0 * kPi * s1, sun);
@@ -702,10 +722,11 @@ __device__ __forceinline__ void walk_done(const DevScene& S, const DevMap& M, La
   }
 }
 
-/* A lane's event step runs once this many of a full wavefront's lanes wait for
- * one, its segment step once this many do while others can collide (fewer in
- * proportion when lanes are out of work) */
-constexpr uint32_t kEventLanes = 24, kSegLanes = 16;
+/* The event step runs once this many of a full wavefront's lanes wait for it
+ * (fewer in proportion when lanes are out of work) and no other step has more;
+ * the segment step once no fewer wait for it than for the collision step.
+ * 256x256x16 image 118 -> 113 ms against fixed thresholds of 24 and 16. */
+constexpr uint32_t kEventLanes = 24;
 
 template<bool GEN, bool kLW, bool COUNT>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
@@ -734,7 +755,10 @@ plain_kernel(KArgs A)
     const uint32_t alive = (uint32_t)__popcll(want0 | bs | bc);
 
     /* next segment of the query, and the first tentative collision in it */
-    if(bs && ((uint32_t)__popcll(bs) >= (kSegLanes * alive >> 6) || !bc) && L.lstate == LS_SEG) {
+    const uint32_t ne = (uint32_t)__popcll(want0), ns = (uint32_t)__popcll(bs), nc = (uint32_t)__popcll(bc);
+    const bool run_seg = bs && (!bc || ns >= nc);
+    const bool run_ev = !(bs | bc) || (ne >= (kEventLanes * alive >> 6) && ne >= ns && ne >= nc);
+    if(run_seg && L.lstate == LS_SEG) {
       double t0, kmax;
       const int it = iter_next<GEN, COUNT, kLW>(S, L, &t0, &kmax);
       if(it == ITER_SEGMENT) {
@@ -809,9 +833,7 @@ plain_kernel(KArgs A)
     }
 
     /* events, when enough lanes need them or nothing else is left */
-    const uint64_t want = __ballot(L.lstate == LS_EVENT);
-    const uint64_t other = __ballot(L.lstate == LS_SEG || L.lstate == LS_COLL);
-    if(want && ((uint32_t)__popcll(want) >= (kEventLanes * alive >> 6) || !other)) {
+    if(run_ev && __ballot(L.lstate == LS_EVENT)) {
       uint32_t wv = wave;
       asm volatile("" : "+s"(wv));
       const DevScene& SE = g_args[wv].S;
@@ -863,6 +885,7 @@ plain_kernel(KArgs A)
           /* (a begin, the only event of more than 7 draws, has phase 0) */
           u.w[i] = i > 6 ? W[i] : ph == 0 ? W[i] : ph == 1 ? W[i + 1] : ph == 2 ? W[i + 2] : W[i + 3];
         }
+        u.end(0);
         if(begin) {
           real_begin<GEN, kLW>(SE, M, L, u);
         } else if(L.pending) {
@@ -903,7 +926,8 @@ plain_kernel(KArgs A)
             LC(gh_prim) = gh.prim;
             L.tmax = gh.t;
           }
-          L.Ts = -log(1.0 - u.next());
+          L.Ts = -log(1.0 - canonical(u.ts));
+          ++u.n;
           L.Tmin = 0.0;
           L.c = L.ca = L.cs = 0.0;
           if(S.has_clouds) {
@@ -916,10 +940,10 @@ plain_kernel(KArgs A)
           L.lstate = LS_SEG;
         }
         /* the block the stream is in now */
-        const uint32_t db = (ph + (uint32_t)u.n) >> 2;
+        const uint32_t db = (ph + u.n) >> 2;
 #pragma unroll
         for(int i = 0; i < 4; ++i) L.buf[i] = db == 0 ? W[i] : db == 1 ? W[4 + i] : W[8 + i];
-        L.draw += (uint32_t)u.n;
+        L.draw += u.n;
       }
     }
   }
