@@ -377,7 +377,12 @@ int htgx_draw_map
  * `accum' is a DEVICE pointer to width*height struct htgx_mc_accum, row-major
  * (for a CIE XYZ image: 3 such planes, X then Y then Z; channel c draws from
  * streams keyed by seed ^ (c+1) << 56); `stream' is a hipStream_t (NULL =
- * default stream). Asynchronous. */
+ * default stream). Asynchronous: the accumulators are updated in the order of
+ * `stream'. On the FP32 solver and a stream other than NULL, the drawing that
+ * fills a call's partial sums may run ahead of earlier work on `stream' (it
+ * takes the device as an earlier call's last walks leave it), each context
+ * holding two sets of partial sums for it; under stream capture and with
+ * counters enabled it stays on `stream'. */
 int htgx_render_accum
   (struct htgx_ctx* ctx,
    const struct htgx_map_desc* desc,
