@@ -270,7 +270,12 @@ struct Lane {
  * weights, ground-hit records, chunk sums), kept in LDS as arrays over the
  * block's lanes so that it takes no registers across the tracking steps.
  * Lane t touches element t of each array: no bank conflicts. */
-constexpr int kBlock = 256;
+/* One wavefront to a block: it gives its LDS back when its own last walk ends,
+ * to the blocks of the next call (take_slot); with four it waited for the
+ * longest of theirs (1024x1024 image in two slices 250 -> 241 ms; a terrain
+ * map of 64x64 from scene to pixels 64.9 -> 61.6; other maps alone, the same) */
+constexpr int kBlock = 64;
+constexpr uint32_t kUnit = 4; /* blocks per unit of the grid parameter, 256 lanes */
 struct LaneCold {
   double sum[kBlock], sum2[kBlock]; /* plain FP64 sums over the few realisations of a chunk */
   float pdf[kBlock], g[kBlock], L_sun[kBlock], wlen[kBlock];
@@ -1235,14 +1240,14 @@ __device__ __forceinline__ void walk_done(const SceneF& S, Lane& L)
   }
 }
 
-/* The arguments of the map each wavefront of the block works on (of a batch,
- * the wavefronts may be at different maps). The event step reads its scene,
+/* The arguments of the map the wavefront works on (of a batch, one after the
+ * other). The event step reads its scene,
  * map and launch constants from here: 60-odd of them, in scalar registers
  * they would be live across the tracking steps, and loaded by scalar loads at
  * each event they cost ten dependent waits on the kernel argument segment,
  * 1800-3200 cycles per event step. An LDS broadcast read answers in about
  * 100 cycles. */
-__shared__ KArgs g_args[kBlock / 64];
+__shared__ KArgs g_args[1];
 
 /* The persistent loop of one wavefront over the chunks of one map */
 template<int SENSOR, int SPECTRAL, bool COUNT, int FEAT, bool LIST = false>
@@ -1252,9 +1257,8 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
   const SceneF S = kload(&pK->S);
   const Launch P = kload(&pK->P);
   const uint64_t seed = kload(&pK->M.seed);
-  /* this wavefront's copy of the arguments, for the event step */
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  copy_to_lds(pK, &g_args[wave]);
+  /* the arguments' copy for the event step */
+  copy_to_lds(pK, &g_args[0]);
   /* canonicals per event: 8, plus 2 for the sun of a SW flux map */
   constexpr int NP = (SENSOR == HTGX_SENSOR_RECTANGLE && SPECTRAL == HTGX_SPECTRAL_SW) ? 5 : 4;
   Lane L;
@@ -1444,11 +1448,11 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
       /* the index is opaque to the optimiser (an empty asm statement), so
        * that the reads stay where they are written */
       const SceneF& S_t = S; /* what the tracking steps keep in registers */
-      uint32_t wv = wave;
-      asm volatile("" : "+s"(wv));
-      const SceneF& S = g_args[wv].S;
-      const DevMap& M = g_args[wv].M;
-      const Launch& P = g_args[wv].P;
+      uint32_t at = 0;
+      asm volatile("" : "+s"(at));
+      const SceneF& S = g_args[at].S;
+      const DevMap& M = g_args[at].M;
+      const Launch& P = g_args[at].P;
       if(COUNT) { d_ee++; d_el += __popcll(want); }
       const bool fetch = L.lstate == LS_EVENT && LC(stage) == ST_FETCH;
       if(LIST) {
@@ -1649,7 +1653,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
 /* 3 waves per SIMD: the register cap (168) spills a little but hides more
  * latency than 2 waves without spills (measured 14% faster at 1024^2) */
 template<int SENSOR, int SPECTRAL, bool COUNT, int FEAT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
 wavefront_kernel(KArgs A)
 {
   (void)A;
@@ -1662,7 +1666,7 @@ wavefront_kernel(KArgs A)
  * kernels with the rare and mesh features compiled in, which give the same
  * arithmetic as the leaner instances */
 template<int SENSOR, int SPECTRAL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
 wavefront_list_kernel(KArgs A)
 {
   (void)A;
@@ -1673,7 +1677,7 @@ wavefront_list_kernel(KArgs A)
 /* The FP32 segment iterator on given rays over [0, range[1]] (a debug
  * entry): the segments and their property bounds as the production kernels
  * see them, with the leaf id read back from the leaf record */
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kBlock)
 wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop, uint32_t iband,
                          uint32_t iquad, htgx_segment* segs, uint32_t max_segs, uint32_t* nsegs)
 {
@@ -1733,14 +1737,13 @@ struct BatchScene {
  * uneven scenes of 6.9 M realisations, 135 ms shared out). The map is uniform
  * over a wavefront, so its constants stay scalar. */
 template<int SENSOR, int SPECTRAL, int FEAT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
 wavefront_batch_kernel(const BatchScene* __restrict__ scenes, uint32_t nscenes)
 {
   const uint32_t per_xcd = (gridDim.x + kXcds - 1) / kXcds;
   const uint32_t block = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
-  const uint32_t wave = block * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t s = 0;
-  while(s + 1 < nscenes && scenes[s + 1].first_wave <= wave) ++s;
+  while(s + 1 < nscenes && scenes[s + 1].first_wave <= block) ++s;
   for(uint32_t k = 0; k < nscenes; ++k, s = s + 1 < nscenes ? s + 1 : 0) {
     const BatchScene& B = scenes[s];
     const unsigned int ex = __hip_atomic_load(B.A.P.exhausted, __ATOMIC_RELAXED,
@@ -1814,7 +1817,7 @@ template<class F>
 int launch_variant(F kernel, const SceneF& S, const DevMap& M, const Launch& P, uint32_t grid,
                    hipStream_t stream)
 {
-  kernel<<<grid, 256, 0, stream>>>(KArgs{S, M, P});
+  kernel<<<grid * kUnit, kBlock, 0, stream>>>(KArgs{S, M, P});
   HIP_OK(hipGetLastError());
   return HTGX_OK;
 }
@@ -2135,8 +2138,8 @@ wavefront_build(htgx_ctx* ctx, htgx_wavefront_state* st)
   HIP_OK(hipGetDevice(&dev));
   HIP_OK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu,
-    wavefront_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_SW, false, 0>, 256, 0));
-  st->grid = st->grid_max = (uint32_t)std::max(1, ncu * std::max(1, per_cu));
+    wavefront_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_SW, false, 0>, kBlock, 0));
+  st->grid = st->grid_max = (uint32_t)std::max(1, ncu * std::max(1, per_cu / (int)kUnit));
   if(const char* e = std::getenv("HTGX_WF_GRID")) st->grid = (uint32_t)std::max(1, atoi(e));
   if(const char* e = std::getenv("HTGX_WF_EVTHRESH")) st->ev_thresh = (uint32_t)std::max(1, atoi(e));
   if(const char* e = std::getenv("HTGX_WF_CHUNK")) st->K = (uint32_t)std::min(16, std::max(1, atoi(e)));
@@ -2161,7 +2164,7 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
    * device's grid and not the caller's, so that the sums do not depend on
    * the launch parameters other than the chunk size. */
   const uint64_t nreal = (uint64_t)P->ntiles * 64u * M.spp;
-  const uint64_t most = nreal / ((uint64_t)kChunksPerLane * st->grid_max * kBlock);
+  const uint64_t most = nreal / ((uint64_t)kChunksPerLane * st->grid_max * kUnit * kBlock);
   uint32_t K = (uint32_t)std::min<uint64_t>(std::min(st->K, M.spp), std::max<uint64_t>(1, most));
   while(M.spp % K) --K;
   P->K = K;
@@ -2186,7 +2189,7 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
 static uint32_t
 spread_launch(uint32_t grid, Launch* P)
 {
-  const uint64_t nchunks = (uint64_t)P->ntiles * P->nsub * 64u, nw = kBlock / 64;
+  const uint64_t nchunks = (uint64_t)P->ntiles * P->nsub * 64u, nw = kUnit;
   const uint32_t g = (uint32_t)std::min<uint64_t>(grid, (nchunks + nw - 1) / nw);
   P->lanes = (uint32_t)std::min<uint64_t>(64, (nchunks + nw * g - 1) / (nw * g));
   return g;
@@ -2462,14 +2465,14 @@ static void launch_batch(const htgx_batch_plan* p, hipStream_t stream)
   const uint32_t n = p->n;
   if(p->sensor == HTGX_SENSOR_CAMERA) {
     if(p->spectral == HTGX_SPECTRAL_LW)
-      wavefront_batch_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_LW, FEAT><<<p->grid, 256, 0, stream>>>(p->table, n);
+      wavefront_batch_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_LW, FEAT><<<p->grid * kUnit, kBlock, 0, stream>>>(p->table, n);
     else
-      wavefront_batch_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_SW, FEAT><<<p->grid, 256, 0, stream>>>(p->table, n);
+      wavefront_batch_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_SW, FEAT><<<p->grid * kUnit, kBlock, 0, stream>>>(p->table, n);
   } else {
     if(p->spectral == HTGX_SPECTRAL_LW)
-      wavefront_batch_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_LW, FEAT><<<p->grid, 256, 0, stream>>>(p->table, n);
+      wavefront_batch_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_LW, FEAT><<<p->grid * kUnit, kBlock, 0, stream>>>(p->table, n);
     else
-      wavefront_batch_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_SW, FEAT><<<p->grid, 256, 0, stream>>>(p->table, n);
+      wavefront_batch_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_SW, FEAT><<<p->grid * kUnit, kBlock, 0, stream>>>(p->table, n);
   }
 }
 
@@ -2571,12 +2574,12 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
     total += (double)A.M.width * A.M.height * A.M.spp;
     nchunks += (uint64_t)A.P.ntiles * A.P.nsub * 64u;
   }
-  const uint64_t nw = (uint64_t)p->grid * (kBlock / 64);
+  const uint64_t nw = (uint64_t)p->grid * kUnit;
   for(uint32_t k = 0; k < n; ++k)
     p->table_h[k].A.P.lanes = (uint32_t)std::min<uint64_t>(64, (nchunks + nw - 1) / nw);
   for(uint32_t k = 0; k < n; ++k) {
     const DevMap& M = p->table_h[k].A.M;
-    p->table_h[k].first_wave = (uint32_t)(before / total * ((double)p->grid * (kBlock / 64)));
+    p->table_h[k].first_wave = (uint32_t)(before / total * ((double)p->grid * kUnit));
     before += (double)M.width * M.height * M.spp;
   }
   if(n == 1) {
@@ -2881,14 +2884,14 @@ int htgx_debug_realisations_fp32(htgx_ctx* ctx, const htgx_map_desc* desc, const
     const uint32_t grid = std::min(st->grid_max, (m + 255) / 256);
     if(Mc.sensor == HTGX_SENSOR_CAMERA) {
       if(Mc.spectral_type == HTGX_SPECTRAL_LW)
-        wavefront_list_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_LW><<<grid, 256>>>(KArgs{st->S, Mc, P});
+        wavefront_list_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_LW><<<grid * kUnit, kBlock>>>(KArgs{st->S, Mc, P});
       else
-        wavefront_list_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_SW><<<grid, 256>>>(KArgs{st->S, Mc, P});
+        wavefront_list_kernel<HTGX_SENSOR_CAMERA, HTGX_SPECTRAL_SW><<<grid * kUnit, kBlock>>>(KArgs{st->S, Mc, P});
     } else {
       if(Mc.spectral_type == HTGX_SPECTRAL_LW)
-        wavefront_list_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_LW><<<grid, 256>>>(KArgs{st->S, Mc, P});
+        wavefront_list_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_LW><<<grid * kUnit, kBlock>>>(KArgs{st->S, Mc, P});
       else
-        wavefront_list_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_SW><<<grid, 256>>>(KArgs{st->S, Mc, P});
+        wavefront_list_kernel<HTGX_SENSOR_RECTANGLE, HTGX_SPECTRAL_SW><<<grid * kUnit, kBlock>>>(KArgs{st->S, Mc, P});
     }
     HIP_OK(hipGetLastError());
     std::vector<htgx_mc_accum> acc(m);
@@ -2918,7 +2921,7 @@ int htgx_debug_trace_segments_fp32_impl(htgx_ctx* ctx, const double* rays, uint3
      (res = d_n.alloc(nrays)))
     return res;
   HIP_OK(hipMemcpy(d_rays.p, rays, (size_t)nrays * 8 * sizeof(double), hipMemcpyHostToDevice));
-  wf_trace_segments_kernel<<<(nrays + 255) / 256, 256>>>(ctx->wf->S, d_rays.p, nrays, prop, iband,
+  wf_trace_segments_kernel<<<(nrays + kBlock - 1) / kBlock, kBlock>>>(ctx->wf->S, d_rays.p, nrays, prop, iband,
                                                          iquad, d_segs.p, max_segs, d_n.p);
   HIP_OK(hipGetLastError());
   HIP_OK(hipMemcpy(segs, d_segs.p, (size_t)nrays * max_segs * sizeof(htgx_segment),
