@@ -161,7 +161,7 @@ int device_alloc(htgx_ctx* ctx, size_t n, T** out)
 }
 
 template<class T>
-int upload(htgx_ctx* ctx, const T* host, size_t n, const T** out)
+int upload(htgx_ctx* ctx, const T* host, size_t n, Gptr<const T>* out)
 {
   void* d = nullptr;
   if(!n) { *out = nullptr; return HTGX_OK; }

@@ -55,9 +55,9 @@ struct Launch {
   uint32_t planes;    /* 3 for the channels of a CIE XYZ image, else 1 */
   uint32_t plane_tiles, ntiles, xcd_tiles;
   uint32_t lanes;     /* lanes of each wavefront that take work */
-  unsigned int* counters;   /* [kXcds] next chunk of each XCD range */
-  htgx_mc_accum* partials;  /* [ntiles * nsub * 64] */
-  unsigned long long* stats;
+  Gptr<unsigned int> counters;   /* [kXcds] next chunk of each XCD range */
+  Gptr<htgx_mc_accum> partials;  /* [ntiles * nsub * 64] */
+  Gptr<unsigned long long> stats;
 };
 
 struct KArgs {

@@ -70,20 +70,20 @@ constexpr float kPif = 3.14159265358979323846f;
  * solver where the layout is the same) */
 struct SceneF {
   uint32_t nbands;
-  const double* band_hi;
-  const uint32_t* quad_off;
-  const double* quad_cdf;
+  Gptr<const double> band_hi;
+  Gptr<const uint32_t> quad_off;
+  Gptr<const double> quad_cdf;
   uint32_t nlayers;
   float zb, dzl, inv_dzl;
-  const float* gas_ka; /* [#quads][nlayers] */
-  const float* gas_ks; /* [nbands][nlayers] */
+  Gptr<const float> gas_ka; /* [#quads][nlayers] */
+  Gptr<const float> gas_ks; /* [nbands][nlayers] */
   /* vertical optical depth of gas_ka / gas_ks from the bottom of the gas to
    * the bottom of each layer, same layout (FP64 sums of the FP32 values: a
    * run's depth is a difference of two of them, which FP32 would round to
    * about 1e-7 of the whole column) */
-  const double* cum_ka;
-  const double* cum_ks;
-  const float* gas_T;
+  Gptr<const double> cum_ka;
+  Gptr<const double> cum_ks;
+  Gptr<const float> gas_T;
   int has_clouds;
   uint32_t B;
   uint32_t def[3];
@@ -91,34 +91,34 @@ struct SceneF {
   float lower[3], bs[3], inv_bs[3], inv_cs[3];
   int repeat;        /* clouds repeated along X and Y (-r) */
   float period[2];   /* repetition period: dims0 * bs */
-  const float* lwc;
+  Gptr<const float> lwc;
   /* per finest block: x = level-map word (level << 28 | leaf id), y = the
    * leaf's LWC min (low half) and max (high half) as FP16 multiples of
    * lwc_scale, rounded outwards */
-  const uint2* leafrec;
+  Gptr<const uint2> leafrec;
   float lwc_scale;
-  const float* cka; /* [nbands] cext*(1-ssa) */
-  const float* cks; /* [nbands] cext*ssa */
-  const float* hg_g;
+  Gptr<const float> cka; /* [nbands] cext*(1-ssa) */
+  Gptr<const float> cks; /* [nbands] cext*ssa */
+  Gptr<const float> hg_g;
   int ground_type;
   float plane_z;
   uint32_t plane_mtl;
-  const BvhNode* bvh;   /* mesh ground (shared with the FP64 solver) */
+  Gptr<const BvhNode> bvh;   /* mesh ground (shared with the FP64 solver) */
   uint32_t nbvh;
-  const BvhTri* tris;
-  const uint32_t* tri_mtl;
+  Gptr<const BvhTri> tris;
+  Gptr<const uint32_t> tri_mtl;
   int ground_repeat;         /* -R: the mesh repeats along X, Y */
   float glo[3], ghi[3];      /* the mesh's bounding box */
-  const float* mtl_albedo;
-  const float* mtl_T;
+  Gptr<const float> mtl_albedo;
+  Gptr<const float> mtl_T;
   /* general materials (the FP64 solver's tables): tri_mtl and plane_mtl
    * then index interfaces */
   int gmat;
   int explicit_ifc;
   int32_t sky_mtl;
-  const DevMtl* mtls;
-  const DevBrdf* brdfs;
-  const DevIfc* ifcs;
+  Gptr<const DevMtl> mtls;
+  Gptr<const DevBrdf> brdfs;
+  Gptr<const DevIfc> ifcs;
   float sun_dir[3];
   float sun_cos_half;
   float sun_solid_angle;
@@ -137,26 +137,26 @@ struct Launch {
                             (0: no fewer than can) */
   uint32_t max_steps;    /* micro-step budget of one query */
   uint32_t lanes;        /* lanes of each wavefront that take work (64: all) */
-  unsigned int* counters; /* [kXcds] next chunk of each XCD range */
-  htgx_mc_accum* partials; /* [ntiles*nsub*64] */
-  unsigned long long* stats; /* event counters */
+  Gptr<unsigned int> counters; /* [kXcds] next chunk of each XCD range */
+  Gptr<htgx_mc_accum> partials; /* [ntiles*nsub*64] */
+  Gptr<unsigned long long> stats; /* event counters */
   /* batched launches only (null otherwise): set once the chunk queues are
    * empty; chunks completed, out of nvalid; wall clock of the last one */
-  unsigned int* exhausted;
-  unsigned int* done_count;
-  unsigned long long* done_tick;
+  Gptr<unsigned int> exhausted;
+  Gptr<unsigned int> done_count;
+  Gptr<unsigned long long> done_tick;
   uint32_t nvalid;
   /* queries cut short, counted whether or not counting is on (null: not
    * counted): [0] by the tentative-collision budget, [1] by the segment
    * iterator's bound on passes without a segment */
-  unsigned long long* trunc;
+  Gptr<unsigned long long> trunc;
   /* list launches only (null otherwise): nvalid (pixel, realisation) pairs,
    * one realisation each, whose accumulators go to partials[0..nvalid) */
-  const uint32_t* list;
+  Gptr<const uint32_t> list;
   /* single-map plans replayed from a HIP graph (null otherwise): the
    * realisation offset of the step, read at each chunk fetch instead of
    * spp_offset and advanced on the device after each step */
-  const uint32_t* spp_offset_dev;
+  Gptr<const uint32_t> spp_offset_dev;
 };
 
 /* The arguments of the single-map kernels, one struct: the first argument
@@ -543,8 +543,8 @@ __device__ __forceinline__ TrackRegs track_regs(const SceneF& S, uint32_t max_st
   g.def1 = S.def[1];
   g.B = (float)S.B;
   g.max_steps = max_steps;
-  g.lwc = (GlobalF)S.lwc;
-  g.leafrec = (GlobalU64)S.leafrec;
+  g.lwc = (GlobalF)(const float*)S.lwc;
+  g.leafrec = (GlobalU64)(const uint2*)S.leafrec;
   g.lwc_scale = S.lwc_scale;
   return g;
 }
@@ -1746,7 +1746,7 @@ wavefront_batch_kernel(const BatchScene* __restrict__ scenes, uint32_t nscenes)
   while(s + 1 < nscenes && scenes[s + 1].first_wave <= block) ++s;
   for(uint32_t k = 0; k < nscenes; ++k, s = s + 1 < nscenes ? s + 1 : 0) {
     const BatchScene& B = scenes[s];
-    const unsigned int ex = __hip_atomic_load(B.A.P.exhausted, __ATOMIC_RELAXED,
+    const unsigned int ex = __hip_atomic_load(B.A.P.exhausted.p, __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT);
     if(__builtin_amdgcn_readfirstlane(ex)) continue;
     run_scene<SENSOR, SPECTRAL, false, FEAT>((KPtr<KArgs>)&B.A);
@@ -1951,7 +1951,7 @@ struct DevArrayLite {
 };
 
 template<class T>
-static int upload_f(htgx_wavefront_state* st, const std::vector<T>& v, const T** out)
+static int upload_f(htgx_wavefront_state* st, const std::vector<T>& v, Gptr<const T>* out)
 {
   void* d = nullptr;
   if(v.empty()) { *out = nullptr; return HTGX_OK; }
@@ -1964,7 +1964,7 @@ static int upload_f(htgx_wavefront_state* st, const std::vector<T>& v, const T**
 
 /* FP32 copy of a device FP64 table, uploaded as a new device table */
 template<class T>
-static int upload_as_float(htgx_wavefront_state* st, const T* dptr, size_t n, const float** out)
+static int upload_as_float(htgx_wavefront_state* st, Gptr<const T> dptr, size_t n, Gptr<const float>* out)
 {
   std::vector<T> h(n);
   std::vector<float> f(n);
@@ -2550,7 +2550,7 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
       /* the context's partials and wavelength tables may be reallocated by
        * its next map: the plan keeps copies of its own */
       const size_t np = (size_t)e.A.P.ntiles * e.A.P.nsub * 64u;
-      if((res = plan_alloc(p, np, &e.A.P.partials))) return res;
+      if((res = plan_alloc(p, np, &e.A.P.partials.p))) return res;
       if(e.A.M.nwbands) {
         double *cdf = nullptr, *pdf = nullptr;
         if((res = plan_alloc(p, e.A.M.nwbands, &cdf)) || (res = plan_alloc(p, e.A.M.nwbands, &pdf)))
