@@ -278,22 +278,34 @@ constexpr int kBlock = 64;
 constexpr uint32_t kUnit = 4; /* blocks per unit of the grid parameter, 256 lanes */
 struct LaneCold {
   double sum[kBlock], sum2[kBlock]; /* plain FP64 sums over the few realisations of a chunk */
-  float pdf[kBlock], g[kBlock], L_sun[kBlock], wlen[kBlock];
-  float org[3][kBlock], dir0[3][kBlock], cosN[kBlock], Ld[kBlock]; /* flux SW */
+  float pdf[kBlock], g[kBlock], wlen[kBlock];
   uint32_t t0[kBlock];  /* realisation start, low bits of the wall clock */
-  int stage[kBlock], mask[kBlock], phase[kBlock];
+  int stage[kBlock], phase[kBlock];
   float dir_next[3][kBlock];
-  float ksi[kBlock], w[kBlock], Tr_abs[kBlock], R[kBlock], refl[kBlock], gas_ratio[kBlock],
-        ev_dst[kBlock];
+  float w[kBlock], ev_dst[kBlock];
   int32_t ev_layer[kBlock];
   int32_t prev_prim[kBlock], gh_prim[kBlock]; /* previous surface hit (-1: none), current hit */
   uint32_t gh_mtl[kBlock];
   float tsum[kBlock], tsum2[kBlock];
   uint32_t n[kBlock], nfail[kBlock], chunk[kBlock], r_end[kBlock], plane[kBlock];
+};
+/* what only some kernels have: variables of their own, which take LDS only
+ * where they are used */
+struct LaneColdSw {
+  float L_sun[kBlock], ksi[kBlock], Tr_abs[kBlock], R[kBlock], refl[kBlock], gas_ratio[kBlock];
+  int mask[kBlock];
+};
+struct LaneColdSwFlux {
+  float org[3][kBlock], dir0[3][kBlock], cosN[kBlock], Ld[kBlock];
+};
+struct LaneColdRepeat {
   float shift[2][kBlock]; /* -r: world X/Y of the origin of the lane's frame */
   uint32_t ntiles[kBlock]; /* -r: copies of the grid the query has crossed */
 };
 __shared__ LaneCold g_cold;
+__shared__ LaneColdSw g_cold_sw;
+__shared__ LaneColdSwFlux g_cold_flux;
+__shared__ LaneColdRepeat g_cold_rep;
 /* Cap on the copies of a repeated cloud grid one query crosses */
 constexpr uint32_t kMaxTilesF = 1u << 16;
 /* Lane::nsteps: tentative collisions of the query (at most the budget
@@ -306,6 +318,11 @@ constexpr uint32_t kCollMask = (1u << kCollBits) - 1u;
 constexpr uint32_t kMaxEmptyPasses = 2000;
 #define LC(f) (g_cold.f[threadIdx.x])
 #define LCA(f, a) (g_cold.f[a][threadIdx.x])
+#define LCS(f) (g_cold_sw.f[threadIdx.x])
+#define LCF(f) (g_cold_flux.f[threadIdx.x])
+#define LCFA(f, a) (g_cold_flux.f[a][threadIdx.x])
+#define LCR(f) (g_cold_rep.f[threadIdx.x])
+#define LCRA(f, a) (g_cold_rep.f[a][threadIdx.x])
 
 /* Next pair of FP32 canonicals of the realisation: one Threefry-2x32-20 block
  * with counter (pair index, seed) under the key (pixel, realisation). The
@@ -436,8 +453,8 @@ __device__ __forceinline__ void world_posf(const SceneF& S, const float p[3], fl
   w[1] = p[1];
   w[2] = p[2];
   if(is_repeated<FEAT>(S) && is_mesh<FEAT>(S)) {
-    w[0] += LCA(shift, 0);
-    w[1] += LCA(shift, 1);
+    w[0] += LCRA(shift, 0);
+    w[1] += LCRA(shift, 1);
   }
 }
 
@@ -644,14 +661,14 @@ __device__ __forceinline__ bool next_cell(const SceneF& S, Lane& L, uint32_t c[3
     /* -r: into the next copy of the grid along X or Y; the lane's frame
      * moves with it (a bounded number of copies per query) */
     const int oa = L.exit_axis;
-    if(oa == 2 || !is_repeated<FEAT>(S) || ++LC(ntiles) > kMaxTilesF) return false;
+    if(oa == 2 || !is_repeated<FEAT>(S) || ++LCR(ntiles) > kMaxTilesF) return false;
 #pragma unroll
     for(int a = 0; a < 2; ++a) {
       if(a == oa) {
         const bool pos_dir = L.dir[a] > 0.f;
         const float dp = pos_dir ? S.period[a] : -S.period[a];
         L.pos[a] -= dp;
-        LCA(shift, a) += dp;
+        LCRA(shift, a) += dp;
         c[a] = pos_dir ? 0u : S.dims0[a] - 1;
       }
     }
@@ -668,7 +685,7 @@ __device__ __forceinline__ void iter_init(const SceneF& S, Lane& L)
   L.tit = 0.f;
   L.cstate = 2;
   L.nsteps = 0;
-  if(is_repeated<FEAT>(S)) LC(ntiles) = 0;
+  if(is_repeated<FEAT>(S)) LCR(ntiles) = 0;
 #pragma unroll
   for(int a = 0; a < 3; ++a) L.inv_dir[a] = 1.f / L.dir[a];
   if(S.has_clouds) {
@@ -696,7 +713,7 @@ __device__ __forceinline__ void iter_init(const SceneF& S, Lane& L)
           const float k = floorf((L.pos[a] + te * L.dir[a] - S.lower[a]) / S.period[a]);
           if(k != 0.f) {
             L.pos[a] -= k * S.period[a];
-            LCA(shift, a) += k * S.period[a];
+            LCRA(shift, a) += k * S.period[a];
           }
         }
       }
@@ -879,7 +896,7 @@ __device__ __forceinline__ void request_ground(Lane& L, int mode, int prop)
 
 __device__ __forceinline__ void sw_after_direct(Lane& L)
 {
-  if(!(LC(mask) & HTGX_RADIANCE_DIFFUSE)) { LC(stage) = ST_WALK_DONE; return; }
+  if(!(LCS(mask) & HTGX_RADIANCE_DIFFUSE)) { LC(stage) = ST_WALK_DONE; return; }
   LC(stage) = ST_SCATTER;
   request_ground(L, MODE_SC, HTGX_Ks);
 }
@@ -894,11 +911,11 @@ template<bool COUNT, int FEAT>
 __device__ __forceinline__ void sw_begin(const SceneF& S, Lane& L, int mask, const float p[3],
                                          const float d[3])
 {
-  LC(mask) = mask;
+  LCS(mask) = mask;
 #pragma unroll
   for(int a = 0; a < 3; ++a) { L.pos[a] = p[a]; L.dir[a] = d[a]; }
-  LCA(shift, 0) = LCA(shift, 1) = 0.f; /* a walk starts from a world position */
-  LC(ksi) = 1.f;
+  if(FEAT & kFeatRare) LCRA(shift, 0) = LCRA(shift, 1) = 0.f; /* a walk starts from a world position */
+  LCS(ksi) = 1.f;
   LC(w) = 0.f;
   LC(prev_prim) = -1;
   L.prev_edge = false;
@@ -920,9 +937,9 @@ __device__ __forceinline__ void sw_begin(const SceneF& S, Lane& L, int mask, con
  * (..._sw.c:494-504); the next scattering query starts from the event */
 __device__ __forceinline__ void sw_accumulate(const SceneF& S, Lane& L, float Tr, float u_rr)
 {
-  LC(ksi) *= LC(Tr_abs);
-  LC(w) += LC(ksi) * LC(L_sun) * Tr * LC(R) * S.sun_solid_angle;
-  if(L.surface && u_rr >= LC(refl)) { LC(stage) = ST_WALK_DONE; return; }
+  LCS(ksi) *= LCS(Tr_abs);
+  LC(w) += LCS(ksi) * LCS(L_sun) * Tr * LCS(R) * S.sun_solid_angle;
+  if(L.surface && u_rr >= LCS(refl)) { LC(stage) = ST_WALK_DONE; return; }
 #pragma unroll
   for(int a = 0; a < 3; ++a) L.dir[a] = LCA(dir_next, a);
   LC(stage) = ST_SCATTER;
@@ -944,7 +961,7 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
   if(kLW ? stage != ST_LW : stage == ST_LW) return;
   switch(stage) {
     case ST_DIRECT:
-      LC(w) = LC(L_sun) * query_tr(L);
+      LC(w) = LCS(L_sun) * query_tr(L);
       sw_after_direct(L);
       break;
 
@@ -962,11 +979,11 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
       LC(prev_prim) = L.surface ? LC(gh_prim) : -1;
       L.prev_edge = L.surface && L.gh_edge;
       LC(ev_dst) = dst;
-      LC(Tr_abs) = L.Tmin != 0.0 ? (float)exp(-L.Tmin) : 1.f;
+      LCS(Tr_abs) = L.Tmin != 0.0 ? (float)exp(-L.Tmin) : 1.f;
     }
       [[fallthrough]];
     case ST_ABS: {
-      if(LC(Tr_abs) <= 0.f) { LC(stage) = ST_WALK_DONE; break; }
+      if(LCS(Tr_abs) <= 0.f) { LC(stage) = ST_WALK_DONE; break; }
       const float dst = LC(ev_dst);
       float N[3] = {0.f, 0.f, 1.f};
 #pragma unroll
@@ -979,10 +996,10 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
            * ..._sw.c:403-411 (the canonical of the phase choice) */
           const int32_t m = interface_mtl(S.ifcs[LC(gh_mtl)], S.mtls, dot3f(N, L.dir) > 0.f);
           const DevBrdf& b = brdf_fetch(S.mtls[m], S.brdfs, (double)LC(wlen), (double)u[4]);
-          LC(refl) = (float)b.refl;
+          LCS(refl) = (float)b.refl;
           specular = b.type == HTGX_BRDF_SPECULAR;
         } else {
-          LC(refl) = S.mtl_albedo[LC(gh_mtl)];
+          LCS(refl) = S.mtl_albedo[LC(gh_mtl)];
         }
         face_forwardf(N, L.dir);
         float dn[3];
@@ -994,13 +1011,13 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
 #pragma unroll
         for(int a = 0; a < 3; ++a) LCA(dir_next, a) = dn[a];
       } else {
-        L.rayleigh = u[4] < LC(gas_ratio);
+        L.rayleigh = u[4] < LCS(gas_ratio);
         const float mu = L.rayleigh ? rayleigh_cosf(u[0]) : hg_cosf(LC(g), u[0]);
         float dn[3];
         local_to_worldf(L.dir, mu, 2.f * kPif * u[1], dn);
 #pragma unroll
         for(int a = 0; a < 3; ++a) LCA(dir_next, a) = dn[a];
-        LC(refl) = 1.f;
+        LCS(refl) = 1.f;
       }
       float sun_dir[3];
       local_to_worldf(S.sun_dir, 1.f - u[2] * (1.f - S.sun_cos_half), 2.f * kPif * u[3], sun_dir);
@@ -1010,15 +1027,15 @@ __device__ __forceinline__ void consume(const SceneF& S, Lane& L, const float* u
 #pragma unroll
         for(int a = 0; a < 3; ++a) sun_dir[a] = LCA(dir_next, a);
         const bool lit = dot3f(sun_dir, S.sun_dir) >= S.sun_cos_half && dot3f(N, sun_dir) >= 0.f;
-        LC(R) = lit ? LC(refl) / S.sun_solid_angle : 0.f;
+        LCS(R) = lit ? LCS(refl) / S.sun_solid_angle : 0.f;
       } else if(L.surface) {
         const float c = dot3f(N, sun_dir);
-        LC(R) = c < 0.f ? 0.f : LC(refl) / kPif * c;
+        LCS(R) = c < 0.f ? 0.f : LCS(refl) / kPif * c;
       } else {
         const float mu = dot3f(L.dir, sun_dir);
-        LC(R) = L.rayleigh ? rayleigh_evalf(mu) : hg_evalf(LC(g), mu);
+        LCS(R) = L.rayleigh ? rayleigh_evalf(mu) : hg_evalf(LC(g), mu);
       }
-      bool shadowed = LC(R) <= 0.f;
+      bool shadowed = LCS(R) <= 0.f;
       if(!shadowed) {
         float wp[3];
         world_posf<FEAT>(S, L.pos, wp);
@@ -1191,7 +1208,7 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
   LC(g) = S.has_clouds ? S.hg_g[band] : 0.f;
   L.cka = S.has_clouds ? S.cka[band] : 0.f;
   L.cks = S.has_clouds ? S.cks[band] : 0.f;
-  LC(L_sun) = planckf(LC(wlen), 5778.f);
+  if(SPECTRAL != HTGX_SPECTRAL_LW) LCS(L_sun) = planckf(LC(wlen), 5778.f);
 
   if(SPECTRAL == HTGX_SPECTRAL_LW) {
     LC(phase) = 0;
@@ -1209,11 +1226,11 @@ __device__ __forceinline__ void real_begin(const SceneF& S, const DevMap& M, Lan
     float sun_dir[3];
     local_to_worldf(S.sun_dir, 1.f - u[7] * (1.f - S.sun_cos_half), 2.f * kPif * u[8], sun_dir);
     const float z[3] = {(float)M.z[0], (float)M.z[1], (float)M.z[2]};
-    LC(cosN) = dot3f(z, sun_dir);
-    LC(Ld) = 0.f;
+    LCF(cosN) = dot3f(z, sun_dir);
+    LCF(Ld) = 0.f;
 #pragma unroll
-    for(int a = 0; a < 3; ++a) { LCA(org, a) = org[a]; LCA(dir0, a) = dir[a]; }
-    if(LC(cosN) > 0.f) { LC(phase) = 1; sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_DIRECT, org, sun_dir); }
+    for(int a = 0; a < 3; ++a) { LCFA(org, a) = org[a]; LCFA(dir0, a) = dir[a]; }
+    if(LCF(cosN) > 0.f) { LC(phase) = 1; sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_DIRECT, org, sun_dir); }
     else { LC(phase) = 2; sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_DIFFUSE, org, dir); }
   }
 }
@@ -1228,15 +1245,15 @@ __device__ __forceinline__ void walk_done(const SceneF& S, Lane& L)
     LC(stage) = ST_REAL_DONE;
     LC(w) = LC(w) * kPif / LC(pdf);
   } else if(LC(phase) == 1) {
-    LC(Ld) = LC(w);
+    LCF(Ld) = LC(w);
     LC(phase) = 2;
     float o[3], d[3];
 #pragma unroll
-    for(int a = 0; a < 3; ++a) { o[a] = LCA(org, a); d[a] = LCA(dir0, a); }
+    for(int a = 0; a < 3; ++a) { o[a] = LCFA(org, a); d[a] = LCFA(dir0, a); }
     sw_begin<COUNT, FEAT>(S, L, HTGX_RADIANCE_DIFFUSE, o, d);
   } else {
     LC(stage) = ST_REAL_DONE;
-    LC(w) = (LC(cosN) * S.sun_solid_angle * LC(Ld) + kPif * LC(w)) / LC(pdf);
+    LC(w) = (LCF(cosN) * S.sun_solid_angle * LCF(Ld) + kPif * LC(w)) / LC(pdf);
   }
 }
 
@@ -1408,7 +1425,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
           L.ev = uu.x < proba ? EV_HIT : EV_NONE;
           if(!kLW && L.mode == MODE_SC && L.ev != EV_NONE) {
             /* gas vs particle scattering at the event, ..._sw.c:427-438 */
-            LC(gas_ratio) = gks / ks;
+            LCS(gas_ratio) = gks / ks;
             /* the absorption optical depth stops at the event */
             const float amin = gka + (L.s_cloud ? L.cka * L.lmn : 0.f);
             L.Tmin -= (double)(L.s_t1 - tx) * (double)amin;
@@ -1504,7 +1521,7 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
         if(begin) {
           L.pair = 0;
           LC(t0) = (uint32_t)wall_clock64();
-          LCA(shift, 0) = LCA(shift, 1) = 0.f; /* sensor rays start in world coordinates */
+          if(FEAT & kFeatRare) LCRA(shift, 0) = LCRA(shift, 1) = 0.f; /* sensor rays start in world coordinates */
         }
         /* one set of canonicals per event, drawn at a single site */
         float u[2 * NP];
@@ -1650,10 +1667,18 @@ __device__ __forceinline__ void run_scene(KPtr<KArgs> pK)
   }
 }
 
-/* 3 waves per SIMD: the register cap (168) spills a little but hides more
- * latency than 2 waves without spills (measured 14% faster at 1024^2) */
+/* Wavefronts per SIMD. Shortwave: 3; the register cap (168) spills a little
+ * with the rare features but hides more latency than 2 wavefronts without
+ * spills (14 % faster at 1024x1024), and 4 would spill a fifth of the tracking
+ * state. Longwave without the rare features: its tracking has no second
+ * optical thickness and no sun, and fits the 128 registers of 4 without
+ * spills; with its own 7.5 KB of LDS the compute unit holds them (512x512 flux
+ * map x 64: 158 -> 140 ms, x 16: 55.6 -> 52.2) */
+template<int SPECTRAL, int FEAT>
+constexpr int waves() { return SPECTRAL == HTGX_SPECTRAL_LW && !(FEAT & kFeatRare) ? 4 : 3; }
+
 template<int SENSOR, int SPECTRAL, bool COUNT, int FEAT>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves<SPECTRAL, FEAT>())))
 wavefront_kernel(KArgs A)
 {
   (void)A;
@@ -1692,7 +1717,7 @@ wf_trace_segments_kernel(SceneF S, const double* rays, uint32_t nrays, int prop,
   L.gks_off = iband * S.nlayers;
   L.cka = S.has_clouds ? S.cka[iband] : 0.f;
   L.cks = S.has_clouds ? S.cks[iband] : 0.f;
-  LCA(shift, 0) = LCA(shift, 1) = 0.f;
+  LCRA(shift, 0) = LCRA(shift, 1) = 0.f;
   iter_init<kFeatRare>(S, L);
   uint32_t n = 0;
   float t0;
@@ -1737,7 +1762,7 @@ struct BatchScene {
  * uneven scenes of 6.9 M realisations, 135 ms shared out). The map is uniform
  * over a wavefront, so its constants stay scalar. */
 template<int SENSOR, int SPECTRAL, int FEAT>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves<SPECTRAL, FEAT>())))
 wavefront_batch_kernel(const BatchScene* __restrict__ scenes, uint32_t nscenes)
 {
   const uint32_t per_xcd = (gridDim.x + kXcds - 1) / kXcds;
@@ -2182,6 +2207,20 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
   return HTGX_OK;
 }
 
+/* Grid of a launch: the grid parameter, which counts a device filled at 3
+ * wavefronts per SIMD, and a third more for the kernels that hold 4 (waves())
+ * if that leaves a lane of the former 16 realisations at least. With fewer, the longest
+ * walks bound the launch and run slower four to a SIMD: longwave images of
+ * 256x256 and 512x512 at 5.3, 10.7, 21 and 85 realisations a lane 15.4 / 22.4
+ * / 27.7 / 59.4 ms against 14.5 / 20.4 / 27.7 / 63.5 with 3; flux maps 23.6 /
+ * 32.3 / 53.3 / 140 against 22.0 / 33.6 / 54.8 / 158. */
+static uint32_t
+kernel_grid(uint32_t grid, int spectral, int feat, uint64_t nreal)
+{
+  const bool four = spectral == HTGX_SPECTRAL_LW && !(feat & kFeatRare);
+  return four && nreal >= 16ull * grid * kUnit * kBlock ? grid + grid / 3 : grid;
+}
+
 /* Grid of a launch of its own, at most `grid' blocks: with fewer chunks than
  * lanes, the chunks spread evenly over all wavefronts (one to a wavefront if
  * there are that few) instead of filling the first ones: a lane that shares
@@ -2309,7 +2348,8 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   }
   CallSlot* slot = nullptr;
   if((res = setup_launch(ctx, M, planes, &P, stream, &slot)) != HTGX_OK) return res;
-  const uint32_t grid = spread_launch(st->grid, &P);
+  const uint32_t grid = spread_launch(kernel_grid(st->grid, M.spectral_type, features(st->S, M),
+                                                (uint64_t)M.width * M.height * planes * M.spp), &P);
   const hipStream_t draw = slot ? slot->stream : stream;
   /* the slot's partials are free once its last call has merged them */
   if(slot && slot->used) HIP_OK(hipStreamWaitEvent(draw, slot->merged, 0));
@@ -2370,7 +2410,8 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, uint32_t plane
             kScratchBytes >> 20);
     return HTGX_BAD_ARG;
   }
-  const uint32_t grid = spread_launch(st->grid, &P);
+  const uint32_t grid = spread_launch(kernel_grid(st->grid, M.spectral_type, features(st->S, M),
+                                                (uint64_t)M.width * M.height * planes * M.spp), &P);
   P.counters = (unsigned int*)base;
   P.partials = (htgx_mc_accum*)(base + kScratchHead);
   /* fill kernels, no memset: the call may be captured in a graph */
@@ -2574,6 +2615,7 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
     total += (double)A.M.width * A.M.height * A.M.spp;
     nchunks += (uint64_t)A.P.ntiles * A.P.nsub * 64u;
   }
+  p->grid = kernel_grid(p->grid, p->spectral, p->feat, (uint64_t)total);
   const uint64_t nw = (uint64_t)p->grid * kUnit;
   for(uint32_t k = 0; k < n; ++k)
     p->table_h[k].A.P.lanes = (uint32_t)std::min<uint64_t>(64, (nchunks + nw - 1) / nw);
