@@ -1954,7 +1954,7 @@ struct htgx_wavefront_state {
   void* d_partials = nullptr;
   size_t partials_cap = 0;
   uint32_t grid = 0;
-  uint32_t grid_max = 0; /* resident blocks of the device */
+  uint32_t grid_max = 0; /* resident units of 256 lanes */
   uint32_t K = 4;
   uint32_t ev_thresh = 24;
   uint32_t seg_thresh = 0;

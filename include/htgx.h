@@ -88,7 +88,7 @@ enum htgx_projection {
 };
 
 enum htgx_solver {
-  HTGX_SOLVER_PLAIN_FP64 = 0,    /* one path per thread, FP64 everywhere */
+  HTGX_SOLVER_PLAIN_FP64 = 0,    /* one path per lane, FP64 everywhere */
   HTGX_SOLVER_WAVEFRONT_FP32 = 1 /* FP32 transport, FP64 Tmin + accumulators */
 };
 
@@ -424,9 +424,11 @@ struct htgx_wf_params {
                          step */
   uint32_t chunk;     /* realisations per work-queue chunk at most (1-16; 0 =
                          default 4; small maps take smaller ones) */
-  uint32_t grid;      /* blocks of 256 lanes of the persistent launch
-                         (1-grid_max; 0 = grid_max) */
-  uint32_t grid_max;  /* read only: blocks resident on the device at once */
+  uint32_t grid;      /* units of 256 lanes of the persistent launch
+                         (1-grid_max; 0 = grid_max); large longwave maps
+                         take a third more */
+  uint32_t grid_max;  /* read only: units resident on the device at once, at 3
+                         wavefronts per SIMD */
   uint32_t seg_thresh; /* lanes of a 64-lane wavefront that must wait for the
                           segment step before it runs while other lanes can
                           take a collision step (1-64, 1: run it whenever a
