@@ -770,6 +770,7 @@ extern "C" int
 htgx_ctx_destroy(htgx_ctx* ctx)
 {
   if(!ctx) return HTGX_BAD_ARG;
+  htgx_wavefront_release(ctx); /* waits for its own streams, which read the buffers below */
   for(void* p : ctx->bufs) (void)hipFree(p);
   if(ctx->d_partials) (void)hipFree(ctx->d_partials);
   if(ctx->d_plain_queue) (void)hipFree(ctx->d_plain_queue);
@@ -777,7 +778,6 @@ htgx_ctx_destroy(htgx_ctx* ctx)
   if(ctx->d_wpdf) (void)hipFree(ctx->d_wpdf);
   if(ctx->d_cie_cdf) (void)hipFree(ctx->d_cie_cdf);
   if(ctx->d_counters) (void)hipFree(ctx->d_counters);
-  htgx_wavefront_release(ctx);
   delete ctx;
   return HTGX_OK;
 }
