@@ -2312,7 +2312,7 @@ setup_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P, hipStre
     return HTGX_OK;
   }
   if(need > st->partials_cap) {
-    if(st->d_partials) { HIP_OK(hipFree(st->d_partials)); st->d_partials = nullptr; }
+    if(st->d_partials) { HIP_OK(hipFree(st->d_partials)); st->d_partials = nullptr; st->partials_cap = 0; }
     HIP_OK(hipMalloc(&st->d_partials, need));
     st->partials_cap = need;
   }

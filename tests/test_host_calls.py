@@ -1,0 +1,78 @@
+"""What the library does around its kernels, on the CPU: the buffers it holds,
+the streams it launches on and what it waits for, recorded by a HIP runtime
+without a device (hip_recorder.cpp, preloaded into a process of its own)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C
+from htrdr_kmin_amd import _ffi as F
+from htrdr_kmin_amd import atmosphere as A
+
+R = C.CDLL(None)
+R.recorder_log.restype = R.recorder_live_bytes.restype = C.c_size_t
+R.recorder_log.argtypes = [C.c_char_p, C.c_size_t]
+R.recorder_fail_above.argtypes = [C.c_size_t]
+synth = A.Synth(0, seed=0)
+
+
+def log():
+    buf = C.create_string_buffer(R.recorder_log(None, 0) + 1)
+    R.recorder_log(buf, len(buf))
+    return buf.value.decode().splitlines()
+
+
+def map_of(width, height, spp, solver=F.SOLVER_WAVEFRONT_FP32, **kw):
+    return A.map_preset(0, width=width, height=height, spp=spp, solver=solver, **kw)
+
+
+def recorded(f, *args):
+    R.recorder_clear()
+    f(*args)
+    return log()
+
+
+ACCUM = 1 << 40  # only kernels would read it
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    lib = tmp_path_factory.mktemp("recorder") / "recorder.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", str(lib),
+                    os.path.join(HERE, "hip_recorder.cpp")], check=True)
+
+    def call(code):
+        before = os.environ.get("LD_PRELOAD")
+        env = dict(os.environ, LD_PRELOAD=f"{lib}:{before}" if before else str(lib))
+        r = subprocess.run([sys.executable, "-c", PRELUDE + code], cwd=ROOT, env=env, timeout=300,
+                           capture_output=True, text=True)
+        assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
+        return r.stdout
+
+    return call
+
+
+@pytest.mark.parametrize("solver", ["F.SOLVER_WAVEFRONT_FP32", "F.SOLVER_PLAIN_FP64"])
+def test_partials_after_a_failed_allocation(run, solver):
+    """A call that finds no memory for its partial sums is an error; the next
+    one, smaller, has partial sums to write to."""
+    run(f"""
+small, big = map_of(16, 16, 4, {solver}), map_of(256, 256, 32, {solver})
+with A.Context(synth.scene_ptr) as ctx:
+    ctx.render_accum(small, ACCUM)
+    R.recorder_fail_above(1 << 20)
+    try:
+        ctx.render_accum(big, ACCUM)
+        raise SystemExit("no error")
+    except F.HtgxError as e:
+        assert e.code == F.MEM_ERR
+    lines = recorded(ctx.render_accum, small, ACCUM)
+    assert any(l.startswith("malloc") for l in lines[:-2]), lines
+""")
