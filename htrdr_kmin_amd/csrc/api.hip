@@ -962,6 +962,7 @@ htgx_map_setup(htgx_ctx* ctx, const htgx_map_desc* d, DevMap* M, bool may_alloca
       cdf[nwb - 1] = 1.0;
       if(ctx->d_wcdf) { (void)hipFree(ctx->d_wcdf); ctx->d_wcdf = nullptr; }
       if(ctx->d_wpdf) { (void)hipFree(ctx->d_wpdf); ctx->d_wpdf = nullptr; }
+      ctx->w_nbands = 0; /* no map's until both are filled */
       HIP_OK(hipMalloc(&ctx->d_wcdf, nwb * sizeof(double)));
       HIP_OK(hipMalloc(&ctx->d_wpdf, nwb * sizeof(double)));
       HIP_OK(hipMemcpy(ctx->d_wcdf, cdf.data(), nwb * sizeof(double), hipMemcpyHostToDevice));

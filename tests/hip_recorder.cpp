@@ -29,6 +29,7 @@ std::map<void*, size_t> live;
 std::map<void*, std::set<Event*>> waits; /* per stream */
 std::set<Event*> events;
 size_t fail_above = SIZE_MAX;
+int fail_in = 0; /* the allocation to fail: 1 the next */
 void* captured = nullptr;
 int capture_mode = 0;
 Dim3 grid_, block_;
@@ -56,6 +57,7 @@ size_t recorder_log(char* out, size_t n)
 }
 void recorder_clear(void) { log_.clear(); }
 void recorder_fail_above(size_t n) { fail_above = n; }
+void recorder_fail_in(int n) { fail_in = n; }
 size_t recorder_live_bytes(void)
 {
   size_t n = 0;
@@ -89,7 +91,7 @@ int hipLaunchKernel(const void* f, Dim3 g, Dim3, void**, size_t, void* s)
 }
 int hipMalloc(void** p, size_t n)
 {
-  if(refused() || n > fail_above) {
+  if(refused() || n > fail_above || (fail_in && !--fail_in)) {
     note("malloc %zu refused", n);
     return refused() ? (int)CAPTURING : (int)NO_MEMORY;
   }

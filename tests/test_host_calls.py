@@ -19,7 +19,7 @@ R = C.CDLL(None)
 R.recorder_log.restype = R.recorder_live_bytes.restype = C.c_size_t
 R.recorder_log.argtypes = [C.c_char_p, C.c_size_t]
 R.recorder_fail_above.argtypes = [C.c_size_t]
-synth = A.Synth(0, seed=0)
+synth = A.Synth(0, seed=0, nbands=4, wlen_lo=380.0, wlen_hi=780.0)
 
 
 def log():
@@ -75,4 +75,26 @@ with A.Context(synth.scene_ptr) as ctx:
         assert e.code == F.MEM_ERR
     lines = recorded(ctx.render_accum, small, ACCUM)
     assert any(l.startswith("malloc") for l in lines[:-2]), lines
+""")
+
+
+@pytest.mark.parametrize("spectral", ["F.SPECTRAL_SW", "F.SPECTRAL_SW_CIE_XYZ"])
+@pytest.mark.parametrize("at", [1, 2])
+def test_wavelength_tables_after_a_failed_allocation(run, spectral, at):
+    """A map of another wavelength range whose tables find no memory is an
+    error; the next map of the range before has tables to read."""
+    run(f"""
+def band(lo, hi):
+    return map_of(16, 16, 4, spectral_type={spectral}, wlen_range=(lo, hi))
+
+with A.Context(synth.scene_ptr) as ctx:
+    ctx.render_accum(band(500.0, 600.0), ACCUM)
+    R.recorder_fail_in({at})
+    try:
+        ctx.render_accum(band(450.0, 700.0), ACCUM)
+    except F.HtgxError as e:
+        assert e.code == F.MEM_ERR
+        lines = recorded(ctx.render_accum, band(500.0, 600.0), ACCUM)
+        assert any(l.startswith("malloc") for l in lines[:-2]), lines
+    R.recorder_fail_in(0)
 """)
