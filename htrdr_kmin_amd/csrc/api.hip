@@ -927,6 +927,7 @@ htgx_map_setup(htgx_ctx* ctx, const htgx_map_desc* d, DevMap* M, bool may_alloca
         }
         f[nwb - 1] = 1.0;
       }
+      if(const int res = htgx_wavefront_wait(ctx)) return res; /* drawings that read the old ones */
       if(ctx->d_cie_cdf) { (void)hipFree(ctx->d_cie_cdf); ctx->d_cie_cdf = nullptr; }
       ctx->cie_nbands = 0;
       HIP_OK(hipMalloc(&ctx->d_cie_cdf, 3 * nwb * sizeof(double)));
@@ -960,6 +961,7 @@ htgx_map_setup(htgx_ctx* ctx, const htgx_map_desc* d, DevMap* M, bool may_alloca
         cdf[i] = i ? pdf[i] + cdf[i - 1] : pdf[i];
       }
       cdf[nwb - 1] = 1.0;
+      if(const int res = htgx_wavefront_wait(ctx)) return res; /* drawings that read the old ones */
       if(ctx->d_wcdf) { (void)hipFree(ctx->d_wcdf); ctx->d_wcdf = nullptr; }
       if(ctx->d_wpdf) { (void)hipFree(ctx->d_wpdf); ctx->d_wpdf = nullptr; }
       ctx->w_nbands = 0; /* no map's until both are filled */

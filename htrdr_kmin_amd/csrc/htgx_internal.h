@@ -114,6 +114,9 @@ int htgx_render_channels(htgx_ctx* ctx, const htgx::DevMap& map, uint32_t planes
  * and partials in the library's static scratch array */
 int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const htgx::DevMap& map, uint32_t planes,
                                   htgx_mc_accum* accum, hipStream_t stream);
+/* Wait for the calls in flight on the FP32 solver, whose drawings may run on
+ * streams of the context's own */
+int htgx_wavefront_wait(htgx_ctx* ctx);
 void htgx_wavefront_release(htgx_ctx* ctx);
 
 #endif /* HTGX_INTERNAL_H */

@@ -2972,6 +2972,14 @@ int htgx_debug_trace_segments_fp32_impl(htgx_ctx* ctx, const double* rays, uint3
   return HTGX_OK;
 }
 
+int htgx_wavefront_wait(htgx_ctx* ctx)
+{
+  if(!ctx->wf) return HTGX_OK;
+  for(const CallSlot& s : ctx->wf->slots)
+    if(s.used) HIP_OK(hipEventSynchronize(s.merged));
+  return HTGX_OK;
+}
+
 void htgx_wavefront_release(htgx_ctx* ctx)
 {
   if(!ctx || !ctx->wf) return;

@@ -32,6 +32,10 @@ def map_of(width, height, spp, solver=F.SOLVER_WAVEFRONT_FP32, **kw):
     return A.map_preset(0, width=width, height=height, spp=spp, solver=solver, **kw)
 
 
+def first(lines, what):
+    return next(i for i, l in enumerate(lines) if l.startswith(what))
+
+
 def recorded(f, *args):
     R.recorder_clear()
     f(*args)
@@ -97,4 +101,22 @@ with A.Context(synth.scene_ptr) as ctx:
         lines = recorded(ctx.render_accum, band(500.0, 600.0), ACCUM)
         assert any(l.startswith("malloc") for l in lines[:-2]), lines
     R.recorder_fail_in(0)
+""")
+
+
+@pytest.mark.parametrize("spectral", ["F.SPECTRAL_SW", "F.SPECTRAL_SW_CIE_XYZ"])
+def test_wavelength_tables_outlive_the_drawings_that_read_them(run, spectral):
+    """A map of another range waits for the drawings in flight, on whichever
+    stream they run, before it frees the tables these read."""
+    run(f"""
+def band(lo, hi):
+    return map_of(16, 16, 4, spectral_type={spectral}, wlen_range=(lo, hi))
+
+with A.Context(synth.scene_ptr) as ctx:
+    for i in range(3):
+        ctx.render_accum(band(500.0, 600.0), ACCUM, 64)
+    merges = {{l.split()[-1] for l in log() if l.startswith("record stream 0x40 ")}}
+    lines = recorded(ctx.render_accum, band(450.0, 700.0), ACCUM, 64)
+    before = lines[:first(lines, "free")]
+    assert merges and merges == {{l.split()[-1] for l in before if l.startswith("sync event")}}, lines
 """)
