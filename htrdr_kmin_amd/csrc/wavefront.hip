@@ -2250,6 +2250,33 @@ same_schedule(hipStream_t stream, hipStream_t own)
     && hipExtStreamGetCUMask(own, 16, n) == hipSuccess && !std::memcmp(m, n, sizeof(m));
 }
 
+/* Whether `stream' is being captured (or cannot say) */
+static bool
+is_captured(hipStream_t stream)
+{
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if(stream && hipStreamIsCapturing(stream, &cs) != hipSuccess) { (void)hipGetLastError(); return true; }
+  return cs != hipStreamCaptureStatusNone;
+}
+
+/* Make the partials of a slot those of the calls on the caller's stream, where
+ * these are too few for a call under capture, which cannot allocate: a caller
+ * that drew the map before it captures the call holds enough of them in a
+ * slot. A graph may hold the former ones: they stay until the context goes. */
+static void
+take_over_partials(htgx_wavefront_state* st, size_t need)
+{
+  for(CallSlot& s : st->slots) {
+    if(s.cap < need) continue;
+    if(st->d_partials) st->bufs.push_back(st->d_partials);
+    st->d_partials = s.partials;
+    st->partials_cap = s.cap;
+    s.partials = nullptr;
+    s.cap = 0;
+    break;
+  }
+}
+
 /* The slot of a call on `stream' whose partials take `need' bytes, or null to
  * run the call on `stream' itself.
  * A map's last walks leave most of the device idle: some 45 of the 140 ms of
@@ -2272,9 +2299,7 @@ take_slot(htgx_ctx* ctx, size_t need, hipStream_t stream)
 {
   htgx_wavefront_state* st = ctx->wf;
   if(!stream || ctx->counting || need > kMaxSlotPartials) return nullptr;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if(hipStreamIsCapturing(stream, &cs) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-  if(cs != hipStreamCaptureStatusNone) return nullptr;
+  if(is_captured(stream)) return nullptr;
   int dev = 0;
   if(hipGetDevice(&dev) != hipSuccess || dev != ctx->device) return nullptr;
   CallSlot& s = st->slots[st->next_slot];
@@ -2311,6 +2336,7 @@ setup_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P, hipStre
     P->partials = (htgx_mc_accum*)(*slot)->partials;
     return HTGX_OK;
   }
+  if(need > st->partials_cap && is_captured(stream)) take_over_partials(st, need);
   if(need > st->partials_cap) {
     if(st->d_partials) { HIP_OK(hipFree(st->d_partials)); st->d_partials = nullptr; st->partials_cap = 0; }
     HIP_OK(hipMalloc(&st->d_partials, need));

@@ -382,7 +382,10 @@ int htgx_draw_map
  * fills a call's partial sums may run ahead of earlier work on `stream' (it
  * takes the device as an earlier call's last walks leave it), each context
  * holding two sets of partial sums for it; under stream capture and with
- * counters enabled it stays on `stream'. */
+ * counters enabled it stays on `stream'. A call can be captured, in any
+ * capture mode, once one of as many realisations has been made uncaptured on
+ * any stream: it then allocates nothing. What the graph reads stays until the
+ * context is destroyed. */
 int htgx_render_accum
   (struct htgx_ctx* ctx,
    const struct htgx_map_desc* desc,

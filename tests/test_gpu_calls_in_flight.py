@@ -1,5 +1,7 @@
 """FP32 calls in flight together, whose results are those of the same calls one
 at a time, bit for bit (the run times of the realisations aside)."""
+import ctypes as C
+
 import pytest
 
 from htrdr_kmin_amd import _ffi as F
@@ -33,3 +35,34 @@ def test_the_wavelength_range_changes_between_calls(ctx, spectral):
     stream.destroy()
     for d, acc in zip(ds, accs):
         assert same(acc, one_at_a_time(ctx, [d, d]), d)
+
+
+@pytest.mark.parametrize("mode", [0, 1])  # global, thread-local: both refuse allocations
+@pytest.mark.parametrize("calls", [1, 3])
+def test_capture_after_calls_on_the_same_stream(mode, calls):
+    """From a new context, calls on a stream, then the capture of one like
+    them on it, replayed with larger ones in between."""
+    h = H.hip()
+    s = A.Synth(0, seed=6)
+    d, e = (A.map_preset(0, width=w, height=w, spp=8, seed=3, solver=F.SOLVER_WAVEFRONT_FP32)
+            for w in (40, 64))
+    graph, run = C.c_void_p(), C.c_void_p()
+    acc, other, stream = buffer(d), buffer(e), H.Stream()
+    with A.Context(s.scene_ptr) as ctx:
+        for _ in range(calls):
+            ctx.render_accum(d, acc.address, stream.h.value)
+        H.ok("hipStreamBeginCapture", h.hipStreamBeginCapture(stream.h, C.c_int(mode)))
+        ctx.render_accum(d, acc.address, stream.h.value)
+        H.ok("hipStreamEndCapture", h.hipStreamEndCapture(stream.h, C.byref(graph)))
+        H.ok("hipGraphInstantiate", h.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+        for _ in range(3):
+            H.ok("hipGraphLaunch", h.hipGraphLaunch(run, stream.h))
+            ctx.render_accum(e, other.address, stream.h.value)
+        H.ok("hipGraphLaunch", h.hipGraphLaunch(run, stream.h))
+        stream.synchronize()
+        assert same(acc, one_at_a_time(ctx, [d] * (calls + 4)), d)
+        assert same(other, one_at_a_time(ctx, [e] * 3), e)
+        h.hipGraphExecDestroy(run)
+        h.hipGraphDestroy(graph)
+        stream.destroy()
+    s.close()
