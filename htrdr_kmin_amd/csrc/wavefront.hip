@@ -271,7 +271,7 @@ struct Lane {
  * block's lanes so that it takes no registers across the tracking steps.
  * Lane t touches element t of each array: no bank conflicts. */
 /* One wavefront to a block: it gives its LDS back when its own last walk ends,
- * to the blocks of the next call (take_slot); with four it waited for the
+ * to the blocks of the next call (take_set); with four it waited for the
  * longest of theirs (1024x1024 image in two slices 250 -> 241 ms; a terrain
  * map of 64x64 from scene to pixels 64.9 -> 61.6; other maps alone, the same) */
 constexpr int kBlock = 64;
@@ -1933,9 +1933,10 @@ static void* scratch_of(int dev)
 /*******************************************************************************
  * Host side
  ******************************************************************************/
-/* One of the two sets of buffers and streams that the calls of a context take
- * turns with (take_slot) */
-struct CallSlot {
+/* What one call in flight uses: partial sums, chunk counters and, if it draws
+ * ahead of the caller's stream (take_set), a stream. merged is recorded on the
+ * caller's stream behind the call. */
+struct CallSet {
   hipStream_t stream = nullptr;
   hipEvent_t drawn = nullptr, merged = nullptr;
   unsigned int* counters = nullptr;
@@ -1946,11 +1947,12 @@ struct CallSlot {
 
 struct htgx_wavefront_state {
   SceneF S;
-  CallSlot slots[2];
-  uint32_t next_slot = 0;
+  CallSet sets[2];
+  uint32_t last_set = 0;
   std::vector<void*> bufs;
   unsigned int* d_counters = nullptr;
   unsigned long long* d_trunc = nullptr; /* [2] queries cut short, Launch::trunc */
+  /* partial sums of the captured calls (with d_counters): what graphs read */
   void* d_partials = nullptr;
   size_t partials_cap = 0;
   uint32_t grid = 0;
@@ -1999,13 +2001,13 @@ static int upload_as_float(htgx_wavefront_state* st, Gptr<const T> dptr, size_t 
 }
 
 static void
-slot_free(CallSlot& s)
+set_free(CallSet& s)
 {
   if(s.stream) {
     (void)hipStreamSynchronize(s.stream);
-    if(s.used) (void)hipEventSynchronize(s.merged);
     (void)hipStreamDestroy(s.stream);
   }
+  if(s.used) (void)hipEventSynchronize(s.merged);
   if(s.drawn) (void)hipEventDestroy(s.drawn);
   if(s.merged) (void)hipEventDestroy(s.merged);
   if(s.counters) (void)hipFree(s.counters);
@@ -2015,7 +2017,7 @@ slot_free(CallSlot& s)
 static void
 wavefront_free(htgx_wavefront_state* st)
 {
-  for(CallSlot& s : st->slots) slot_free(s);
+  for(CallSet& s : st->sets) set_free(s);
   for(void* p : st->bufs) (void)hipFree(p);
   if(st->d_counters) (void)hipFree(st->d_counters);
   if(st->d_trunc) (void)hipFree(st->d_trunc);
@@ -2234,9 +2236,9 @@ spread_launch(uint32_t grid, Launch* P)
   return g;
 }
 
-/* Chunk partials a slot may hold: a larger map runs for seconds, to which its
- * last walks add little */
-constexpr size_t kMaxSlotPartials = size_t(1) << 30;
+/* Chunk partials of a call that may draw ahead: a larger map runs for seconds,
+ * to which its last walks add little */
+constexpr size_t kMaxAheadPartials = size_t(1) << 30;
 
 /* Whether a kernel on stream `own' is scheduled as one on `stream' is: same
  * priority, same compute units */
@@ -2259,26 +2261,65 @@ is_captured(hipStream_t stream)
   return cs != hipStreamCaptureStatusNone;
 }
 
-/* Make the partials of a slot those of the calls on the caller's stream, where
- * these are too few for a call under capture, which cannot allocate: a caller
- * that drew the map before it captures the call holds enough of them in a
- * slot. A graph may hold the former ones: they stay until the context goes. */
-static void
-take_over_partials(htgx_wavefront_state* st, size_t need)
+/* Whether the last call of a set is in flight. Asked in the relaxed mode: in
+ * another one the question would break a capture that another thread has begun
+ * in the global mode. */
+static bool
+is_pending(const CallSet& s)
 {
-  for(CallSlot& s : st->slots) {
-    if(s.cap < need) continue;
-    if(st->d_partials) st->bufs.push_back(st->d_partials);
-    st->d_partials = s.partials;
-    st->partials_cap = s.cap;
-    s.partials = nullptr;
-    s.cap = 0;
-    break;
-  }
+  if(!s.used) return false;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const bool done = hipEventQuery(s.merged) == hipSuccess;
+  if(!done) (void)hipGetLastError();
+  if(relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return !done;
 }
 
-/* The slot of a call on `stream' whose partials take `need' bytes, or null to
- * run the call on `stream' itself.
+/* Buffers for `need' bytes of partials in a set */
+static int
+size_set(CallSet& s, size_t need)
+{
+  if(!s.merged) HIP_OK(hipEventCreateWithFlags(&s.merged, hipEventDisableTiming));
+  if(!s.counters) HIP_OK(hipMalloc(&s.counters, kXcds * sizeof(unsigned int)));
+  if(need <= s.cap) return HTGX_OK;
+  if(s.partials) {
+    if(s.used) HIP_OK(hipEventSynchronize(s.merged));
+    HIP_OK(hipFree(s.partials));
+    s.partials = nullptr;
+    s.cap = 0;
+  }
+  HIP_OK(hipMalloc(&s.partials, need));
+  s.cap = need;
+  return HTGX_OK;
+}
+
+/* Partials of `need' bytes for a captured call, which the graph reads as long
+ * as the context lives. A call under capture cannot allocate: the partials are
+ * those of a set, which a caller that drew the map before it captures the call
+ * has large enough, and the set does without until its next call. */
+static int
+size_captured(htgx_wavefront_state* st, size_t need)
+{
+  if(need <= st->partials_cap) return HTGX_OK;
+  if(st->d_partials) {
+    st->bufs.push_back(st->d_partials);
+    st->d_partials = nullptr;
+    st->partials_cap = 0;
+  }
+  for(CallSet& s : st->sets) {
+    if(s.cap < need) continue;
+    std::swap(st->d_partials, s.partials);
+    std::swap(st->partials_cap, s.cap);
+    return HTGX_OK;
+  }
+  HIP_OK(hipMalloc(&st->d_partials, need)); /* a capture mode that allows it */
+  st->partials_cap = need;
+  return HTGX_OK;
+}
+
+/* The set of a call on `stream' whose partials take `need' bytes, and the
+ * stream it draws on.
  * A map's last walks leave most of the device idle: some 45 of the 140 ms of
  * 1024x1024x8 realisations of a shortwave image. A map's kernel reads the
  * context and writes partial sums, nothing of the caller's; only the merge
@@ -2286,64 +2327,43 @@ take_over_partials(htgx_wavefront_state* st, size_t need)
  * own, where it need not wait for the merge of the call before: the next
  * call's blocks take the compute units that the last walks leave. The merges
  * run on the caller's stream, each after its kernel, in the order of the
- * calls, and the accumulators are the same bit for bit. Two slots suffice, as
- * one kernel fills the device but for its end. Two slices of 8 realisations
- * of a 1024x1024 image: 273 -> 249 ms; four of 64x64 x 8: 100 -> 56; four of
- * 1024x1024 x 16: 898 -> 785. A call alone takes as long as before.
- * On the caller's stream as before: the null stream, which other streams wait
- * for; a stream being captured, whose graph must hold the whole call; one with
- * a priority or compute units of its own; a counted call, as the counters are
- * the context's; and where the buffers cannot be had. */
-static CallSlot*
-take_slot(htgx_ctx* ctx, size_t need, hipStream_t stream)
-{
-  htgx_wavefront_state* st = ctx->wf;
-  if(!stream || ctx->counting || need > kMaxSlotPartials) return nullptr;
-  if(is_captured(stream)) return nullptr;
-  int dev = 0;
-  if(hipGetDevice(&dev) != hipSuccess || dev != ctx->device) return nullptr;
-  CallSlot& s = st->slots[st->next_slot];
-  bool ok = (s.stream || hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) == hipSuccess)
-    && (s.drawn || hipEventCreateWithFlags(&s.drawn, hipEventDisableTiming) == hipSuccess)
-    && (s.merged || hipEventCreateWithFlags(&s.merged, hipEventDisableTiming) == hipSuccess)
-    && (s.counters || hipMalloc(&s.counters, kXcds * sizeof(unsigned int)) == hipSuccess)
-    && same_schedule(stream, s.stream);
-  if(ok && need > s.cap) {
-    if(s.partials) {
-      ok = (!s.used || hipEventSynchronize(s.merged) == hipSuccess) && hipFree(s.partials) == hipSuccess;
-      s.partials = nullptr;
-      s.cap = 0;
-    }
-    if((ok = ok && hipMalloc(&s.partials, need) == hipSuccess)) s.cap = need;
-  }
-  if(!ok) { (void)hipGetLastError(); return nullptr; }
-  st->next_slot ^= 1u;
-  return &s;
-}
-
-/* Launch parameters of one map; sizes the chunk partials of the context, or of
- * the slot that the call takes */
+ * calls, and the accumulators are the same bit for bit. Two sets suffice, as
+ * one kernel fills the device but for its end; the second is taken only while
+ * the call that uses the first is in flight, so a caller that waits for each
+ * call holds one. Two slices of 8 realisations of a 1024x1024 image: 273 ->
+ * 249 ms; four of 64x64 x 8: 100 -> 56; four of 1024x1024 x 16: 898 -> 785. A
+ * call alone takes as long as before.
+ * On the caller's stream, in the first set: the null stream, which other
+ * streams wait for; one with a priority or compute units of its own; a counted
+ * call, as the counters are the context's; and where the set or its stream
+ * cannot be had. */
 static int
-setup_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P, hipStream_t stream = nullptr,
-             CallSlot** slot = nullptr)
+take_set(htgx_ctx* ctx, size_t need, hipStream_t stream, CallSet** set, hipStream_t* draw)
 {
   htgx_wavefront_state* st = ctx->wf;
+  const bool pending[2] = {is_pending(st->sets[0]), is_pending(st->sets[1])};
+  int dev = 0;
+  uint32_t k = 0;
+  *draw = stream;
+  if(stream && !ctx->counting && need <= kMaxAheadPartials && hipGetDevice(&dev) == hipSuccess &&
+     dev == ctx->device) {
+    const uint32_t i = !pending[0] ? 0u : !pending[1] ? 1u : st->last_set ^ 1u;
+    CallSet& s = st->sets[i];
+    if((s.stream || hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) == hipSuccess) &&
+       (s.drawn || hipEventCreateWithFlags(&s.drawn, hipEventDisableTiming) == hipSuccess) &&
+       same_schedule(stream, s.stream) && size_set(s, need) == HTGX_OK) {
+      k = i;
+      *draw = s.stream;
+    } else {
+      (void)hipGetLastError();
+    }
+  }
+  CallSet& s = st->sets[k];
   int res;
-  if((res = fill_launch(ctx, M, planes, P)) != HTGX_OK) return res;
-  const size_t need = (size_t)P->ntiles * P->nsub * 64u * sizeof(htgx_mc_accum);
-  if(slot && (*slot = take_slot(ctx, need, stream))) {
-    P->counters = (*slot)->counters;
-    P->partials = (htgx_mc_accum*)(*slot)->partials;
-    return HTGX_OK;
-  }
-  if(need > st->partials_cap && is_captured(stream)) take_over_partials(st, need);
-  if(need > st->partials_cap) {
-    if(st->d_partials) { HIP_OK(hipFree(st->d_partials)); st->d_partials = nullptr; st->partials_cap = 0; }
-    HIP_OK(hipMalloc(&st->d_partials, need));
-    st->partials_cap = need;
-  }
-  P->counters = st->d_counters;
-  P->partials = (htgx_mc_accum*)st->d_partials;
+  if((res = size_set(s, need)) != HTGX_OK) return res;
+  if(pending[k]) HIP_OK(hipStreamWaitEvent(*draw, s.merged, 0)); /* its last call may be another stream's */
+  st->last_set = k;
+  *set = &s;
   return HTGX_OK;
 }
 
@@ -2365,20 +2385,26 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   if((res = wavefront_prepare(ctx)) != HTGX_OK) return res;
   htgx_wavefront_state* st = ctx->wf;
   Launch P;
-  if(planes > 1) {
-    /* a large image's channels one after the other, as they need a third of
-     * the partial sums then and have no use for a common tail */
-    res = fill_launch(ctx, M, planes, &P);
-    if(res != HTGX_OK || (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum) > kMaxPlanePartials)
-      return htgx_render_channels(ctx, M, planes, accum, stream, htgx_render_wavefront);
+  res = fill_launch(ctx, M, planes, &P);
+  const uint64_t need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
+  /* a large image's channels one after the other, as they need a third of the
+   * partial sums then and have no use for a common tail */
+  if(planes > 1 && (res != HTGX_OK || need > kMaxPlanePartials))
+    return htgx_render_channels(ctx, M, planes, accum, stream, htgx_render_wavefront);
+  if(res != HTGX_OK) return res;
+  CallSet* set = nullptr; /* of a captured call: none */
+  hipStream_t draw = stream;
+  if(is_captured(stream)) {
+    if((res = size_captured(st, need)) != HTGX_OK) return res;
+    P.counters = st->d_counters;
+    P.partials = (htgx_mc_accum*)st->d_partials;
+  } else {
+    if((res = take_set(ctx, need, stream, &set, &draw)) != HTGX_OK) return res;
+    P.counters = set->counters;
+    P.partials = (htgx_mc_accum*)set->partials;
   }
-  CallSlot* slot = nullptr;
-  if((res = setup_launch(ctx, M, planes, &P, stream, &slot)) != HTGX_OK) return res;
   const uint32_t grid = spread_launch(kernel_grid(st->grid, M.spectral_type, features(st->S, M),
                                                 (uint64_t)M.width * M.height * planes * M.spp), &P);
-  const hipStream_t draw = slot ? slot->stream : stream;
-  /* the slot's partials are free once its last call has merged them */
-  if(slot && slot->used) HIP_OK(hipStreamWaitEvent(draw, slot->merged, 0));
   zero_u32_kernel<<<1, 64, 0, draw>>>(P.counters, kXcds);
   HIP_OK(hipGetLastError());
   if(ctx->counting) {
@@ -2388,16 +2414,16 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   } else {
     if((res = launch<false>(st->S, M, P, grid, draw))) return res;
   }
-  if(slot) {
-    HIP_OK(hipEventRecord(slot->drawn, draw));
-    HIP_OK(hipStreamWaitEvent(stream, slot->drawn, 0));
+  if(draw != stream) {
+    HIP_OK(hipEventRecord(set->drawn, draw));
+    HIP_OK(hipStreamWaitEvent(stream, set->drawn, 0));
   }
   const uint32_t npix = M.width * M.height * planes;
   merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P, accum);
   HIP_OK(hipGetLastError());
-  if(slot) {
-    HIP_OK(hipEventRecord(slot->merged, stream));
-    slot->used = true;
+  if(set) {
+    HIP_OK(hipEventRecord(set->merged, stream));
+    set->used = true;
   }
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
   return HTGX_OK;
@@ -2607,16 +2633,22 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
     e.A.S = ctxs[i]->wf->S;
     e.A.M = Ms[i];
     e.accum = accums[i];
-    if((res = setup_launch(ctxs[i], Ms[i], 1, &e.A.P)) != HTGX_OK) return res;
+    if((res = fill_launch(ctxs[i], Ms[i], 1, &e.A.P)) != HTGX_OK) return res;
     e.A.P.stats = nullptr;
     e.A.P.counters = p->queues + (size_t)k * kXcds;
     e.A.P.exhausted = p->flags + k;
     e.A.P.done_count = p->flags + n + k;
     e.A.P.done_tick = p->ticks + k;
-    if(own_partials) {
+    const size_t np = (size_t)e.A.P.ntiles * e.A.P.nsub * 64u;
+    if(!own_partials) {
+      /* a set of the context, which no call in flight uses */
+      CallSet& set = ctxs[i]->wf->sets[0];
+      if((res = size_set(set, np * sizeof(htgx_mc_accum))) != HTGX_OK) return res;
+      if(set.used) HIP_OK(hipEventSynchronize(set.merged));
+      e.A.P.partials = (htgx_mc_accum*)set.partials;
+    } else {
       /* the context's partials and wavelength tables may be reallocated by
        * its next map: the plan keeps copies of its own */
-      const size_t np = (size_t)e.A.P.ntiles * e.A.P.nsub * 64u;
       if((res = plan_alloc(p, np, &e.A.P.partials.p))) return res;
       if(e.A.M.nwbands) {
         double *cdf = nullptr, *pdf = nullptr;
@@ -3001,7 +3033,7 @@ int htgx_debug_trace_segments_fp32_impl(htgx_ctx* ctx, const double* rays, uint3
 int htgx_wavefront_wait(htgx_ctx* ctx)
 {
   if(!ctx->wf) return HTGX_OK;
-  for(const CallSlot& s : ctx->wf->slots)
+  for(const CallSet& s : ctx->wf->sets)
     if(s.used) HIP_OK(hipEventSynchronize(s.merged));
   return HTGX_OK;
 }

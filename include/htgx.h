@@ -380,9 +380,9 @@ int htgx_draw_map
  * default stream). Asynchronous: the accumulators are updated in the order of
  * `stream'. On the FP32 solver and a stream other than NULL, the drawing that
  * fills a call's partial sums may run ahead of earlier work on `stream' (it
- * takes the device as an earlier call's last walks leave it), each context
- * holding two sets of partial sums for it; under stream capture and with
- * counters enabled it stays on `stream'. A call can be captured, in any
+ * takes the device as an earlier call's last walks leave it); a call made while
+ * one of the context is in flight takes a second set of partial sums for it.
+ * Under stream capture and with counters enabled it stays on `stream'. A call can be captured, in any
  * capture mode, once one of as many realisations has been made uncaptured on
  * any stream: it then allocates nothing. What the graph reads stays until the
  * context is destroyed. */

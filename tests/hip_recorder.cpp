@@ -7,7 +7,7 @@
  * through a wrong pointer.
  *
  * An event is pending from its record until its stream, a stream that waited
- * for it, the event or the device is synchronised. While a stream is captured
+ * for it, the device, it itself or a later one of its stream is synchronised. While a stream is captured
  * in another mode than relaxed, allocating and freeing fail as on a device. */
 #include <cstdint>
 #include <cstdio>
@@ -21,7 +21,7 @@
 namespace {
 enum { OK = 0, BAD_VALUE = 1, NO_MEMORY = 2, NOT_READY = 600, CAPTURING = 900 };
 struct Dim3 { uint32_t x, y, z; };
-struct Event { void* stream; bool pending; };
+struct Event { void* stream; bool pending; int order; };
 
 std::vector<std::string> log_;
 std::map<const void*, std::string> kernels;
@@ -163,6 +163,7 @@ int hipStreamWaitEvent(void* s, void* e, unsigned)
 int hipStreamGetPriority(void*, int* p) { *p = 0; return OK; }
 int hipExtStreamGetCUMask(void*, uint32_t n, uint32_t* m) { memset(m, 255, 4 * n); return OK; }
 int hipStreamIsCapturing(void* s, int* status) { *status = s && s == captured; return OK; }
+int hipThreadExchangeStreamCaptureMode(int*) { return OK; }
 int hipStreamBeginCapture(void* s, int mode) { captured = s; capture_mode = mode; return OK; }
 int hipStreamEndCapture(void*, void** g) { captured = nullptr; *g = malloc(16); return OK; }
 int hipGraphInstantiate(void** x, void*, void*, char*, size_t) { *x = malloc(16); return OK; }
@@ -171,7 +172,7 @@ int hipGraphDestroy(void* g) { free(g); return OK; }
 int hipGraphExecDestroy(void* x) { free(x); return OK; }
 int hipEventCreateWithFlags(void** e, unsigned)
 {
-  *e = new Event{nullptr, false};
+  *e = new Event{nullptr, false, 0};
   events.insert((Event*)*e);
   return OK;
 }
@@ -186,14 +187,16 @@ int hipEventDestroy(void* e)
 int hipEventRecord(void* e, void* s)
 {
   note("record stream %p event %p", s, e);
-  *(Event*)e = Event{s, true};
+  static int order = 0;
+  *(Event*)e = Event{s, true, ++order};
   return OK;
 }
 int hipEventQuery(void* e) { return ((Event*)e)->pending ? NOT_READY : OK; }
 int hipEventSynchronize(void* e)
 {
   note("sync event %p", e);
-  ((Event*)e)->pending = false;
+  for(Event* b : events)
+    if(b->stream == ((Event*)e)->stream && b->order <= ((Event*)e)->order) b->pending = false;
   return OK;
 }
 int hipEventElapsedTime(float* ms, void*, void*) { *ms = 1.f; return OK; }

@@ -1,6 +1,7 @@
 """FP32 calls in flight together, whose results are those of the same calls one
 at a time, bit for bit (the run times of the realisations aside)."""
 import ctypes as C
+import threading
 
 import pytest
 
@@ -65,4 +66,46 @@ def test_capture_after_calls_on_the_same_stream(mode, calls):
         h.hipGraphExecDestroy(run)
         h.hipGraphDestroy(graph)
         stream.destroy()
+    s.close()
+
+
+def test_calls_of_one_thread_while_another_captures(ctx):
+    """Calls in flight of one context while another thread captures, in global
+    mode, a call of another one."""
+    h = H.hip()
+    s = A.Synth(0, seed=7)
+    d = A.map_preset(0, width=40, height=40, spp=8, seed=3, solver=F.SOLVER_WAVEFRONT_FP32)
+    graph, run = C.c_void_p(), C.c_void_p()
+    acc, other = buffer(d), buffer(d)
+    streams = [H.Stream(), H.Stream()]
+    errors = []
+
+    def calls():
+        try:
+            for _ in range(3):
+                ctx.render_accum(d, other.address, streams[1].h.value)
+        except Exception as e:
+            errors.append(e)
+
+    with A.Context(s.scene_ptr) as captured:
+        captured.render_accum(d, acc.address, streams[0].h.value)
+        calls()  # the buffers of calls in flight exist
+        H.synchronize()
+        H.ok("hipStreamBeginCapture", h.hipStreamBeginCapture(streams[0].h, C.c_int(0)))
+        t = threading.Thread(target=calls)
+        t.start()
+        t.join()
+        captured.render_accum(d, acc.address, streams[0].h.value)
+        H.ok("hipStreamEndCapture", h.hipStreamEndCapture(streams[0].h, C.byref(graph)))
+        H.ok("hipGraphInstantiate", h.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+        for _ in range(3):
+            H.ok("hipGraphLaunch", h.hipGraphLaunch(run, streams[0].h))
+        H.synchronize()
+        assert not errors
+        assert same(acc, one_at_a_time(captured, [d] * 4), d)
+        assert same(other, one_at_a_time(ctx, [d] * 6), d)
+        h.hipGraphExecDestroy(run)
+        h.hipGraphDestroy(graph)
+        for st in streams:
+            st.destroy()
     s.close()

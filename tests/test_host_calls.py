@@ -143,3 +143,51 @@ for _ in range(3):
     lines = recorded(ctx.render_accum, big, ACCUM, 64)
     assert not held & {{l.split()[-1] for l in lines if l.startswith("free")}}, lines
 """)
+
+
+def test_a_caller_that_waits_uses_one_set_of_partials(run):
+    run("""
+R.hipStreamSynchronize.argtypes = [C.c_void_p]
+with A.Context(synth.scene_ptr) as ctx:
+    d = map_of(64, 48, 8)
+    ctx.render_accum(d, ACCUM, 64)
+    for _ in range(3):
+        R.hipStreamSynchronize(64)
+        lines = recorded(ctx.render_accum, d, ACCUM, 64)
+        assert not any(l.startswith(("malloc", "stream")) for l in lines), lines
+    # calls in flight take a second set, and no third one
+    held = R.recorder_live_bytes()
+    grown, draws = [], set()
+    for _ in range(4):
+        lines = recorded(ctx.render_accum, d, ACCUM, 64)
+        grown.append(R.recorder_live_bytes() - held)
+        draws |= {l.split()[-1] for l in lines if "wavefront_kernel" in l}
+        assert lines[-2].endswith("0x40") and "merge" in lines[-2], lines
+    assert 0 < grown[0] == grown[-1], grown
+    assert len(draws) == 2 and "0x40" not in draws, draws
+""")
+
+
+def test_calls_on_the_null_stream_and_counted_ones_draw_there(run):
+    run("""
+with A.Context(synth.scene_ptr) as ctx:
+    d = map_of(64, 48, 8)
+    ctx.render_accum(d, ACCUM, 64)
+    for stream, count in ((0, False), (64, True), (0, True)):
+        ctx.set_counting(count)
+        lines = recorded(ctx.render_accum, d, ACCUM, stream)
+        # after the call in flight, which uses the same partial sums
+        assert lines[0].startswith("wait"), lines
+        assert {int(l.split()[-1].replace("(nil)", "0"), 16) for l in lines if l.startswith("launch")} == {stream}
+""")
+
+
+def test_tuning_grows_the_partials_once_per_size(run):
+    """A trial is timed twice: the first pays for larger partial sums, the
+    second does not."""
+    run("""
+with A.Context(synth.scene_ptr) as ctx:
+    lines = recorded(ctx.autotune, map_of(256, 256, 64), 1e9)
+    sizes = [int(l.split()[1]) for l in lines if l.startswith("malloc") and int(l.split()[1]) > 1 << 21]
+    assert len(sizes) > 2 and len(set(sizes)) == len(sizes), sizes
+""")
