@@ -1943,6 +1943,7 @@ struct CallSet {
   void* partials = nullptr;
   size_t cap = 0;
   bool used = false; /* merged has been recorded */
+  hipStream_t last = nullptr; /* where */
 };
 
 struct htgx_wavefront_state {
@@ -2261,19 +2262,25 @@ is_captured(hipStream_t stream)
   return cs != hipStreamCaptureStatusNone;
 }
 
-/* Whether the last call of a set is in flight. Asked in the relaxed mode: in
- * another one the question would break a capture that another thread has begun
- * in the global mode. */
+/* The relaxed capture mode for the calling thread, in which it may ask about
+ * and wait for events: in another one that would break a capture that this
+ * thread, or in the global mode any other, has begun. */
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool set;
+  RelaxedCapture() : set(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+  ~RelaxedCapture() { if(set) (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+/* Whether the last call of a set is in flight */
 static bool
 is_pending(const CallSet& s)
 {
   if(!s.used) return false;
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-  const bool done = hipEventQuery(s.merged) == hipSuccess;
-  if(!done) (void)hipGetLastError();
-  if(relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-  return !done;
+  RelaxedCapture relaxed;
+  if(hipEventQuery(s.merged) == hipSuccess) return false;
+  (void)hipGetLastError();
+  return true;
 }
 
 /* Buffers for `need' bytes of partials in a set */
@@ -2299,7 +2306,7 @@ size_set(CallSet& s, size_t need)
  * those of a set, which a caller that drew the map before it captures the call
  * has large enough, and the set does without until its next call. */
 static int
-size_captured(htgx_wavefront_state* st, size_t need)
+size_captured(htgx_wavefront_state* st, size_t need, hipStream_t stream)
 {
   if(need <= st->partials_cap) return HTGX_OK;
   if(st->d_partials) {
@@ -2309,6 +2316,10 @@ size_captured(htgx_wavefront_state* st, size_t need)
   }
   for(CallSet& s : st->sets) {
     if(s.cap < need) continue;
+    if(s.used && s.last != stream) { /* no replay waits for the set's last call */
+      RelaxedCapture relaxed;
+      HIP_OK(hipEventSynchronize(s.merged));
+    }
     std::swap(st->d_partials, s.partials);
     std::swap(st->partials_cap, s.cap);
     return HTGX_OK;
@@ -2395,7 +2406,7 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   CallSet* set = nullptr; /* of a captured call: none */
   hipStream_t draw = stream;
   if(is_captured(stream)) {
-    if((res = size_captured(st, need)) != HTGX_OK) return res;
+    if((res = size_captured(st, need, stream)) != HTGX_OK) return res;
     P.counters = st->d_counters;
     P.partials = (htgx_mc_accum*)st->d_partials;
   } else {
@@ -2424,6 +2435,7 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   if(set) {
     HIP_OK(hipEventRecord(set->merged, stream));
     set->used = true;
+    set->last = stream;
   }
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
   return HTGX_OK;

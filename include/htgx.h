@@ -382,10 +382,12 @@ int htgx_draw_map
  * fills a call's partial sums may run ahead of earlier work on `stream' (it
  * takes the device as an earlier call's last walks leave it); a call made while
  * one of the context is in flight takes a second set of partial sums for it.
- * Under stream capture and with counters enabled it stays on `stream'. A call can be captured, in any
- * capture mode, once one of as many realisations has been made uncaptured on
- * any stream: it then allocates nothing. What the graph reads stays until the
- * context is destroyed. */
+ * Under stream capture and with counters enabled it stays on `stream'. A call
+ * can be captured, in any capture mode, once one like it has been made
+ * uncaptured on any stream: it then allocates nothing. The graph's partial sums
+ * stay until the context is destroyed; the wavelength tables of a band or CIE
+ * map until the context draws a map with others, after which the graph must not
+ * be replayed. */
 int htgx_render_accum
   (struct htgx_ctx* ctx,
    const struct htgx_map_desc* desc,

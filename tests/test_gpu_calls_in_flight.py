@@ -39,19 +39,20 @@ def test_the_wavelength_range_changes_between_calls(ctx, spectral):
 
 
 @pytest.mark.parametrize("mode", [0, 1])  # global, thread-local: both refuse allocations
-@pytest.mark.parametrize("calls", [1, 3])
-def test_capture_after_calls_on_the_same_stream(mode, calls):
+@pytest.mark.parametrize("calls,elsewhere", [(1, False), (3, False), (2, True)])
+def test_capture_after_calls_on_a_stream(mode, calls, elsewhere):
     """From a new context, calls on a stream, then the capture of one like
-    them on it, replayed with larger ones in between."""
+    them, on it or on another one, replayed with larger ones in between."""
     h = H.hip()
     s = A.Synth(0, seed=6)
     d, e = (A.map_preset(0, width=w, height=w, spp=8, seed=3, solver=F.SOLVER_WAVEFRONT_FP32)
             for w in (40, 64))
     graph, run = C.c_void_p(), C.c_void_p()
-    acc, other, stream = buffer(d), buffer(e), H.Stream()
+    acc, before, other, stream = buffer(d), buffer(d), buffer(e), H.Stream()
+    first = H.Stream() if elsewhere else stream
     with A.Context(s.scene_ptr) as ctx:
         for _ in range(calls):
-            ctx.render_accum(d, acc.address, stream.h.value)
+            ctx.render_accum(d, before.address, first.h.value)
         H.ok("hipStreamBeginCapture", h.hipStreamBeginCapture(stream.h, C.c_int(mode)))
         ctx.render_accum(d, acc.address, stream.h.value)
         H.ok("hipStreamEndCapture", h.hipStreamEndCapture(stream.h, C.byref(graph)))
@@ -60,8 +61,9 @@ def test_capture_after_calls_on_the_same_stream(mode, calls):
             H.ok("hipGraphLaunch", h.hipGraphLaunch(run, stream.h))
             ctx.render_accum(e, other.address, stream.h.value)
         H.ok("hipGraphLaunch", h.hipGraphLaunch(run, stream.h))
-        stream.synchronize()
-        assert same(acc, one_at_a_time(ctx, [d] * (calls + 4)), d)
+        H.synchronize()
+        assert same(before, one_at_a_time(ctx, [d] * calls), d)
+        assert same(acc, one_at_a_time(ctx, [d] * 4), d)
         assert same(other, one_at_a_time(ctx, [e] * 3), e)
         h.hipGraphExecDestroy(run)
         h.hipGraphDestroy(graph)
