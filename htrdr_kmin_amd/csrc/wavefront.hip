@@ -1943,7 +1943,6 @@ struct CallSet {
   void* partials = nullptr;
   size_t cap = 0;
   bool used = false; /* merged has been recorded */
-  hipStream_t last = nullptr; /* where */
 };
 
 struct htgx_wavefront_state {
@@ -2262,12 +2261,11 @@ is_captured(hipStream_t stream)
   return cs != hipStreamCaptureStatusNone;
 }
 
-/* The relaxed capture mode for the calling thread, in which it may ask about
- * and wait for events: in another one that would break a capture that this
- * thread, or in the global mode any other, has begun. */
+/* The relaxed capture mode for the calling thread: buffers of the context's own
+ * may be had and its calls asked about in it while this thread, or any other in the global mode, captures */
 struct RelaxedCapture {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  bool set;
+  const bool set;
   RelaxedCapture() : set(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
   ~RelaxedCapture() { if(set) (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
@@ -2277,7 +2275,6 @@ static bool
 is_pending(const CallSet& s)
 {
   if(!s.used) return false;
-  RelaxedCapture relaxed;
   if(hipEventQuery(s.merged) == hipSuccess) return false;
   (void)hipGetLastError();
   return true;
@@ -2301,30 +2298,17 @@ size_set(CallSet& s, size_t need)
   return HTGX_OK;
 }
 
-/* Partials of `need' bytes for a captured call, which the graph reads as long
- * as the context lives. A call under capture cannot allocate: the partials are
- * those of a set, which a caller that drew the map before it captures the call
- * has large enough, and the set does without until its next call. */
+/* Partials of `need' bytes for a captured call. The graph reads them as long as
+ * the context lives. */
 static int
-size_captured(htgx_wavefront_state* st, size_t need, hipStream_t stream)
+size_captured(htgx_wavefront_state* st, size_t need)
 {
   if(need <= st->partials_cap) return HTGX_OK;
-  if(st->d_partials) {
-    st->bufs.push_back(st->d_partials);
-    st->d_partials = nullptr;
-    st->partials_cap = 0;
-  }
-  for(CallSet& s : st->sets) {
-    if(s.cap < need) continue;
-    if(s.used && s.last != stream) { /* no replay waits for the set's last call */
-      RelaxedCapture relaxed;
-      HIP_OK(hipEventSynchronize(s.merged));
-    }
-    std::swap(st->d_partials, s.partials);
-    std::swap(st->partials_cap, s.cap);
-    return HTGX_OK;
-  }
-  HIP_OK(hipMalloc(&st->d_partials, need)); /* a capture mode that allows it */
+  RelaxedCapture relaxed;
+  void* p = nullptr;
+  HIP_OK(hipMalloc(&p, need));
+  if(st->d_partials) st->bufs.push_back(st->d_partials);
+  st->d_partials = p;
   st->partials_cap = need;
   return HTGX_OK;
 }
@@ -2352,6 +2336,7 @@ static int
 take_set(htgx_ctx* ctx, size_t need, hipStream_t stream, CallSet** set, hipStream_t* draw)
 {
   htgx_wavefront_state* st = ctx->wf;
+  RelaxedCapture relaxed;
   const bool pending[2] = {is_pending(st->sets[0]), is_pending(st->sets[1])};
   int dev = 0;
   uint32_t k = 0;
@@ -2406,7 +2391,7 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   CallSet* set = nullptr; /* of a captured call: none */
   hipStream_t draw = stream;
   if(is_captured(stream)) {
-    if((res = size_captured(st, need, stream)) != HTGX_OK) return res;
+    if((res = size_captured(st, need)) != HTGX_OK) return res;
     P.counters = st->d_counters;
     P.partials = (htgx_mc_accum*)st->d_partials;
   } else {
@@ -2435,7 +2420,6 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   if(set) {
     HIP_OK(hipEventRecord(set->merged, stream));
     set->used = true;
-    set->last = stream;
   }
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
   return HTGX_OK;

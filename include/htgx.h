@@ -384,10 +384,10 @@ int htgx_draw_map
  * one of the context is in flight takes a second set of partial sums for it.
  * Under stream capture and with counters enabled it stays on `stream'. A call
  * can be captured, in any capture mode, once one like it has been made
- * uncaptured on any stream: it then allocates nothing. The graph's partial sums
- * stay until the context is destroyed; the wavelength tables of a band or CIE
- * map until the context draws a map with others, after which the graph must not
- * be replayed. */
+ * uncaptured. The graphs of a context share partial sums that no other call
+ * uses (replay them one after the other) and that stay until the context is
+ * destroyed; the wavelength tables of a band or CIE map stay until the context
+ * draws a map with others, after which the graph must not be replayed. */
 int htgx_render_accum
   (struct htgx_ctx* ctx,
    const struct htgx_map_desc* desc,

@@ -16,6 +16,7 @@
 #include <map>
 #include <set>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -163,7 +164,11 @@ int hipStreamWaitEvent(void* s, void* e, unsigned)
 int hipStreamGetPriority(void*, int* p) { *p = 0; return OK; }
 int hipExtStreamGetCUMask(void*, uint32_t n, uint32_t* m) { memset(m, 255, 4 * n); return OK; }
 int hipStreamIsCapturing(void* s, int* status) { *status = s && s == captured; return OK; }
-int hipThreadExchangeStreamCaptureMode(int*) { return OK; }
+int hipThreadExchangeStreamCaptureMode(int* mode)
+{
+  std::swap(*mode, capture_mode);
+  return OK;
+}
 int hipStreamBeginCapture(void* s, int mode) { captured = s; capture_mode = mode; return OK; }
 int hipStreamEndCapture(void*, void** g) { captured = nullptr; *g = malloc(16); return OK; }
 int hipGraphInstantiate(void** x, void*, void*, char*, size_t) { *x = malloc(16); return OK; }
