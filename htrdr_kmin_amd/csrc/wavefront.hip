@@ -2318,20 +2318,24 @@ size_captured(htgx_wavefront_state* st, size_t need)
  * A map's last walks leave most of the device idle: some 45 of the 140 ms of
  * 1024x1024x8 realisations of a shortwave image. A map's kernel reads the
  * context and writes partial sums, nothing of the caller's; only the merge
- * touches the accumulators. So the kernel runs on a stream of the context's
- * own, where it need not wait for the merge of the call before: the next
- * call's blocks take the compute units that the last walks leave. The merges
- * run on the caller's stream, each after its kernel, in the order of the
- * calls, and the accumulators are the same bit for bit. Two sets suffice, as
- * one kernel fills the device but for its end; the second is taken only while
- * the call that uses the first is in flight, so a caller that waits for each
- * call holds one. Two slices of 8 realisations of a 1024x1024 image: 273 ->
- * 249 ms; four of 64x64 x 8: 100 -> 56; four of 1024x1024 x 16: 898 -> 785. A
- * call alone takes as long as before.
- * On the caller's stream, in the first set: the null stream, which other
- * streams wait for; one with a priority or compute units of its own; a counted
- * call, as the counters are the context's; and where the set or its stream
- * cannot be had. */
+ * touches the accumulators. So a call made while another of its context is in
+ * flight draws on a stream of the context's own, where it need not wait for the
+ * merge of the call before: its blocks take the compute units that the last
+ * walks leave. The merges run on the caller's stream, each after its kernel, in
+ * the order of the calls, and the accumulators are the same bit for bit. Two
+ * sets suffice, as one kernel fills the device but for its end; a caller that
+ * waits for each call holds one. Two slices of 8 realisations of a 1024x1024
+ * image: 273 -> 249 ms; four of 64x64 x 8: 100 -> 56; four of 1024x1024 x 16:
+ * 898 -> 785. A call alone takes as long as before.
+ * A call with no other in flight draws on the caller's stream: a process has
+ * few hardware queues, and where streams share one, a draw can come to wait
+ * behind another context's merge, which waits for its own draw. A map of 64x64
+ * x 32 on each of 2, 3 and 6 contexts and streams at a time, by the queues they
+ * come to share: 31-55, 35-57 and 60-77 ms; with draws on streams of the
+ * contexts' own, 32-54, 36-82 and 75-86.
+ * So do calls on the null stream, which other streams wait for; on one with a
+ * priority or compute units of its own; counted ones, as the counters are the
+ * context's; and those whose set or stream cannot be had. */
 static int
 take_set(htgx_ctx* ctx, size_t need, hipStream_t stream, CallSet** set, hipStream_t* draw)
 {
@@ -2341,8 +2345,8 @@ take_set(htgx_ctx* ctx, size_t need, hipStream_t stream, CallSet** set, hipStrea
   int dev = 0;
   uint32_t k = 0;
   *draw = stream;
-  if(stream && !ctx->counting && need <= kMaxAheadPartials && hipGetDevice(&dev) == hipSuccess &&
-     dev == ctx->device) {
+  if((pending[0] || pending[1]) && stream && !ctx->counting && need <= kMaxAheadPartials &&
+     hipGetDevice(&dev) == hipSuccess && dev == ctx->device) {
     const uint32_t i = !pending[0] ? 0u : !pending[1] ? 1u : st->last_set ^ 1u;
     CallSet& s = st->sets[i];
     if((s.stream || hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) == hipSuccess) &&

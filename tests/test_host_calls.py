@@ -194,3 +194,23 @@ with A.Context(synth.scene_ptr) as ctx:
     sizes = [int(l.split()[1]) for l in lines if l.startswith("malloc") and int(l.split()[1]) > 1 << 21]
     assert len(sizes) > 2 and len(set(sizes)) == len(sizes), sizes
 """)
+
+
+def test_a_call_with_no_other_in_flight_draws_on_the_callers_stream(run):
+    run("""
+R.hipStreamSynchronize.argtypes = [C.c_void_p]
+
+def draws_on(ctx, stream):
+    lines = recorded(ctx.render_accum, map_of(64, 48, 8), ACCUM, stream)
+    draw = [l for l in lines if "wavefront_kernel" in l]
+    assert len(draw) == 1
+    return draw[0].endswith(hex(stream))
+
+with A.Context(synth.scene_ptr) as a, A.Context(synth.scene_ptr) as b:
+    b.wavefront_params()  # its set-up waits for the device
+    for k in range(2):
+        assert [draws_on(a, 64) for _ in range(4)] == [True, False, False, False]
+        assert [draws_on(b, 80) for _ in range(2)] == [True, False]
+        for stream in (64, 80):
+            R.hipStreamSynchronize(stream)
+""")
