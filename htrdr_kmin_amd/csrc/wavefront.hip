@@ -1811,6 +1811,13 @@ batch_merge_kernel(const BatchScene* scenes)
   if(p < P.width * P.height) merge_pixel(P, B.accum, p);
 }
 
+/* A call's number to host memory, behind its merge */
+__global__ void
+done_kernel(uint32_t* done, uint32_t call)
+{
+  __hip_atomic_store(done, call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 /* FP16 bits of a bound of v >= 0 in units of scale >= v, rounded down (lower
  * bound) or up (upper bound) so that the decoded value, FP32
  * half_bits_to_float(b) * scale as load_leaf computes it, never lies inside
@@ -1942,7 +1949,10 @@ struct CallSet {
   unsigned int* counters = nullptr;
   void* partials = nullptr;
   size_t cap = 0;
-  bool used = false; /* merged has been recorded */
+  /* number of the set's last call and, in host memory, of its last one done: an
+   * event cannot be asked about while the stream it was recorded on is captured */
+  uint32_t call = 0;
+  uint32_t* done = nullptr;
 };
 
 struct htgx_wavefront_state {
@@ -2000,6 +2010,13 @@ static int upload_as_float(htgx_wavefront_state* st, Gptr<const T> dptr, size_t 
   return upload_f(st, f, out);
 }
 
+/* Whether the last call of a set is in flight */
+static bool
+is_pending(const CallSet& s)
+{
+  return s.done && __atomic_load_n(s.done, __ATOMIC_ACQUIRE) != s.call;
+}
+
 static void
 set_free(CallSet& s)
 {
@@ -2007,11 +2024,12 @@ set_free(CallSet& s)
     (void)hipStreamSynchronize(s.stream);
     (void)hipStreamDestroy(s.stream);
   }
-  if(s.used) (void)hipEventSynchronize(s.merged);
+  if(is_pending(s)) (void)hipEventSynchronize(s.merged);
   if(s.drawn) (void)hipEventDestroy(s.drawn);
   if(s.merged) (void)hipEventDestroy(s.merged);
   if(s.counters) (void)hipFree(s.counters);
   if(s.partials) (void)hipFree(s.partials);
+  if(s.done) (void)hipHostFree(s.done);
 }
 
 static void
@@ -2157,6 +2175,10 @@ wavefront_build(htgx_ctx* ctx, htgx_wavefront_state* st)
 
   HIP_OK(hipMalloc(&st->d_counters, kXcds * sizeof(unsigned int)));
   HIP_OK(hipMalloc(&st->d_trunc, 2 * sizeof(unsigned long long)));
+  for(CallSet& s : st->sets) {
+    HIP_OK(hipHostMalloc((void**)&s.done, sizeof(uint32_t), hipHostMallocDefault));
+    *s.done = 0;
+  }
   if((res = scratch_lookup()) != HTGX_OK) return res;
   const unsigned long long none[2] = {0, 0};
   HIP_OK(hipMemcpy(st->d_trunc, none, sizeof(none), hipMemcpyHostToDevice));
@@ -2262,23 +2284,13 @@ is_captured(hipStream_t stream)
 }
 
 /* The relaxed capture mode for the calling thread: buffers of the context's own
- * may be had and its calls asked about in it while this thread, or any other in the global mode, captures */
+ * may be had in it while this thread, or any other in the global mode, captures */
 struct RelaxedCapture {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   const bool set;
   RelaxedCapture() : set(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
   ~RelaxedCapture() { if(set) (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
-
-/* Whether the last call of a set is in flight */
-static bool
-is_pending(const CallSet& s)
-{
-  if(!s.used) return false;
-  if(hipEventQuery(s.merged) == hipSuccess) return false;
-  (void)hipGetLastError();
-  return true;
-}
 
 /* Buffers for `need' bytes of partials in a set */
 static int
@@ -2288,7 +2300,7 @@ size_set(CallSet& s, size_t need)
   if(!s.counters) HIP_OK(hipMalloc(&s.counters, kXcds * sizeof(unsigned int)));
   if(need <= s.cap) return HTGX_OK;
   if(s.partials) {
-    if(s.used) HIP_OK(hipEventSynchronize(s.merged));
+    if(is_pending(s)) HIP_OK(hipEventSynchronize(s.merged));
     HIP_OK(hipFree(s.partials));
     s.partials = nullptr;
     s.cap = 0;
@@ -2422,8 +2434,10 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P, accum);
   HIP_OK(hipGetLastError());
   if(set) {
+    done_kernel<<<1, 1, 0, stream>>>(set->done, set->call + 1u);
+    HIP_OK(hipGetLastError());
+    ++set->call;
     HIP_OK(hipEventRecord(set->merged, stream));
-    set->used = true;
   }
   ctx->last_nrealisations = (uint64_t)npix * M.spp;
   return HTGX_OK;
@@ -2644,7 +2658,7 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
       /* a set of the context, which no call in flight uses */
       CallSet& set = ctxs[i]->wf->sets[0];
       if((res = size_set(set, np * sizeof(htgx_mc_accum))) != HTGX_OK) return res;
-      if(set.used) HIP_OK(hipEventSynchronize(set.merged));
+      if(is_pending(set)) HIP_OK(hipEventSynchronize(set.merged));
       e.A.P.partials = (htgx_mc_accum*)set.partials;
     } else {
       /* the context's partials and wavelength tables may be reallocated by
@@ -3034,7 +3048,7 @@ int htgx_wavefront_wait(htgx_ctx* ctx)
 {
   if(!ctx->wf) return HTGX_OK;
   for(const CallSet& s : ctx->wf->sets)
-    if(s.used) HIP_OK(hipEventSynchronize(s.merged));
+    if(is_pending(s)) HIP_OK(hipEventSynchronize(s.merged));
   return HTGX_OK;
 }
 

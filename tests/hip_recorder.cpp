@@ -6,8 +6,8 @@
  * allocation and under stream capture, and without a kernel that would write
  * through a wrong pointer.
  *
- * An event is pending from its record until its stream, a stream that waited
- * for it, the device, it itself or a later one of its stream is synchronised. While a stream is captured
+ * What a stream was given is done once it, a stream that waited for it, an event
+ * recorded behind it or the device is synchronised. While a stream is captured
  * in another mode than relaxed, allocating and freeing fail as on a device. */
 #include <cstdint>
 #include <cstdio>
@@ -20,15 +20,18 @@
 #include <vector>
 
 namespace {
-enum { OK = 0, BAD_VALUE = 1, NO_MEMORY = 2, NOT_READY = 600, CAPTURING = 900 };
+enum { OK = 0, BAD_VALUE = 1, NO_MEMORY = 2, CAPTURING = 900 };
 struct Dim3 { uint32_t x, y, z; };
-struct Event { void* stream; bool pending; int order; };
+struct Event { void* stream; int order; };
 
 std::vector<std::string> log_;
 std::map<const void*, std::string> kernels;
 std::map<void*, size_t> live;
 std::map<void*, std::set<Event*>> waits; /* per stream */
-std::set<Event*> events;
+/* calls' numbers that a stream is to write to host memory */
+struct Done { void* stream; uint32_t* to; uint32_t value; int order; };
+std::vector<Done> done;
+int order = 0;
 size_t fail_above = SIZE_MAX;
 int fail_in = 0; /* the allocation to fail: 1 the next */
 void* captured = nullptr;
@@ -42,6 +45,13 @@ template<class... A> void note(const char* fmt, A... a)
   char line[256];
   snprintf(line, sizeof(line), fmt, a...);
   log_.push_back(line);
+}
+
+/* what a stream (or all) was given up to `last' is done */
+void finish(void* s, bool all, int last)
+{
+  for(auto& d : done)
+    if(d.to && (all || d.stream == s) && d.order <= last) { *d.to = d.value; d.to = nullptr; }
 }
 
 bool refused() { return captured && capture_mode != 2; }
@@ -85,8 +95,10 @@ int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* sh, void** s)
   *g = grid_; *b = block_; *sh = shared_; *s = stream_;
   return OK;
 }
-int hipLaunchKernel(const void* f, Dim3 g, Dim3, void**, size_t, void* s)
+int hipLaunchKernel(const void* f, Dim3 g, Dim3, void** args, size_t, void* s)
 {
+  if(kernels[f].find("done_kernel") != std::string::npos)
+    done.push_back({s, *(uint32_t**)args[0], *(uint32_t*)args[1], ++order});
   note("launch %.160s grid %u stream %p", kernels[f].c_str(), g.x, s);
   return OK;
 }
@@ -111,6 +123,8 @@ int hipFree(void* p)
   free(p);
   return OK;
 }
+int hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(n, 1); return OK; }
+int hipHostFree(void* p) { free(p); return OK; }
 int hipMemcpy(void* d, const void* s, size_t n, int)
 {
   if(refused()) return CAPTURING;
@@ -142,7 +156,7 @@ int hipGetSymbolAddress(void** p, const void*)
 int hipDeviceSynchronize(void)
 {
   note("sync device%s", "");
-  for(Event* e : events) e->pending = false;
+  finish(nullptr, true, order);
   return OK;
 }
 int hipStreamCreateWithFlags(void** s, unsigned) { *s = malloc(16); note("stream %p", *s); return OK; }
@@ -150,8 +164,8 @@ int hipStreamDestroy(void* s) { free(s); return OK; }
 int hipStreamSynchronize(void* s)
 {
   note("sync stream %p", s);
-  for(Event* e : events) if(e->stream == s) e->pending = false;
-  for(Event* e : waits[s]) e->pending = false;
+  finish(s, false, order);
+  for(Event* e : waits[s]) finish(e->stream, false, e->order);
   waits[s].clear();
   return OK;
 }
@@ -177,31 +191,26 @@ int hipGraphDestroy(void* g) { free(g); return OK; }
 int hipGraphExecDestroy(void* x) { free(x); return OK; }
 int hipEventCreateWithFlags(void** e, unsigned)
 {
-  *e = new Event{nullptr, false, 0};
-  events.insert((Event*)*e);
+  *e = new Event{nullptr, 0};
   return OK;
 }
 int hipEventCreate(void** e) { return hipEventCreateWithFlags(e, 0); }
 int hipEventDestroy(void* e)
 {
   for(auto& w : waits) w.second.erase((Event*)e);
-  events.erase((Event*)e);
   delete (Event*)e;
   return OK;
 }
 int hipEventRecord(void* e, void* s)
 {
   note("record stream %p event %p", s, e);
-  static int order = 0;
-  *(Event*)e = Event{s, true, ++order};
+  *(Event*)e = Event{s, ++order};
   return OK;
 }
-int hipEventQuery(void* e) { return ((Event*)e)->pending ? NOT_READY : OK; }
 int hipEventSynchronize(void* e)
 {
   note("sync event %p", e);
-  for(Event* b : events)
-    if(b->stream == ((Event*)e)->stream && b->order <= ((Event*)e)->order) b->pending = false;
+  finish(((Event*)e)->stream, false, ((Event*)e)->order);
   return OK;
 }
 int hipEventElapsedTime(float* ms, void*, void*) { *ms = 1.f; return OK; }

@@ -111,3 +111,29 @@ def test_calls_of_one_thread_while_another_captures(ctx):
         for st in streams:
             st.destroy()
     s.close()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_calls_on_a_stream_while_one_used_before_is_captured(ctx, mode):
+    """Calls of a context leave alone the capture of a stream that it drew on
+    before."""
+    h = H.hip()
+    h.hipMemcpyAsync.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p]
+    d = A.map_preset(0, width=40, height=40, spp=8, seed=3, solver=F.SOLVER_WAVEFRONT_FP32)
+    graph = C.c_void_p()
+    acc, other, copy = buffer(d), buffer(d), buffer(d)
+    streams = [H.Stream(), H.Stream()]
+    for _ in range(2):  # in flight together: both sets of buffers exist
+        ctx.render_accum(d, acc.address, streams[0].h.value)
+    H.synchronize()
+    H.ok("hipStreamBeginCapture", h.hipStreamBeginCapture(streams[0].h, C.c_int(mode)))
+    for _ in range(3):
+        ctx.render_accum(d, other.address, streams[1].h.value)
+    H.ok("hipMemcpyAsync", h.hipMemcpyAsync(copy.ptr, acc.ptr, acc.nbytes, 3, streams[0].h))
+    H.ok("hipStreamEndCapture", h.hipStreamEndCapture(streams[0].h, C.byref(graph)))
+    h.hipGraphDestroy(graph)
+    H.synchronize()
+    assert same(acc, one_at_a_time(ctx, [d] * 2), d)
+    assert same(other, one_at_a_time(ctx, [d] * 3), d)
+    for st in streams:
+        st.destroy()
