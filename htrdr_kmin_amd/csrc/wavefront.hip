@@ -1905,8 +1905,13 @@ int launch(const SceneF& S, const DevMap& M, const Launch& P, uint32_t grid, hip
  * on and held until the process ends, instead of memory the call allocates.
  * Every call on a GPU shares that GPU's copy: calls that overlap on one GPU
  * race. */
-constexpr size_t kScratchBytes = (size_t)64 << 20;
+constexpr size_t kScratchBytes = (size_t)96 << 20;
 constexpr size_t kScratchHead = 256;
+/* The largest map it takes, in chunks of the chunk-size parameter. A small map
+ * has more, smaller chunks (fill_launch), which the scratch holds at the default
+ * parameter but for odd multiples of 3 realisations (256x256 x 16 and x 20: 41
+ * and 42 ms in 64 MiB, full chunks instead; 29 and 33). */
+constexpr uint64_t kNoallocChunks = ((64ull << 20) - kScratchHead) / sizeof(htgx_mc_accum);
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 /* Device address of each GPU's copy, looked up once per device (at the FP32
@@ -2198,6 +2203,15 @@ wavefront_build(htgx_ctx* ctx, htgx_wavefront_state* st)
 
 constexpr uint32_t kChunksPerLane = 4;
 
+/* The largest chunk of a map: a divisor of spp not above the parameter */
+static uint32_t
+full_chunk(const htgx_wavefront_state* st, uint32_t spp)
+{
+  uint32_t K = std::min(st->K, spp);
+  while(spp % K) --K;
+  return K;
+}
+
 /* Launch parameters of one map, its partials and counters aside */
 static int
 fill_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
@@ -2214,7 +2228,7 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
    * the launch parameters other than the chunk size. */
   const uint64_t nreal = (uint64_t)P->ntiles * 64u * M.spp;
   const uint64_t most = nreal / ((uint64_t)kChunksPerLane * st->grid_max * kUnit * kBlock);
-  uint32_t K = (uint32_t)std::min<uint64_t>(std::min(st->K, M.spp), std::max<uint64_t>(1, most));
+  uint32_t K = std::min(full_chunk(st, M.spp), (uint32_t)std::min<uint64_t>(M.spp, std::max<uint64_t>(1, most)));
   while(M.spp % K) --K;
   P->K = K;
   P->nsub = M.spp / K;
@@ -2443,6 +2457,42 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
   return HTGX_OK;
 }
 
+/* Chunks [first, first + P.nsub) of every pixel, in the static scratch at
+ * `base', added to the accumulators */
+static int
+launch_noalloc(htgx_ctx* ctx, const DevMap& M, Launch P, uint32_t first, bool first_launch,
+               unsigned char* base, htgx_mc_accum* accum, hipStream_t stream)
+{
+  htgx_wavefront_state* st = ctx->wf;
+  int res;
+  const uint32_t npix = M.width * M.height * P.planes;
+  P.spp_offset += first * P.K;
+  P.nvalid = npix * P.nsub;
+  P.counters = (unsigned int*)base;
+  P.partials = (htgx_mc_accum*)(base + kScratchHead);
+  const uint32_t grid = spread_launch(kernel_grid(st->grid, M.spectral_type, features(st->S, M),
+                                                (uint64_t)npix * P.nsub * P.K), &P);
+  /* fill kernels, no memset: the call may be captured in a graph */
+  zero_u32_kernel<<<1, 64, 0, stream>>>(P.counters, kXcds);
+  HIP_OK(hipGetLastError());
+  if(ctx->counting) {
+    if(first_launch) zero_u64_kernel<<<1, 64, 0, stream>>>(ctx->d_counters, HTGX_NSTATS);
+    HIP_OK(hipGetLastError());
+    if((res = launch<true>(st->S, M, P, grid, stream))) return res;
+  } else {
+    if((res = launch<false>(st->S, M, P, grid, stream))) return res;
+  }
+  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P, accum);
+  HIP_OK(hipGetLastError());
+  return HTGX_OK;
+}
+
+/* The chunks are those of htgx_render_wavefront, so that the sums are the same
+ * bit for bit. Where the scratch does not hold all of them -- of an image's
+ * planes, or of a small map's small chunks -- they go through it a range of each
+ * pixel's chunks at a time, and plane by plane if one chunk of each pixel is too
+ * many: the merge adds to the accumulators in chunk order, in one launch or in
+ * several. */
 int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_mc_accum* accum,
                                   hipStream_t stream)
 {
@@ -2455,45 +2505,29 @@ int htgx_render_wavefront_noalloc(htgx_ctx* ctx, const DevMap& M, uint32_t plane
   if(!base) return HTGX_BAD_OP;
   Launch P;
   if((res = fill_launch(ctx, M, planes, &P)) != HTGX_OK) return res;
-  uint64_t need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
-  if(need > kScratchBytes - kScratchHead && P.K < st->K) {
-    /* small chunks were preferred: the full ones need less scratch */
-    uint32_t K = std::min(st->K, M.spp);
-    while(M.spp % K) --K;
-    P.K = K;
-    P.nsub = M.spp / K;
-    P.nvalid = (uint32_t)((uint64_t)M.width * M.height * planes * P.nsub);
-    need = (uint64_t)P.ntiles * P.nsub * 64u * sizeof(htgx_mc_accum);
-  }
-  if(need > kScratchBytes - kScratchHead && planes > 1) {
-    /* the channels one after the other, each in the whole scratch */
-    return htgx_render_channels(ctx, M, planes, accum, stream, htgx_render_wavefront_noalloc);
-  }
-  if(need > kScratchBytes - kScratchHead) {
-    fprintf(stderr, "htgx: htgx_render_accum_noalloc: %llu chunk partials of %zu B exceed the "
-            "%zu MiB scratch (fewer pixels, fewer realisations per call, or a larger chunk)\n",
-            (unsigned long long)(need / sizeof(htgx_mc_accum)), sizeof(htgx_mc_accum),
-            kScratchBytes >> 20);
+  const uint64_t plane = (uint64_t)P.plane_tiles * 64u; /* chunks of a plane, one for each pixel */
+  const uint64_t full = plane * (M.spp / full_chunk(st, M.spp));
+  if(full > kNoallocChunks) {
+    fprintf(stderr, "htgx: htgx_render_accum_noalloc: %llu chunks, more than %llu "
+            "(fewer pixels, fewer realisations per call, or a larger chunk)\n",
+            (unsigned long long)full, (unsigned long long)kNoallocChunks);
     return HTGX_BAD_ARG;
   }
-  const uint32_t grid = spread_launch(kernel_grid(st->grid, M.spectral_type, features(st->S, M),
-                                                (uint64_t)M.width * M.height * planes * M.spp), &P);
-  P.counters = (unsigned int*)base;
-  P.partials = (htgx_mc_accum*)(base + kScratchHead);
-  /* fill kernels, no memset: the call may be captured in a graph */
-  zero_u32_kernel<<<1, 64, 0, stream>>>(P.counters, kXcds);
-  HIP_OK(hipGetLastError());
-  if(ctx->counting) {
-    zero_u64_kernel<<<1, 64, 0, stream>>>(ctx->d_counters, HTGX_NSTATS);
-    HIP_OK(hipGetLastError());
-    if((res = launch<true>(st->S, M, P, grid, stream))) return res;
-  } else {
-    if((res = launch<false>(st->S, M, P, grid, stream))) return res;
+  const uint64_t capacity = (kScratchBytes - kScratchHead) / sizeof(htgx_mc_accum);
+  const bool together = planes == 1 || plane * planes <= capacity;
+  const uint32_t nsub = P.nsub, n = together ? 1u : planes;
+  const uint64_t most = capacity / (plane * (planes / n)), nlaunch = (nsub + most - 1) / most;
+  const uint32_t step = (uint32_t)((nsub + nlaunch - 1) / nlaunch);
+  if(n > 1) set_queue_size(P, M.width, M.height, 1);
+  for(uint32_t c = 0; c < n; ++c) {
+    const DevMap C = n > 1 ? htgx_cie_channel_map(ctx, M, (int)c) : M;
+    for(uint32_t s = 0; s < nsub; s += step) {
+      P.nsub = std::min(step, nsub - s);
+      res = launch_noalloc(ctx, C, P, s, c + s == 0, base, accum + (size_t)c * M.width * M.height, stream);
+      if(res != HTGX_OK) return res;
+    }
   }
-  const uint32_t npix = M.width * M.height * planes;
-  merge_chunks_kernel<<<(npix + 255) / 256, 256, 0, stream>>>(P, accum);
-  HIP_OK(hipGetLastError());
-  ctx->last_nrealisations = (uint64_t)npix * M.spp;
+  ctx->last_nrealisations = (uint64_t)M.width * M.height * planes * M.spp;
   return HTGX_OK;
 }
 

@@ -398,10 +398,12 @@ int htgx_render_accum
  * No counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). Its chunk counters and partial sums live
- * in a static device array of 64 MiB that each GPU holds from the first FP32
- * set-up of a context on it until the process ends; a map needing more
- * chunk partials than it holds ((64 MiB - 256 B) / 64 B, one per pixel and
- * chunk of the context's chunk-size launch parameter) returns HTGX_BAD_ARG.
+ * in a static device array of 96 MiB that each GPU holds from the first FP32
+ * set-up of a context on it until the process ends; a map of more than 2^20 - 4
+ * chunks (pixels in whole tiles of 8x8 x realisations / the largest divisor of
+ * these not above the context's chunk-size launch parameter) returns
+ * HTGX_BAD_ARG, and one whose chunks the array does not hold at once takes
+ * several launches.
  * The context's FP32 tables must exist (built by its first FP32 map or by
  * htgx_get_wavefront_params), and a band or CIE map must use the wavelength
  * tables of the context's last map (same range and reference temperature):

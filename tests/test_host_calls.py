@@ -214,3 +214,20 @@ with A.Context(synth.scene_ptr) as a, A.Context(synth.scene_ptr) as b:
         for stream in (64, 80):
             R.hipStreamSynchronize(stream)
 """)
+
+
+def test_noalloc_limit(run):
+    """2^20 - 4 chunks of the chunk-size parameter, whatever the chunks are."""
+    run("""
+with A.Context(synth.scene_ptr) as ctx:
+    ctx.wavefront_params()
+    def call(*size):
+        d = map_of(*size)
+        return F.load().htgx_render_accum_noalloc(ctx.handle, C.byref(d), C.c_void_p(ACCUM), None)
+    assert call(512, 512, 16) == F.BAD_ARG
+    assert recorded(call, 504, 512, 16) and call(504, 512, 16) == F.OK
+    for spp, launches in ((16, 1), (20, 1), (24, 1), (33, 2)):
+        lines = recorded(call, 256, 256, spp)
+        assert sum("wavefront_kernel" in l for l in lines) == launches, (spp, lines)
+        assert not any(l.startswith(("malloc", "free")) for l in lines)
+""")
