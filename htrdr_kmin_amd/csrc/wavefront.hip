@@ -2245,18 +2245,19 @@ fill_launch(htgx_ctx* ctx, const DevMap& M, uint32_t planes, Launch* P)
   return HTGX_OK;
 }
 
-/* Grid of a launch: the grid parameter, which counts a device filled at 3
- * wavefronts per SIMD, and a third more for the kernels that hold 4 (waves())
- * if that leaves a lane of the former 16 realisations at least. With fewer, the longest
- * walks bound the launch and run slower four to a SIMD: longwave images of
- * 256x256 and 512x512 at 5.3, 10.7, 21 and 85 realisations a lane 15.4 / 22.4
- * / 27.7 / 59.4 ms against 14.5 / 20.4 / 27.7 / 63.5 with 3; flux maps 23.6 /
- * 32.3 / 53.3 / 140 against 22.0 / 33.6 / 54.8 / 158. */
+/* Grid of a launch: the grid parameter. Where it is the whole device, which
+ * grid_max counts as filled at 3 wavefronts per SIMD, a third more for the
+ * kernels that hold 4 (waves()) if that leaves a lane of the former 16
+ * realisations at least. With fewer, the longest walks bound the launch and run
+ * slower four to a SIMD: longwave images of 256x256 and 512x512 at 5.3, 10.7,
+ * 21 and 85 realisations a lane 15.4 / 22.4 / 27.7 / 59.4 ms against 14.5 /
+ * 20.4 / 27.7 / 63.5 with 3; flux maps 23.6 / 32.3 / 53.3 / 140 against 22.0 /
+ * 33.6 / 54.8 / 158. */
 static uint32_t
-kernel_grid(uint32_t grid, int spectral, int feat, uint64_t nreal)
+kernel_grid(uint32_t grid, uint32_t grid_max, int spectral, int feat, uint64_t nreal)
 {
   const bool four = spectral == HTGX_SPECTRAL_LW && !(feat & kFeatRare);
-  return four && nreal >= 16ull * grid * kUnit * kBlock ? grid + grid / 3 : grid;
+  return four && grid == grid_max && nreal >= 16ull * grid * kUnit * kBlock ? grid + grid / 3 : grid;
 }
 
 /* Grid of a launch of its own, at most `grid' blocks: with fewer chunks than
@@ -2429,7 +2430,7 @@ int htgx_render_wavefront(htgx_ctx* ctx, const DevMap& M, uint32_t planes, htgx_
     P.counters = set->counters;
     P.partials = (htgx_mc_accum*)set->partials;
   }
-  const uint32_t grid = spread_launch(kernel_grid(st->grid, M.spectral_type, features(st->S, M),
+  const uint32_t grid = spread_launch(kernel_grid(st->grid, st->grid_max, M.spectral_type, features(st->S, M),
                                                 (uint64_t)M.width * M.height * planes * M.spp), &P);
   zero_u32_kernel<<<1, 64, 0, draw>>>(P.counters, kXcds);
   HIP_OK(hipGetLastError());
@@ -2470,7 +2471,7 @@ launch_noalloc(htgx_ctx* ctx, const DevMap& M, Launch P, uint32_t first, bool fi
   P.nvalid = npix * P.nsub;
   P.counters = (unsigned int*)base;
   P.partials = (htgx_mc_accum*)(base + kScratchHead);
-  const uint32_t grid = spread_launch(kernel_grid(st->grid, M.spectral_type, features(st->S, M),
+  const uint32_t grid = spread_launch(kernel_grid(st->grid, st->grid_max, M.spectral_type, features(st->S, M),
                                                 (uint64_t)npix * P.nsub * P.K), &P);
   /* fill kernels, no memset: the call may be captured in a graph */
   zero_u32_kernel<<<1, 64, 0, stream>>>(P.counters, kXcds);
@@ -2659,9 +2660,11 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
   p->sensor = Ms[0].sensor;
   p->spectral = Ms[0].spectral_type;
   p->order.resize(n);
+  uint32_t grid_max = 0;
   for(uint32_t i = 0; i < n; ++i) {
     if((res = wavefront_prepare(ctxs[i])) != HTGX_OK) return res;
     p->grid = std::max(p->grid, ctxs[i]->wf->grid);
+    grid_max = std::max(grid_max, ctxs[i]->wf->grid_max);
     p->order[i] = i;
   }
   /* largest maps first */
@@ -2721,7 +2724,7 @@ int wf_plan_build(htgx_ctx* const* ctxs, const DevMap* Ms, htgx_mc_accum* const*
     total += (double)A.M.width * A.M.height * A.M.spp;
     nchunks += (uint64_t)A.P.ntiles * A.P.nsub * 64u;
   }
-  p->grid = kernel_grid(p->grid, p->spectral, p->feat, (uint64_t)total);
+  p->grid = kernel_grid(p->grid, grid_max, p->spectral, p->feat, (uint64_t)total);
   const uint64_t nw = (uint64_t)p->grid * kUnit;
   for(uint32_t k = 0; k < n; ++k)
     p->table_h[k].A.P.lanes = (uint32_t)std::min<uint64_t>(64, (nchunks + nw - 1) / nw);

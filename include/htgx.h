@@ -432,10 +432,11 @@ struct htgx_wf_params {
   uint32_t chunk;     /* realisations per work-queue chunk at most (1-16; 0 =
                          default 4; small maps take smaller ones) */
   uint32_t grid;      /* units of 256 lanes of the persistent launch
-                         (1-grid_max; 0 = grid_max); large longwave maps
-                         take a third more */
+                         (1-grid_max; 0 = grid_max) */
   uint32_t grid_max;  /* read only: units resident on the device at once, at 3
-                         wavefronts per SIMD */
+                         wavefronts per SIMD; as the grid, the whole device:
+                         large longwave maps then take a third more, 4 per
+                         SIMD */
   uint32_t seg_thresh; /* lanes of a 64-lane wavefront that must wait for the
                           segment step before it runs while other lanes can
                           take a collision step (1-64, 1: run it whenever a

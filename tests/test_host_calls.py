@@ -231,3 +231,26 @@ with A.Context(synth.scene_ptr) as ctx:
         assert sum("wavefront_kernel" in l for l in lines) == launches, (spp, lines)
         assert not any(l.startswith(("malloc", "free")) for l in lines)
 """)
+
+
+def test_the_grid_is_the_parameter(run):
+    """The launch has the grid that was asked for, on large longwave maps too;
+    a third more of them only where the whole device was (the default)."""
+    run("""
+def blocks(f, *args):
+    return [int(l.split()[3]) for l in recorded(f, *args) if "wavefront_" in l]
+
+lw = dict(spectral_type=F.SPECTRAL_LW, wlen_range=(400.0, 700.0), ref_temperature=290.0)
+with A.Context(synth.scene_ptr) as ctx, A.Context(synth.scene_ptr) as other:
+    d = map_of(512, 512, 16, **lw)
+    top = ctx.wavefront_params()["grid_max"]
+    assert top == 768
+    for grid, want in ((0, 4 * top * 4 // 3), (top, 4 * top * 4 // 3), (top - 1, 4 * top - 4), (576, 2304), (1, 4)):
+        for c in (ctx, other):
+            c.set_wavefront_params(grid=grid)
+        assert blocks(ctx.render_accum, d, ACCUM) == [want], grid
+        for items in ([(ctx, d, ACCUM)], [(ctx, d, ACCUM), (other, d, ACCUM)]):
+            plan = A.BatchPlan(items, use_graph=False)
+            assert blocks(plan.step) == [want], grid
+            plan.close()
+""")
