@@ -1274,15 +1274,6 @@ HTGX_D void run_until_done(const DevScene& S, const DevMap& M, Path& P, Stream& 
   }
 }
 
-/* Neumaier compensated accumulation */
-HTGX_D void nsum(double& sum, double& c, double x)
-{
-  const double t = sum + x;
-  if(fabs(sum) >= fabs(x)) c += (sum - t) + x;
-  else c += (x - t) + sum;
-  sum = t;
-}
-
 } /* namespace htgx */
 
 #endif /* HTGX_DEVICE_H */
