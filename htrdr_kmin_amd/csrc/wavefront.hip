@@ -1963,6 +1963,7 @@ struct CallSet {
 struct htgx_wavefront_state {
   SceneF S;
   CallSet sets[2];
+  uint32_t* done = nullptr; /* those of the sets, pinned, a cache line each */
   uint32_t last_set = 0;
   std::vector<void*> bufs;
   unsigned int* d_counters = nullptr;
@@ -2034,13 +2035,13 @@ set_free(CallSet& s)
   if(s.merged) (void)hipEventDestroy(s.merged);
   if(s.counters) (void)hipFree(s.counters);
   if(s.partials) (void)hipFree(s.partials);
-  if(s.done) (void)hipHostFree(s.done);
 }
 
 static void
 wavefront_free(htgx_wavefront_state* st)
 {
   for(CallSet& s : st->sets) set_free(s);
+  if(st->done) (void)hipHostFree(st->done);
   for(void* p : st->bufs) (void)hipFree(p);
   if(st->d_counters) (void)hipFree(st->d_counters);
   if(st->d_trunc) (void)hipFree(st->d_trunc);
@@ -2180,9 +2181,10 @@ wavefront_build(htgx_ctx* ctx, htgx_wavefront_state* st)
 
   HIP_OK(hipMalloc(&st->d_counters, kXcds * sizeof(unsigned int)));
   HIP_OK(hipMalloc(&st->d_trunc, 2 * sizeof(unsigned long long)));
-  for(CallSet& s : st->sets) {
-    HIP_OK(hipHostMalloc((void**)&s.done, sizeof(uint32_t), hipHostMallocDefault));
-    *s.done = 0;
+  HIP_OK(hipHostMalloc((void**)&st->done, 2 * 64, hipHostMallocDefault));
+  for(int i = 0; i < 2; ++i) {
+    st->sets[i].done = st->done + i * 16;
+    *st->sets[i].done = 0;
   }
   if((res = scratch_lookup()) != HTGX_OK) return res;
   const unsigned long long none[2] = {0, 0};
