@@ -6,8 +6,10 @@
 #include "htgx.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <cmath>
+#include <new>
 #include <utility>
 
 #include <omp.h>
@@ -243,13 +245,9 @@ struct Top {
   uint32_t count, first;       /* nodes of all below, place of the first */
 };
 
-} /* namespace */
-
-int bvh_build(const float* verts, uint32_t nverts, const uint32_t* tris, const uint32_t* tri_mtl,
-              uint32_t ntris, BvhHost& out)
+int build_tree(const float* verts, uint32_t nverts, const uint32_t* tris, const uint32_t* tri_mtl,
+               uint32_t ntris, BvhHost& out)
 {
-  if(!verts || !tris || !nverts || !ntris) return HTGX_BAD_ARG;
-  if(ntris >= (1u << 29)) return HTGX_BAD_ARG;
   Builder b;
   b.tbox.resize(ntris);
   b.cent.resize(3 * (size_t)ntris);
@@ -293,13 +291,17 @@ int bvh_build(const float* verts, uint32_t nverts, const uint32_t* tris, const u
     for(int k = 0; k < 2; ++k) tops[tops[i].child + k].r = child[k];
   }
   uint32_t depth = 0;
+  std::atomic<bool> nomem{false};
   #pragma omp parallel for schedule(dynamic, 1) reduction(max : depth)
   for(int64_t i = 0; i < (int64_t)tops.size(); ++i) {
     if(tops[i].child) continue;
-    const uint32_t d = b.build(tops[i].r, tops[i].nodes);
+    uint32_t d = 0;
+    try { d = b.build(tops[i].r, tops[i].nodes); }
+    catch(const std::bad_alloc&) { nomem.store(true); } /* it must not leave the thread's loop */
     depth = std::max(depth, d);
     tops[i].count = (uint32_t)tops[i].nodes.size();
   }
+  if(nomem.load()) return HTGX_MEM_ERR;
   out.depth = std::max(out.depth, depth);
 
   /* depth-first layout: the places of the subtrees, then their nodes */
@@ -343,6 +345,17 @@ int bvh_build(const float* verts, uint32_t nverts, const uint32_t* tris, const u
   }
   for(int a = 0; a < 3; ++a) { out.lo[a] = scene.lo[a]; out.hi[a] = scene.hi[a]; }
   return HTGX_OK;
+}
+
+} /* namespace */
+
+int bvh_build(const float* verts, uint32_t nverts, const uint32_t* tris, const uint32_t* tri_mtl,
+              uint32_t ntris, BvhHost& out)
+{
+  if(!verts || !tris || !nverts || !ntris) return HTGX_BAD_ARG;
+  if(ntris >= (1u << 29)) return HTGX_BAD_ARG;
+  try { return build_tree(verts, nverts, tris, tri_mtl, ntris, out); }
+  catch(const std::bad_alloc&) { return HTGX_MEM_ERR; }
 }
 
 } /* namespace htgx */
