@@ -378,11 +378,12 @@ int htgx_draw_map
  * (for a CIE XYZ image: 3 such planes, X then Y then Z; channel c draws from
  * streams keyed by seed ^ (c+1) << 56); `stream' is a hipStream_t (NULL =
  * default stream). Asynchronous: the accumulators are updated in the order of
- * `stream'. On the FP32 solver and a stream other than NULL, the drawing that
- * fills a call's partial sums may run ahead of earlier work on `stream' (it
- * takes the device as an earlier call's last walks leave it); a call made while
- * one of the context is in flight takes a second set of partial sums for it.
- * Under stream capture and with counters enabled it stays on `stream'. A call
+ * `stream'. On the FP32 solver and a stream other than NULL, a call made while
+ * another of the context is in flight may draw ahead of earlier work on
+ * `stream' (it takes the device as that call's last walks leave it), into a
+ * second set of partial sums, which the context keeps; only the update of the
+ * accumulators waits. Under stream capture and with counters enabled all of a
+ * call stays on `stream'. A call
  * can be captured, in any capture mode, once one like it has been made
  * uncaptured. The graphs of a context share partial sums that no other call
  * uses (replay them one after the other) and that stay until the context is
